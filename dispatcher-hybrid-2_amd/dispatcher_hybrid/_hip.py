@@ -15,7 +15,7 @@ import os
 
 import torch
 
-ABI_VERSION = 19
+ABI_VERSION = 20
 _LIB_NAME = "libdh_mixer.so"
 
 DH_F32, DH_BF16 = 0, 1
@@ -57,6 +57,9 @@ def _load():
         "dh_gate_preacts_bwd": ([i32, vp, vp, i64, i64, vp, vp, vp, i64, i64, vp, vp, vp,
                                  vp, i64, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp,
                                  i32, i32, i32, i32, i32, vp], i32),
+        "dh_gate_preacts_bwd_workspace_bytes": ([i32] * 6, i64),
+        "dh_gate_preacts_bwd_ws": ([i32, vp, vp, i64, i64, vp, vp, vp, i64, i64, vp, vp, vp, i64, i64, i64, i64,
+                                    vp, i64, i64, i64, i32] + [vp] * 8 + [i32] * 6 + [vp, i64, vp], i32),
         "dh_level_scan_fwd": ([i32, vp, vp, vp, i64, i64, i64, i64, vp, i64, i64, i64,
                                vp, i64, i64, vp, i32, i32, i32, i32, i32, i32, vp, i32, vp], i32),
         "dh_decode_mixer_step": ([i32] + [vp] * 13 + [i32] * 7 + [vp], i32),

@@ -121,6 +121,29 @@ def _(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask):
 # ---------------------------------------------------------------------------------------------
 # dispatcher::gate_preacts_bwd
 # ---------------------------------------------------------------------------------------------
+def _preacts_bwd_launch(A, B, Wi, Wf, Wr, dP, mask, outs, n_lv, levels, what):
+    """dh_gate_preacts_bwd_ws into outs = [dA, dB, dWi, dWf, dWr, dbi, dbf, dbr] (one dtype, contiguous; `levels` levels
+    of readouts) from dP, three gradients logically (b, T, n_lv, H) with one set of strides."""
+    b, T, GH = A.shape
+    H = Wi.shape[1]
+    cd = _compute_dtype(A)
+    al = lambda t: t if t.data_ptr() % 16 == 0 else t.clone()                 # (a view off 16-byte alignment)
+    A_, B_ = (al(t.contiguous().to(cd)) for t in (A, B))
+    Wi_, Wf_, Wr_ = (al(w[:n_lv].contiguous().to(cd)) for w in (Wi, Wf, Wr))
+    if not (dP[0].stride() == dP[1].stride() == dP[2].stride()):
+        dP = [g.contiguous() for g in dP]
+    m_, smb, smt, sml = _mask_view(mask, cd)
+    p = _hip.ptr
+    code = _hip.dtype_code(cd)
+    nbytes = _hip.lib.dh_gate_preacts_bwd_workspace_bytes(code, b, T, GH, H, n_lv)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=A.device)     # refused sizes: the call below says why
+    st = _hip.lib.dh_gate_preacts_bwd_ws(
+        code, p(A_), p(B_), A_.stride(0), A_.stride(1), p(Wi_), p(Wf_), p(Wr_), Wi_.stride(0), Wi_.stride(1),
+        *[p(g) for g in dP], *dP[0].stride(), p(m_), smb, smt, sml, _hip.dtype_code(outs[0].dtype),
+        *[p(o) for o in outs], levels, b, T, GH, H, n_lv, p(ws), ws.numel(), _hip.stream_handle(A.device))
+    _hip.check(st, what)
+
+
 @torch.library.custom_op("dispatcher::gate_preacts_bwd", mutates_args=(), device_types="cuda")
 def _gate_preacts_bwd_op(A: torch.Tensor, B: torch.Tensor,
                          Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
@@ -138,18 +161,8 @@ def _gate_preacts_bwd_op(A: torch.Tensor, B: torch.Tensor,
             o.zero_()
         return outs
     cd = _compute_dtype(A)
-    A_ = A.contiguous().to(cd)
-    B_ = B.contiguous().to(cd)
-    Wi_, Wf_, Wr_ = (w[:n_lv].contiguous().to(cd) for w in (Wi, Wf, Wr))
-    dPi_, dPf_, dPr_ = (g.contiguous().to(cd) for g in (dPi, dPf, dPr))
-    m_, smb, smt, sml = _mask_view(mask, cd)
-    p = _hip.ptr
-    st = _hip.lib.dh_gate_preacts_bwd(
-        _hip.dtype_code(cd), p(A_), p(B_), A_.stride(0), A_.stride(1),
-        p(Wi_), p(Wf_), p(Wr_), Wi_.stride(0), Wi_.stride(1),
-        p(dPi_), p(dPf_), p(dPr_), p(m_), smb, smt, sml,
-        *[p(o) for o in outs], b, T, GH, H, n_lv, _hip.stream_handle(dev))
-    _hip.check(st, "dispatcher::gate_preacts_bwd")
+    _preacts_bwd_launch(A, B, Wi, Wf, Wr, [g.to(cd) for g in (dPi, dPf, dPr)], mask, outs, n_lv, n_lv,
+                        "dispatcher::gate_preacts_bwd")
     return outs
 
 

@@ -29,7 +29,7 @@
 extern "C" {
 #endif
 
-#define DH_ABI_VERSION 19
+#define DH_ABI_VERSION 20
 
 enum dh_status {
   DH_OK = 0,
@@ -105,6 +105,23 @@ int dh_gate_preacts_bwd(int dtype, const void* A, const void* B, int64_t stride_
                         float* dA, float* dB, float* dWi, float* dWf, float* dWr, float* dbi,
                         float* dbf, float* dbr,
                         int b, int T, int GH, int H, int n_lv, void* stream);
+
+/*
+ * The same backward on the matrix cores, with caller scratch: every sum in fp32 and in a fixed order (no atomics), the
+ * gradients of A, B and the readouts in `out_dtype` (DH_F32, or DH_BF16 for bf16 inputs), rounded once.
+ *   dP_x      dtype `dtype`, element [b,t,l,h] at b*stride_pb + t*stride_pt + l*stride_pl + h*stride_ph
+ *   dA, dB    (b, T, GH); dW_x (levels, H, GH); db_x (levels, H), contiguous; levels >= n_lv, zeros from level n_lv on
+ *   workspace 16-byte aligned, at least dh_gate_preacts_bwd_workspace_bytes (-1 for refused sizes)
+ */
+int64_t dh_gate_preacts_bwd_workspace_bytes(int dtype, int b, int T, int GH, int H, int n_lv);
+int dh_gate_preacts_bwd_ws(int dtype, const void* A, const void* B, int64_t stride_ab, int64_t stride_at,
+                           const void* Wi, const void* Wf, const void* Wr, int64_t stride_wl,
+                           int64_t stride_wh, const void* dPi, const void* dPf, const void* dPr,
+                           int64_t stride_pb, int64_t stride_pt, int64_t stride_pl, int64_t stride_ph,
+                           const void* mask, int64_t stride_mb, int64_t stride_mt, int64_t stride_ml,
+                           int out_dtype, void* dA, void* dB, void* dWi, void* dWf, void* dWr, void* dbi,
+                           void* dbf, void* dbr, int levels, int b, int T, int GH, int H, int n_lv,
+                           void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * Parallel level scan with the gate activations fused in (sigmoid, masks, heads-first layout).

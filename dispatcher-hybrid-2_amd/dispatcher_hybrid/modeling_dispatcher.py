@@ -161,7 +161,8 @@ class DispatcherMixer(nn.Module):
         if not x.is_cuda:
             raise RuntimeError("fused gates are enabled but the input is on the CPU; move the model "
                                "to the GPU or call enable_fused_gates(False)")
-        from .fused_gates import fused_gate_preacts, fused_gate_scan, input_projections
+        from .fused_gates import (fused_gate_preacts, fused_gate_scan, gate_scan_train, input_projections,
+                                  train_scan_fits)
         Bb, T = x.shape[0], x.shape[1]
         H, hd = self.num_heads, self.head_dim
         needs_grad = torch.is_grad_enabled() and (
@@ -172,8 +173,11 @@ class DispatcherMixer(nn.Module):
             V0, A, Bs = input_projections(x, self)
         m3 = mask[..., :n_lv] if mask.dim() == 3 else None
         (Wi, bi), (Wf, bf), (Wr, br) = self._gate_params()
-        if needs_grad:
-            # differentiable: the fused pre-activations (custom op with autograd) + torch scan
+        if needs_grad and train_scan_fits(A, Bs, V0, mask, H, n_lv):
+            # differentiable: pre-activations and level scan as one operation with its own backward
+            V = gate_scan_train(A, Bs, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, H)
+        elif needs_grad:
+            # the other head widths, lengths and dtypes: fused pre-activations + torch scan
             pre_i, pre_f, pre_r = fused_gate_preacts(A, Bs, Wi, Wf, Wr, bi, bf, br, n_lv, m3)
             _, m_heads = self._masks(mask, Bb, T, n_lv)
             V = V0.view(Bb, T, H, hd).transpose(1, 2).reshape(Bb * H, T, hd)

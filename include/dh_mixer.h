@@ -149,6 +149,29 @@ int dh_level_scan_fwd(int dtype, const void* pre_i, const void* pre_f, const voi
                       int hd, int n_lv, int activated, void* ring, int ring_L, void* stream);
 
 /*
+ * The level scan and its gradient for training (reference dispatcher_hybrid/modeling_dispatcher.py:86-88, 111-121 under
+ * autograd): hd 64, T <= 4096, n_lv <= 12.
+ *   pre_x     pre-activations, element [b,t,l,h] at b*stride_pb + l*stride_pl + h*stride_ph + t; rows start on multiples
+ *             of 8 elements (stride_pl >= T rounded up to 8), 16-byte aligned. dpre_x: their gradients, the same layout.
+ *   mask      nullable, real-valued: m = [t >= 2^l] * mask[b*stride_mb + t*stride_mt + l*stride_ml] multiplies the admit
+ *             gate and blends the forget gate towards 1
+ *   states    (n_lv - 1, b, T, H*hd): the states entering levels 1 .. n_lv - 1, written by the forward, read by the backward
+ *   V, dV     the scanned state (contiguous) and its gradient (rows at b*stride_gb + t*stride_gt)
+ *   scratch   (b, T, H*hd) of the dtype, needed for n_lv > 6; dV0 (b, T, H*hd) contiguous
+ */
+int dh_level_scan_train_fwd(int dtype, const void* pre_i, const void* pre_f, const void* pre_r, int64_t stride_pb,
+                            int64_t stride_pl, int64_t stride_ph, const void* mask, int64_t stride_mb,
+                            int64_t stride_mt, int64_t stride_ml, const void* V0, int64_t stride_vb,
+                            int64_t stride_vt, void* states, void* V, int b, int T, int H, int hd, int n_lv,
+                            void* stream);
+int dh_level_scan_train_bwd(int dtype, const void* pre_i, const void* pre_f, const void* pre_r, int64_t stride_pb,
+                            int64_t stride_pl, int64_t stride_ph, const void* mask, int64_t stride_mb,
+                            int64_t stride_mt, int64_t stride_ml, const void* V0, int64_t stride_vb,
+                            int64_t stride_vt, const void* states, const void* dV, int64_t stride_gb,
+                            int64_t stride_gt, void* scratch, void* dV0, void* dpre_i, void* dpre_f, void* dpre_r,
+                            int b, int T, int H, int hd, int n_lv, void* stream);
+
+/*
  * The feed-forward block's SwiGLU activation over n elements:
  *   out[i] = silu(gate[i]) * up[i],  silu(x) = x / (1 + e^-x)
  * Replaces F.silu(linear_gate(h)) * linear_up(h) of reference

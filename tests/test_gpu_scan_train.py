@@ -1,0 +1,116 @@
+"""dispatcher::gate_scan_train (pre-activations + level scan with one backward) against float64 autograd of the eager
+mixer's formula, at the edges of its tiles: 64-position tiles with a 63-position halo, levels 0-5 inside a tile, levels
+6-11 along residue classes mod 64 of at most 16 / 32 / 64 positions.
+
+Tolerances (2-norm relative). fp32: sums of at most a few thousand terms and 12 levels of fp32 updates, and the hardware
+exponential's 1 ulp: 2e-5 bounds 12 levels x ~2^-20. bf16: pre-activations, states and their gradients are each rounded once
+per level (2^-9 relative), 12 levels and 3 roundings each in quadrature ~ 6 x 2^-9 = 1.2e-2; 2.5e-2 holds twice that."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _truth(A, B, W, bias, mask, V0, dV, H, n_lv):
+    leaves = [t.detach().double().requires_grad_() for t in (A, B, *W, *bias, V0)]
+    A, B, Wi, Wf, Wr, bi, bf, br, V0 = leaves
+    b, T, d = V0.shape
+    V = V0.view(b, T, H, d // H)
+    m_all = mask.double().expand(b, T, mask.shape[-1])
+    t = torch.arange(T, device=DEV)
+    for l in range(n_lv):
+        lag = 1 << l
+        src = lambda x: torch.cat([torch.zeros_like(x[:, :min(lag, T)]), x[:, :max(T - lag, 0)]], 1)
+        m = m_all[..., l:l + 1] * (t >= lag).view(1, T, 1)
+        hid = torch.relu(A + src(B) * (m > 0 if mask.dim() == 3 else (t >= lag).view(1, T, 1))) ** 2
+        si, sf, sr = (torch.sigmoid(hid @ w[l].T + c[l]) for w, c in ((Wi, bi), (Wf, bf), (Wr, br)))
+        V = (sf * m + 1 - m).unsqueeze(-1) * V + (si * m).unsqueeze(-1) * src(sr.unsqueeze(-1) * V)
+    V = V.reshape(b, T, d)
+    V.backward(dV.double())
+    return [V.detach()] + [x.grad for x in leaves]
+
+
+CASES = [  # b, T, H, mask kind ("level", "doc", "soft": fractional values)
+    (1, 1, 1, "level"), (2, 2, 3, "doc"), (1, 63, 4, "doc"), (1, 64, 5, "soft"), (2, 65, 2, "doc"), (1, 127, 1, "level"),
+    (3, 129, 4, "soft"), (1, 777, 3, "level"), (2, 1024, 2, "doc"), (1, 1025, 2, "doc"), (1, 2048, 1, "level"),
+    (1, 2049, 5, "doc"), (1, 4095, 1, "doc"), (1, 4096, 2, "doc")]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,T,H,kind", CASES)
+def test_gate_scan_train_against_float64(b, T, H, kind, dtype):
+    from dispatcher_hybrid.fused_gates import gate_scan_train
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=g)
+    d, L = 64 * H, 12
+    n_lv = min(L, T.bit_length())
+    A, B, V0 = (rn(b, T, d).mul(0.6).to(dtype) for _ in range(3))
+    W = [(rn(L, H, d) * 0.05).to(dtype) for _ in range(3)]
+    bias = [torch.full((L, H), c, device=DEV).add(rn(L, H) * 0.1).to(dtype) for c in (-1.0, 1.5, 2.0)]
+    lag = 1 << torch.arange(L, device=DEV)
+    t = torch.arange(T, device=DEV).unsqueeze(1)
+    mask = ((t >= lag) & (lag < T)).to(dtype)
+    if kind != "level":
+        mask = mask * (torch.rand(b, T, L, device=DEV, generator=g) < 0.9)
+    if kind == "soft":
+        mask = mask * (0.5 + 0.5 * torch.rand(b, T, L, device=DEV, generator=g)).to(dtype)
+    dV = rn(b, T, d).to(dtype)
+    ref = _truth(A, B, W, bias, mask, V0, dV, H, n_lv)
+    leaves = [x.clone().requires_grad_() for x in (A, B, *W, *bias, V0)]
+    V = gate_scan_train(leaves[0], leaves[1], *leaves[2:8], n_lv, mask, leaves[8], H)
+    V.backward(dV)
+    got = [V.detach()] + [x.grad for x in leaves]
+    names = ["V", "dA", "dB", "dWi", "dWf", "dWr", "dbi", "dbf", "dbr", "dV0"]
+    for n, x, y in zip(names, got, ref):
+        assert x.dtype == dtype and x.shape == y.shape
+        err, size = (x.double() - y).norm().item(), y.norm().item()
+        assert err <= (2e-5 if dtype == torch.float32 else 2.5e-2) * size + 1e-30, (n, err / max(size, 1e-30))
+
+
+def test_gate_scan_train_matches_module_fallback():
+    """The mixer's training pass through the operation and through the torch scan (a mask that takes gradients keeps it
+    there) give the same fp32 output and gradients."""
+    from dispatcher_hybrid import DispatcherConfig
+    from dispatcher_hybrid.modeling_dispatcher import DispatcherMixer
+    torch.manual_seed(3)
+    cfg = DispatcherConfig(d_model=128, num_heads=2, max_len=256, num_layers=1, attn_layers=(), vocab_size=64,
+                           dim_feedforward=128)
+    mx = DispatcherMixer(cfg).to(DEV)
+    with torch.no_grad():
+        for p in mx.parameters():
+            if p.dim() > 1 and p.shape != (8, 2):
+                p.normal_(std=0.1)
+    mx.use_fused_gates = True
+    x0 = torch.randn(2, 150, 128, device=DEV)
+    t = torch.arange(150, device=DEV).unsqueeze(1)
+    mask = (t >= (1 << torch.arange(8, device=DEV))).float()
+    outs = []
+    for m in (mask, mask.clone().requires_grad_()):
+        x = x0.clone().requires_grad_()
+        mx.zero_grad()
+        y = mx(x, m)
+        y.square().sum().backward()
+        outs.append([y.detach(), x.grad] + [p.grad.clone() for p in mx.parameters()])
+    for a, b in zip(*outs):
+        assert (a - b).norm() <= 2e-5 * b.norm()
+
+
+def test_gate_scan_train_under_checkpoint_and_autocast():
+    """Activation checkpointing recomputes the operation; under autocast (bf16 activations, fp32 weights) the weights'
+    gradients come back in fp32."""
+    from dispatcher_hybrid.fused_gates import gate_scan_train
+    from torch.utils.checkpoint import checkpoint
+    g = torch.Generator(device=DEV).manual_seed(1)
+    b, T, H, L = 1, 100, 2, 7
+    A, B, V0 = (torch.randn(b, T, 64 * H, device=DEV, generator=g).bfloat16().requires_grad_() for _ in range(3))
+    W = [(torch.randn(L, H, 64 * H, device=DEV, generator=g) * 0.05).requires_grad_() for _ in range(3)]
+    bias = [torch.zeros(L, H, device=DEV).requires_grad_() for _ in range(3)]
+    mask = (torch.arange(T, device=DEV).unsqueeze(1) >= (1 << torch.arange(L, device=DEV))).float()
+    leaves = [A, B, *W, *bias, V0]
+    f = lambda *xs: gate_scan_train(*xs[:8], L, mask, xs[8], H)
+    plain = torch.autograd.grad(f(*leaves).float().square().sum(), leaves)
+    again = torch.autograd.grad(checkpoint(f, *leaves, use_reentrant=False).float().square().sum(), leaves)
+    assert all(p.dtype == x.dtype for p, x in zip(plain, leaves))
+    assert all(torch.equal(p, q) for p, q in zip(plain, again))

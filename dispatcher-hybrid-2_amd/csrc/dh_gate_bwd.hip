@@ -193,8 +193,9 @@ struct AbArgs {
   int64_t swl, swh;
   const void* p1;
   const uint32_t* ok;
-  void* dA;
+  void* dA;                     // rows of GH at b sgb + t sgt, both
   void* dB;
+  int64_t sgb, sgt;
   Dims d;
 };
 
@@ -406,7 +407,7 @@ __global__ __launch_bounds__(kAbThreads, 4) void gate_bwd_ab(AbArgs a) {
     }
     const int t = t0 + r;
     if (live && t < d.T) {
-      OT* o = (OT*)(is_b ? a.dB : a.dA) + ((int64_t)b * d.T + t) * d.GH + k0;
+      OT* o = (OT*)(is_b ? a.dB : a.dA) + (int64_t)b * a.sgb + (int64_t)t * a.sgt + k0;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         OT* oj = o + (4 * j + g) * K;
@@ -735,7 +736,7 @@ extern "C" int dh_gate_preacts_bwd_ws(int dtype, const void* A, const void* B, i
                                       int64_t stride_wh, const void* dPi, const void* dPf, const void* dPr,
                                       int64_t stride_pb, int64_t stride_pt, int64_t stride_pl, int64_t stride_ph,
                                       const void* mask, int64_t stride_mb, int64_t stride_mt, int64_t stride_ml,
-                                      int out_dtype, void* dA, void* dB, void* dWi, void* dWf, void* dWr, void* dbi,
+                                      int out_dtype, void* dA, void* dB, int64_t stride_gb, int64_t stride_gt, void* dWi, void* dWf, void* dWr, void* dbi,
                                       void* dbf, void* dbr, int levels, int b, int T, int GH, int H, int n_lv,
                                       void* workspace, int64_t workspace_bytes, void* stream) {
   const char* who = "dh_gate_preacts_bwd_ws";
@@ -745,6 +746,8 @@ extern "C" int dh_gate_preacts_bwd_ws(int dtype, const void* A, const void* B, i
              "%s: gradients of dtype %d for inputs of dtype %d", who, out_dtype, dtype);
   DH_REQUIRE(A && B && Wi && Wf && Wr && dPi && dPf && dPr && dA && dB && dWi && dWf && dWr && dbi && dbf && dbr,
              DH_ERR_INVALID_ARG, "%s: null pointer argument", who);
+  DH_REQUIRE(stride_gt >= GH && stride_gb >= 0 && stride_gt % 8 == 0 && stride_gb % 8 == 0, DH_ERR_INVALID_ARG,
+             "%s: gradient row stride %lld", who, (long long)stride_gt);
   DH_REQUIRE(levels >= n_lv && levels <= 64, DH_ERR_INVALID_ARG, "%s: levels=%d below n_lv=%d", who, levels, n_lv);
   const int vec = dtype == DH_BF16 ? 8 : 4;
   const int64_t esz = dtype == DH_BF16 ? 2 : 4;
@@ -766,7 +769,7 @@ extern "C" int dh_gate_preacts_bwd_ws(int dtype, const void* A, const void* B, i
   PackArgs pa{{dPi, dPf, dPr}, stride_pb, stride_pt, stride_pl, stride_ph, mask, stride_mb, stride_mt, stride_ml,
               ws + sp.p1, (uint4*)(ws + sp.p2), (uint32_t*)(ws + sp.ok), d};
   AbArgs aa{A, B, stride_ab, stride_at, {Wi, Wf, Wr}, stride_wl, stride_wh, ws + sp.p1, (const uint32_t*)(ws + sp.ok),
-            dA, dB, d};
+            dA, dB, stride_gb, stride_gt, d};
   WArgs wa{A, B, stride_ab, stride_at, (const uint4*)(ws + sp.p2), (const uint32_t*)(ws + sp.ok), (float*)(ws + sp.part),
            nsplit, (int)((blocks + nsplit - 1) / nsplit), d};
   void* const dw[6] = {dWi, dWf, dWr, dbi, dbf, dbr};

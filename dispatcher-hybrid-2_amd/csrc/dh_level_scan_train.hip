@@ -137,7 +137,8 @@ struct Args {
   const void* dV;               // backward: its gradient, rows of d at b sgb + t sgt
   int64_t sgb, sgt;
   void* mid;                    // backward: gradient of the state entering level 6 (b, T, d)
-  void* dV0;                    // (b, T, d)
+  void* dV0;                    // rows of d at b sob + t sot
+  int64_t sob, sot;
   void* dpre[3];                // laid out as pre
   int b, T, H, n_lv;
 };
@@ -279,10 +280,11 @@ __global__ __launch_bounds__(256, 2) void scan_local_bwd(Args a) {
       DH_PIN(G[j], j);
     }
   });
-  const __amdgpu_buffer_rsrc_t r = head_rows<T>(a.dV0, (int64_t)b * a.T * d, d, h, a.T);
-  Walk o(s0, ob, cb);
+  const __amdgpu_buffer_rsrc_t r = head_rows<T>(a.dV0, (int64_t)b * a.sob, a.sot, h, a.T);
+  const uint32_t db = (uint32_t)(a.sot * (int64_t)sizeof(T));
+  Walk o(s0, db, cb);
 #pragma unroll
-  for (int j = 0; j < 64; ++j) Row<T>::store(r, o.next(ob), G[j]);
+  for (int j = 0; j < 64; ++j) Row<T>::store(r, o.next(db), G[j]);
 }
 
 // ---- strided levels ----------------------------------------------------------------------------------------------
@@ -501,11 +503,12 @@ extern "C" int dh_level_scan_train_bwd(int dtype, const void* pre_i, const void*
                                        int64_t stride_pb, int64_t stride_pl, int64_t stride_ph, const void* mask,
                                        int64_t stride_mb, int64_t stride_mt, int64_t stride_ml, const void* V0,
                                        int64_t stride_vb, int64_t stride_vt, const void* states, const void* dV,
-                                       int64_t stride_gb, int64_t stride_gt, void* scratch, void* dV0, void* dpre_i,
-                                       void* dpre_f, void* dpre_r, int b, int T, int H, int hd, int n_lv, void* stream) {
+                                       int64_t stride_gb, int64_t stride_gt, void* scratch, void* dV0,
+                                       int64_t stride_ob, int64_t stride_ot, void* dpre_i, void* dpre_f, void* dpre_r, int b, int T, int H, int hd, int n_lv, void* stream) {
   const char* who = "dh_level_scan_train_bwd";
   int st = check_train(who, dtype, stride_pb, stride_pl, stride_ph, stride_vb, stride_vt, b, T, H, hd, n_lv);
   if (!st) st = check_train(who, dtype, stride_pb, stride_pl, stride_ph, stride_gb, stride_gt, b, T, H, hd, n_lv);
+  if (!st) st = check_train(who, dtype, stride_pb, stride_pl, stride_ph, stride_ob, stride_ot, b, T, H, hd, n_lv);
   if (st) return st;
   DH_REQUIRE(pre_i && pre_f && pre_r && V0 && (states || n_lv == 1) && dV && dV0 && dpre_i && dpre_f && dpre_r &&
                  (scratch || n_lv <= kLocal),
@@ -533,6 +536,8 @@ extern "C" int dh_level_scan_train_bwd(int dtype, const void* pre_i, const void*
   a.sgt = stride_gt;
   a.mid = scratch;
   a.dV0 = dV0;
+  a.sob = stride_ob;
+  a.sot = stride_ot;
   a.dpre[0] = dpre_i;
   a.dpre[1] = dpre_f;
   a.dpre[2] = dpre_r;

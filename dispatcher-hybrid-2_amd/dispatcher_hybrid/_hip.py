@@ -59,13 +59,15 @@ def _load():
                                  i32, i32, i32, i32, i32, vp], i32),
         "dh_gate_preacts_bwd_workspace_bytes": ([i32] * 6, i64),
         "dh_gate_preacts_bwd_ws": ([i32, vp, vp, i64, i64, vp, vp, vp, i64, i64, vp, vp, vp, i64, i64, i64, i64,
-                                    vp, i64, i64, i64, i32] + [vp] * 8 + [i32] * 6 + [vp, i64, vp], i32),
+                                    vp, i64, i64, i64, i32, vp, vp, i64, i64] + [vp] * 6 + [i32] * 6 + [vp, i64, vp], i32),
         "dh_level_scan_fwd": ([i32, vp, vp, vp, i64, i64, i64, i64, vp, i64, i64, i64,
                                vp, i64, i64, vp, i32, i32, i32, i32, i32, i32, vp, i32, vp], i32),
         "dh_level_scan_train_fwd": ([i32, vp, vp, vp, i64, i64, i64, vp, i64, i64, i64, vp, i64, i64, vp, vp]
                                      + [i32] * 5 + [vp], i32),
         "dh_level_scan_train_bwd": ([i32, vp, vp, vp, i64, i64, i64, vp, i64, i64, i64, vp, i64, i64, vp, vp, i64, i64]
-                                     + [vp] * 5 + [i32] * 5 + [vp], i32),
+                                     + [vp, vp, i64, i64, vp, vp, vp] + [i32] * 5 + [vp], i32),
+        "dh_wgrad_gemm_workspace_bytes": ([i32, i32, vp, vp], i64),
+        "dh_wgrad_gemm": ([i32, i32, i32] + [vp] * 8 + [i64, vp], i32),
         "dh_decode_mixer_step": ([i32] + [vp] * 13 + [i32] * 7 + [vp], i32),
         "dh_step_gates": ([i32] + [vp] * 12 + [i32] * 5 + [vp], i32),
         "dh_decode_gemv": ([i32, vp, i64, vp, vp, ctypes.c_float, i32, vp, vp, vp, vp, vp,

@@ -121,15 +121,24 @@ def _(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask):
 # ---------------------------------------------------------------------------------------------
 # dispatcher::gate_preacts_bwd
 # ---------------------------------------------------------------------------------------------
+def _rows16(t, n):
+    """t with unit-stride rows whose starts are 16-byte aligned (n elements to 16 bytes), copied if it is not."""
+    t = t if t.stride(-1) == 1 and all(s % n == 0 for s in t.stride()[:-1]) else t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+
+
 def _preacts_bwd_launch(A, B, Wi, Wf, Wr, dP, mask, outs, n_lv, levels, what):
-    """dh_gate_preacts_bwd_ws into outs = [dA, dB, dWi, dWf, dWr, dbi, dbf, dbr] (one dtype, contiguous; `levels` levels
-    of readouts) from dP, three gradients logically (b, T, n_lv, H) with one set of strides."""
+    """dh_gate_preacts_bwd_ws into outs = [dA, dB, dWi, dWf, dWr, dbi, dbf, dbr] (one dtype; dA and dB with unit-stride rows
+    and equal strides, the others contiguous with `levels` levels) from dP, three gradients logically (b, T, n_lv, H) with
+    one set of strides."""
     b, T, GH = A.shape
     H = Wi.shape[1]
     cd = _compute_dtype(A)
-    al = lambda t: t if t.data_ptr() % 16 == 0 else t.clone()                 # (a view off 16-byte alignment)
-    A_, B_ = (al(t.contiguous().to(cd)) for t in (A, B))
-    Wi_, Wf_, Wr_ = (al(w[:n_lv].contiguous().to(cd)) for w in (Wi, Wf, Wr))
+    vec = 8 if cd == torch.bfloat16 else 4
+    A_, B_ = (_rows16(t.to(cd), vec) for t in (A, B))
+    if A_.stride() != B_.stride():
+        A_, B_ = A_.contiguous(), B_.contiguous()
+    Wi_, Wf_, Wr_ = (_rows16(w[:n_lv].contiguous().to(cd), vec) for w in (Wi, Wf, Wr))
     if not (dP[0].stride() == dP[1].stride() == dP[2].stride()):
         dP = [g.contiguous() for g in dP]
     m_, smb, smt, sml = _mask_view(mask, cd)
@@ -139,8 +148,9 @@ def _preacts_bwd_launch(A, B, Wi, Wf, Wr, dP, mask, outs, n_lv, levels, what):
     ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=A.device)     # refused sizes: the call below says why
     st = _hip.lib.dh_gate_preacts_bwd_ws(
         code, p(A_), p(B_), A_.stride(0), A_.stride(1), p(Wi_), p(Wf_), p(Wr_), Wi_.stride(0), Wi_.stride(1),
-        *[p(g) for g in dP], *dP[0].stride(), p(m_), smb, smt, sml, _hip.dtype_code(outs[0].dtype),
-        *[p(o) for o in outs], levels, b, T, GH, H, n_lv, p(ws), ws.numel(), _hip.stream_handle(A.device))
+        *[p(g) for g in dP], *dP[0].stride(), p(m_), smb, smt, sml, _hip.dtype_code(outs[0].dtype), p(outs[0]), p(outs[1]),
+        outs[0].stride(0), outs[0].stride(1), *[p(o) for o in outs[2:]], levels, b, T, GH, H, n_lv, p(ws), ws.numel(),
+        _hip.stream_handle(A.device))
     _hip.check(st, what)
 
 
@@ -308,134 +318,6 @@ def fused_gate_scan(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, num_heads):
     of the activated gates, which follows the eager path (reference
     dispatcher_hybrid/modeling_dispatcher.py:86-88, 100-121)."""
     return torch.ops.dispatcher.gate_scan_fwd(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
-
-
-# ---------------------------------------------------------------------------------------------
-# dispatcher::gate_scan_train -- the gate path of training: pre-activations and level scan with one backward
-# ---------------------------------------------------------------------------------------------
-TRAIN_SCAN_MAX_LEN = 4096
-TRAIN_SCAN_MAX_LEVELS = 12
-TRAIN_SCAN_HEAD = 64
-
-
-def train_scan_fits(A, B, V0, mask, num_heads, n_lv):
-    """Whether dispatcher::gate_scan_train takes these: fp32 or bf16 throughout, 64-wide heads (a wave holds a head's
-    columns), at most 4096 positions and 12 levels, and a mask no gradient flows to."""
-    return (A.dtype in (torch.float32, torch.bfloat16) and B.dtype == A.dtype and V0.dtype == A.dtype
-            and V0.shape[-1] == TRAIN_SCAN_HEAD * num_heads and V0.shape[1] <= TRAIN_SCAN_MAX_LEN
-            and n_lv <= TRAIN_SCAN_MAX_LEVELS and not mask.requires_grad)
-
-
-def _gate_rows(b, H, n_lv, T, like):
-    """Three head-major gate tensors (b, H, n_lv, T) in one allocation, rows padded to a multiple of 8 positions."""
-    return torch.empty(3, b, H, n_lv, -(-T // 8) * 8, device=like.device, dtype=like.dtype)
-
-
-def _scan_mask(mask, b, T, n_lv, cd):
-    """The level (T, L) or document (b, T, L) mask as a (b, T, n_lv) view in dtype cd."""
-    return mask[..., :n_lv].to(cd).expand(b, T, n_lv)
-
-
-@torch.library.custom_op("dispatcher::gate_scan_train", mutates_args=(), device_types="cuda")
-def _gate_scan_train_op(A: torch.Tensor, B: torch.Tensor, Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
-                        bi: torch.Tensor, bf: torch.Tensor, br: torch.Tensor, mask: torch.Tensor, V0: torch.Tensor,
-                        num_heads: int, n_lv: int) -> List[torch.Tensor]:
-    b, T, d = V0.shape
-    H, cd = num_heads, A.dtype
-    V = torch.empty(b, T, d, device=V0.device, dtype=cd)
-    pre = _gate_rows(b, H, n_lv, T, A)
-    states = torch.empty(n_lv - 1, b, T, d, device=V0.device, dtype=cd)
-    if b == 0 or T == 0:
-        return [V, pre, states]
-    ins = _prep_gate_inputs(A, B, Wi, Wf, Wr, bi, bf, br, n_lv)
-    gates = [g[..., :T].permute(0, 3, 2, 1) for g in pre]                     # logical (b, T, n_lv, H)
-    m = _scan_mask(mask, b, T, n_lv, cd)
-    _preacts_launch(*ins, m if mask.dim() == 3 else None, gates, gates[0].stride(), 0, n_lv,
-                    "dispatcher::gate_scan_train")
-    V0 = V0.contiguous()
-    p = _hip.ptr
-    st = _hip.lib.dh_level_scan_train_fwd(
-        _hip.dtype_code(cd), p(pre[0]), p(pre[1]), p(pre[2]), pre.stride(1), pre.stride(3), pre.stride(2), p(m),
-        *m.stride(), p(V0), V0.stride(0), V0.stride(1), p(states), p(V), b, T, H, d // H, n_lv,
-        _hip.stream_handle(V0.device))
-    _hip.check(st, "dispatcher::gate_scan_train")
-    return [V, pre, states]
-
-
-@_gate_scan_train_op.register_fake
-def _(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv):
-    b, T, d = V0.shape
-    return [torch.empty_like(V0, memory_format=torch.contiguous_format), _gate_rows(b, num_heads, n_lv, T, A),
-            A.new_empty(n_lv - 1, b, T, d)]
-
-
-@torch.library.custom_op("dispatcher::gate_scan_train_bwd", mutates_args=(), device_types="cuda")
-def _gate_scan_train_bwd_op(A: torch.Tensor, B: torch.Tensor, Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
-                            mask: torch.Tensor, V0: torch.Tensor, pre: torch.Tensor, states: torch.Tensor,
-                            dV: torch.Tensor, num_heads: int, n_lv: int) -> List[torch.Tensor]:
-    b, T, d = V0.shape
-    H, cd, dev = num_heads, A.dtype, A.device
-    dV0 = torch.empty(b, T, d, device=dev, dtype=cd)
-    # the gradients in the inputs' dtype where they share one, else (autocast: wider weights) in fp32
-    od = cd if Wi.dtype == cd else torch.float32
-    levels = Wi.shape[0]
-    outs = [torch.empty(A.shape, device=dev, dtype=od) for _ in range(2)]
-    outs += [torch.empty(levels, H, A.shape[-1], device=dev, dtype=od) for _ in range(3)]
-    outs += [torch.empty(levels, H, device=dev, dtype=od) for _ in range(3)]
-    if b == 0 or T == 0:
-        return [dV0] + [o.zero_() for o in outs]
-    m = _scan_mask(mask, b, T, n_lv, cd)
-    V0, dV = V0.contiguous(), dV.to(cd).contiguous()
-    dpre = torch.empty_like(pre)
-    # the gradient between the strided and the local levels borrows dA's memory (written only afterwards) where it fits
-    scratch = outs[0] if outs[0].numel() >= V0.numel() else torch.empty_like(dV0)
-    p = _hip.ptr
-    st = _hip.lib.dh_level_scan_train_bwd(
-        _hip.dtype_code(cd), p(pre[0]), p(pre[1]), p(pre[2]), pre.stride(1), pre.stride(3), pre.stride(2), p(m),
-        *m.stride(), p(V0), V0.stride(0), V0.stride(1), p(states), p(dV), dV.stride(0), dV.stride(1), p(scratch), p(dV0),
-        p(dpre[0]), p(dpre[1]), p(dpre[2]), b, T, H, d // H, n_lv, _hip.stream_handle(dev))
-    _hip.check(st, "dispatcher::gate_scan_train_bwd")
-    _preacts_bwd_launch(A, B, Wi, Wf, Wr, [g[..., :T].permute(0, 3, 2, 1) for g in dpre],
-                        m if mask.dim() == 3 else None, outs, n_lv, levels, "dispatcher::gate_scan_train_bwd")
-    return [dV0] + outs
-
-
-@_gate_scan_train_bwd_op.register_fake
-def _(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, num_heads, n_lv):
-    od = A.dtype if Wi.dtype == A.dtype else torch.float32
-    L = Wi.shape[0]
-    return ([A.new_empty(V0.shape)] + [A.new_empty(A.shape, dtype=od) for _ in range(2)]
-            + [A.new_empty((L, num_heads, A.shape[-1]), dtype=od) for _ in range(3)]
-            + [A.new_empty((L, num_heads), dtype=od) for _ in range(3)])
-
-
-def _train_setup(ctx, inputs, output):
-    A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv = inputs
-    _, pre, states = output
-    ctx.save_for_backward(A, B, Wi, Wf, Wr, mask, V0, pre, states)
-    ctx.sizes = (num_heads, n_lv)
-    ctx.dtypes = [t.dtype for t in (A, B, Wi, Wf, Wr, bi, bf, br)]
-
-
-def _train_backward(ctx, grads):
-    dV = grads[0]
-    if dV is None:
-        return (None,) * 12
-    A, B, Wi, Wf, Wr, mask, V0, pre, states = ctx.saved_tensors
-    dV0, *rest = torch.ops.dispatcher.gate_scan_train_bwd(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, *ctx.sizes)
-    return (*[g.to(dt) for g, dt in zip(rest, ctx.dtypes)], None, dV0, None, None)
-
-
-torch.library.register_autograd("dispatcher::gate_scan_train", _train_backward, setup_context=_train_setup)
-
-
-def gate_scan_train(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, num_heads):
-    """Scanned mixer state (b, T, d) as fused_gate_scan's, differentiable in everything but the mask: fused_gate_preacts
-    and the level loop of the eager mixer (reference dispatcher_hybrid/modeling_dispatcher.py:100-121) as one operation with
-    one backward (dh_level_scan_train_fwd / _bwd, dh_gate_preacts_bwd_ws). Sums and the states within a launch are fp32;
-    the pre-activations, the state entering every level and their gradients are kept in A's dtype. `mask`: the (T, L) level
-    mask or the (b, T, L) document mask; edges with t < 2^l do not exist whatever it says. See train_scan_fits."""
-    return torch.ops.dispatcher.gate_scan_train(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)[0]
 
 
 def prefill_gate_scan(A, B, Wi, Wf, Wr, bi, bf, br, V0, num_heads, rg_hist, V_ring):

@@ -1,0 +1,307 @@
+"""Training passes of the fused layers on gfx950 kernels, each one operation with one backward.
+
+    dispatcher::gate_scan_train   gate pre-activations + level scan (from the projections A, B, V0)
+    dispatcher::mixer_train       a whole mixer layer: projections, gate path, output projection
+
+Both run under ``model.enable_fused_gates()`` when gradients are wanted (DispatcherMixer picks the widest one that fits)
+and replace the reference's eager autograd of the level loop (reference dispatcher_hybrid/modeling_dispatcher.py:86-121)
+and its fused gate op's backward (reference dispatcher_hybrid/fused_gates.py:96-173, 225-257). Kernels:
+``dh_gate_preacts_fwd``, ``dh_level_scan_train_fwd`` / ``_bwd``, ``dh_gate_preacts_bwd_ws``, ``dh_wgrad_gemm`` and, for the
+plain products, ``dh_proj_gemm`` or the library.
+
+Importing this module loads the kernel library and raises ImportError if it is missing.
+"""
+
+import ctypes
+from typing import List
+
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from . import _hip
+from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch, _preacts_launch, _rows16,
+                          fused_projections)
+
+SCAN_MAX_LEN = 4096
+SCAN_MAX_LEVELS = 12
+SCAN_HEAD = 64
+
+
+def scan_fits(A, B, V0, mask, num_heads, n_lv):
+    """Whether the training scan takes these: fp32 or bf16 throughout, 64-wide heads (a wave holds a head's columns), at
+    most 4096 positions and 12 levels, and a mask no gradient flows to."""
+    return (A.dtype in (torch.float32, torch.bfloat16) and B.dtype == A.dtype and V0.dtype == A.dtype
+            and V0.shape[-1] == SCAN_HEAD * num_heads and V0.shape[1] <= SCAN_MAX_LEN
+            and n_lv <= SCAN_MAX_LEVELS and not mask.requires_grad)
+
+
+def _gate_rows(b, H, n_lv, T, like):
+    """Three head-major gate tensors (b, H, n_lv, T) in one allocation, rows padded to a multiple of 8 positions."""
+    return torch.empty(3, b, H, n_lv, -(-T // 8) * 8, device=like.device, dtype=like.dtype)
+
+
+def _scan_mask(mask, b, T, n_lv, cd):
+    """The level (T, L) or document (b, T, L) mask as a (b, T, n_lv) view in dtype cd."""
+    return mask[..., :n_lv].to(cd).expand(b, T, n_lv)
+
+
+def _gate_scan_fwd(A, B, W, bias, mask, V0, H, n_lv, what):
+    """(V, pre, states) of the gate path; A, B, V0 (b, T, .) with unit-stride, 16-byte aligned rows, A and B alike."""
+    b, T, d = V0.shape
+    cd, dev = A.dtype, A.device
+    V = torch.empty(b, T, d, device=dev, dtype=cd)
+    pre = _gate_rows(b, H, n_lv, T, A)
+    states = torch.empty(n_lv - 1, b, T, d, device=dev, dtype=cd)
+    W = [_rows16(w[:n_lv].contiguous().to(cd), 8) for w in W]
+    bias = torch.stack(tuple(bias))[:, :n_lv].float().contiguous()             # the kernel reads fp32 biases
+    m = _scan_mask(mask, b, T, n_lv, cd)
+    gates = [g[..., :T].permute(0, 3, 2, 1) for g in pre]                      # logical (b, T, n_lv, H)
+    _preacts_launch(A, B, *W, bias[0], bias[1], bias[2], m if mask.dim() == 3 else None, gates, gates[0].stride(), 0,
+                    n_lv, what)
+    p = _hip.ptr
+    st = _hip.lib.dh_level_scan_train_fwd(
+        _hip.dtype_code(cd), p(pre[0]), p(pre[1]), p(pre[2]), pre.stride(1), pre.stride(3), pre.stride(2), p(m),
+        *m.stride(), p(V0), V0.stride(0), V0.stride(1), p(states), p(V), b, T, H, d // H, n_lv, _hip.stream_handle(dev))
+    _hip.check(st, what)
+    return V, pre, states
+
+
+def _gate_scan_bwd(A, B, W, mask, V0, pre, states, dV, dV0, outs, H, n_lv, what):
+    """Fills dV0 and outs = [dA, dB, dWi, dWf, dWr, dbi, dbf, dbr] from dV; A, B, V0 as _gate_scan_fwd had them, dV0, dA, dB
+    with unit-stride, 16-byte aligned rows."""
+    b, T, d = V0.shape
+    cd = A.dtype
+    m = _scan_mask(mask, b, T, n_lv, cd)
+    dpre = torch.empty_like(pre)
+    scratch = torch.empty(b, T, d, device=A.device, dtype=cd)
+    p = _hip.ptr
+    st = _hip.lib.dh_level_scan_train_bwd(
+        _hip.dtype_code(cd), p(pre[0]), p(pre[1]), p(pre[2]), pre.stride(1), pre.stride(3), pre.stride(2), p(m),
+        *m.stride(), p(V0), V0.stride(0), V0.stride(1), p(states), p(dV), dV.stride(0), dV.stride(1), p(scratch), p(dV0),
+        dV0.stride(0), dV0.stride(1), p(dpre[0]), p(dpre[1]), p(dpre[2]), b, T, H, d // H, n_lv,
+        _hip.stream_handle(A.device))
+    _hip.check(st, what)
+    _preacts_bwd_launch(A, B, *W, [g[..., :T].permute(0, 3, 2, 1) for g in dpre], m if mask.dim() == 3 else None, outs,
+                        n_lv, W[0].shape[0], what)
+
+
+def _gate_grads(W, gh, od, dev):
+    L, H = W.shape[:2]
+    return ([torch.empty(L, H, gh, device=dev, dtype=od) for _ in range(3)]
+            + [torch.empty(L, H, device=dev, dtype=od) for _ in range(3)])
+
+
+# ---------------------------------------------------------------------------------------------
+# dispatcher::gate_scan_train
+# ---------------------------------------------------------------------------------------------
+@torch.library.custom_op("dispatcher::gate_scan_train", mutates_args=(), device_types="cuda")
+def _gate_scan_train_op(A: torch.Tensor, B: torch.Tensor, Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
+                        bi: torch.Tensor, bf: torch.Tensor, br: torch.Tensor, mask: torch.Tensor, V0: torch.Tensor,
+                        num_heads: int, n_lv: int) -> List[torch.Tensor]:
+    b, T, d = V0.shape
+    if b == 0 or T == 0:
+        return [torch.empty_like(V0, memory_format=torch.contiguous_format), _gate_rows(b, num_heads, n_lv, T, A),
+                A.new_empty(n_lv - 1, b, T, d)]
+    A, B, V0 = (_rows16(t.contiguous(), 8) for t in (A, B, V0))
+    return list(_gate_scan_fwd(A, B, (Wi, Wf, Wr), (bi, bf, br), mask, V0, num_heads, n_lv, "dispatcher::gate_scan_train"))
+
+
+@_gate_scan_train_op.register_fake
+def _(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv):
+    b, T, d = V0.shape
+    return [torch.empty_like(V0, memory_format=torch.contiguous_format), _gate_rows(b, num_heads, n_lv, T, A),
+            A.new_empty(n_lv - 1, b, T, d)]
+
+
+@torch.library.custom_op("dispatcher::gate_scan_train_bwd", mutates_args=(), device_types="cuda")
+def _gate_scan_train_bwd_op(A: torch.Tensor, B: torch.Tensor, Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
+                            mask: torch.Tensor, V0: torch.Tensor, pre: torch.Tensor, states: torch.Tensor,
+                            dV: torch.Tensor, num_heads: int, n_lv: int) -> List[torch.Tensor]:
+    # the gradients in the inputs' dtype where they share one, else (autocast: wider weights) in fp32
+    od = A.dtype if Wi.dtype == A.dtype else torch.float32
+    dV0 = torch.empty(V0.shape, device=A.device, dtype=A.dtype)
+    outs = [torch.empty(A.shape, device=A.device, dtype=od) for _ in range(2)] + _gate_grads(Wi, A.shape[-1], od, A.device)
+    if V0.numel() == 0:
+        return [dV0] + [o.zero_() for o in outs]
+    A, B, V0, dV = (_rows16(t.contiguous(), 8) for t in (A, B, V0, dV.to(A.dtype)))
+    _gate_scan_bwd(A, B, (Wi, Wf, Wr), mask, V0, pre, states, dV, dV0, outs, num_heads, n_lv,
+                   "dispatcher::gate_scan_train_bwd")
+    return [dV0] + outs
+
+
+@_gate_scan_train_bwd_op.register_fake
+def _(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, num_heads, n_lv):
+    od = A.dtype if Wi.dtype == A.dtype else torch.float32
+    return ([A.new_empty(V0.shape)] + [A.new_empty(A.shape, dtype=od) for _ in range(2)]
+            + _gate_grads(Wi, A.shape[-1], od, A.device))
+
+
+def _scan_setup(ctx, inputs, output):
+    A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv = inputs
+    _, pre, states = output
+    ctx.set_materialize_grads(False)
+    ctx.save_for_backward(A, B, Wi, Wf, Wr, mask, V0, pre, states)
+    ctx.sizes = (num_heads, n_lv)
+    ctx.dtypes = [t.dtype for t in (A, B, Wi, Wf, Wr, bi, bf, br)]
+
+
+def _scan_backward(ctx, grads):
+    dV = grads[0]
+    if dV is None:
+        return (None,) * 12
+    A, B, Wi, Wf, Wr, mask, V0, pre, states = ctx.saved_tensors
+    dV0, *rest = torch.ops.dispatcher.gate_scan_train_bwd(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, *ctx.sizes)
+    return (*[g.to(dt) for g, dt in zip(rest, ctx.dtypes)], None, dV0, None, None)
+
+
+torch.library.register_autograd("dispatcher::gate_scan_train", _scan_backward, setup_context=_scan_setup)
+
+
+def gate_scan_train(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, num_heads):
+    """Scanned mixer state (b, T, d) as fused_gate_scan's, differentiable in everything but the mask: fused_gate_preacts
+    and the level loop of the eager mixer (reference dispatcher_hybrid/modeling_dispatcher.py:100-121). Sums and the states
+    within a launch are fp32; the pre-activations, the state entering every level and their gradients are kept in A's dtype.
+    `mask`: the (T, L) level mask or the (b, T, L) document mask; edges with t < 2^l do not exist whatever it says. See
+    scan_fits."""
+    return torch.ops.dispatcher.gate_scan_train(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)[0]
+
+
+# ---------------------------------------------------------------------------------------------
+# products of a training pass
+# ---------------------------------------------------------------------------------------------
+def _linear(x2, w, max_rows):
+    """x2 (M, K) . w^T: dh_proj_gemm in bf16 up to max_rows rows (measured in fused_gates), else the library."""
+    if x2.dtype == torch.bfloat16 and x2.shape[0] <= max_rows and w.shape[1] % 64 == 0 and w.shape[0] % 4 == 0:
+        return fused_projections(x2, [w])[0]
+    return F.linear(x2, w)
+
+
+def weight_grads(pairs):
+    """[dY^T X for X (M, K), dY (M, N) in pairs], up to four over the same M rows: bf16 as one dh_wgrad_gemm (fp32 sums in a
+    fixed order, rounded once), fp32 by the library. Rows with unit stride, 16-byte aligned."""
+    if pairs[0][0].dtype != torch.bfloat16:
+        return [torch.mm(dy.t(), x) for x, dy in pairs]
+    n, M, dev = len(pairs), pairs[0][0].shape[0], pairs[0][0].device
+    outs = [torch.empty(dy.shape[1], x.shape[1], device=dev, dtype=x.dtype) for x, dy in pairs]
+    vps, i64s, i32s = ctypes.c_void_p * n, ctypes.c_int64 * n, ctypes.c_int * n
+    K, N = i32s(*[x.shape[1] for x, _ in pairs]), i32s(*[dy.shape[1] for _, dy in pairs])
+    nbytes = _hip.lib.dh_wgrad_gemm_workspace_bytes(M, n, N, K)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)
+    st = _hip.lib.dh_wgrad_gemm(
+        _hip.DH_BF16, M, n, vps(*[x.data_ptr() for x, _ in pairs]), i64s(*[x.stride(0) for x, _ in pairs]), K,
+        vps(*[dy.data_ptr() for _, dy in pairs]), i64s(*[dy.stride(0) for _, dy in pairs]), N,
+        vps(*[o.data_ptr() for o in outs]), _hip.ptr(ws), ws.numel(), _hip.stream_handle(dev))
+    _hip.check(st, "dh_wgrad_gemm")
+    return outs
+
+
+def _plain_linear(l, dtype, n_in):
+    """A bias-free nn.Linear itself (no subclass, adapter, parametrization or hook that a direct use of its weight would
+    pass by) with a plain contiguous weight of this dtype and input width."""
+    w = l.weight if type(l) is nn.Linear else None
+    return (w is not None and l.bias is None and type(w) in (torch.Tensor, nn.Parameter) and w.dtype == dtype
+            and w.shape[1] == n_in and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and not (l._forward_hooks or l._forward_pre_hooks or l._backward_hooks or l._backward_pre_hooks))
+
+
+# ---------------------------------------------------------------------------------------------
+# dispatcher::mixer_train
+# ---------------------------------------------------------------------------------------------
+def mixer_fits(mixer, x, mask, n_lv):
+    """Whether dispatcher::mixer_train takes this layer and input: one dtype (fp32 or bf16) throughout and no autocast,
+    plain bias-free projections, and the training scan's limits."""
+    d, H, dt = mixer.embed_dim, mixer.num_heads, x.dtype
+    if not (x.dim() == 3 and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
+            and dt in (torch.float32, torch.bfloat16) and x.shape[-1] == d
+            and not torch.is_autocast_enabled("cuda") and d == SCAN_HEAD * H and H <= 64 and x.shape[1] <= SCAN_MAX_LEN
+            and n_lv <= SCAN_MAX_LEVELS and not mask.requires_grad
+            and x.numel() * 3 * x.element_size() < 2 ** 31):                   # 32-bit offsets within the (rows, 3 d) buffers
+        return False
+    if not all(w.dtype == dt and b.dtype == dt for w, b in mixer._gate_params()):
+        return False
+    return all(_plain_linear(l, dt, d) and l.weight.shape[0] == d
+               for l in (mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src, mixer.linear_out))
+
+
+@torch.library.custom_op("dispatcher::mixer_train", mutates_args=(), device_types="cuda")
+def _mixer_train_op(x: torch.Tensor, W_in: torch.Tensor, W_x: torch.Tensor, W_s: torch.Tensor, Wi: torch.Tensor,
+                    Wf: torch.Tensor, Wr: torch.Tensor, bi: torch.Tensor, bf: torch.Tensor, br: torch.Tensor,
+                    W_out: torch.Tensor, mask: torch.Tensor, num_heads: int, n_lv: int) -> List[torch.Tensor]:
+    b, T, d = x.shape
+    x2 = _rows16(x.reshape(b * T, d), 8)
+    W_cat = torch.cat((W_in, W_x, W_s))
+    proj = _linear(x2, W_cat, PROJ_GEMM_MAX_ROWS)                              # rows [V0 | A | B]
+    V0, A, B = proj.view(b, T, 3 * d).split(d, -1)
+    V, pre, states = _gate_scan_fwd(A, B, (Wi, Wf, Wr), (bi, bf, br), mask, V0, num_heads, n_lv, "dispatcher::mixer_train")
+    y = _linear(V.view(b * T, d), W_out, OUT_GEMM_MAX_ROWS)
+    return [y.view(b, T, d), proj, V, pre, states, W_cat]
+
+
+@_mixer_train_op.register_fake
+def _(x, W_in, W_x, W_s, Wi, Wf, Wr, bi, bf, br, W_out, mask, num_heads, n_lv):
+    b, T, d = x.shape
+    return [x.new_empty(b, T, d), x.new_empty(b * T, 3 * d), x.new_empty(b, T, d), _gate_rows(b, num_heads, n_lv, T, x),
+            x.new_empty(n_lv - 1, b, T, d), x.new_empty(3 * d, d)]
+
+
+@torch.library.custom_op("dispatcher::mixer_train_bwd", mutates_args=(), device_types="cuda")
+def _mixer_train_bwd_op(dy: torch.Tensor, x: torch.Tensor, Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
+                        W_out: torch.Tensor, mask: torch.Tensor, proj: torch.Tensor, V: torch.Tensor, pre: torch.Tensor,
+                        states: torch.Tensor, W_cat: torch.Tensor, num_heads: int, n_lv: int, need_dx: bool,
+                        need_dw: bool) -> List[torch.Tensor]:
+    b, T, d = x.shape
+    x2, dy2 = _rows16(x.reshape(b * T, d), 8), _rows16(dy.reshape(b * T, d).to(x.dtype), 8)
+    dV = torch.mm(dy2, W_out).view(b, T, d)
+    dproj = torch.empty_like(proj)                                             # rows [dV0 | dA | dB]
+    V0, A, B = proj.view(b, T, 3 * d).split(d, -1)
+    dV0, dA, dB = dproj.view(b, T, 3 * d).split(d, -1)
+    gates = _gate_grads(Wi, d, x.dtype, x.device)
+    _gate_scan_bwd(A, B, (Wi, Wf, Wr), mask, V0, pre, states, dV, dV0, [dA, dB] + gates, num_heads, n_lv,
+                   "dispatcher::mixer_train_bwd")
+    dx = torch.mm(dproj, W_cat).view(b, T, d) if need_dx else x.new_empty(0)
+    if need_dw:
+        dws = weight_grads([(x2, g) for g in dproj.split(d, -1)] + [(V.view(b * T, d), dy2)])
+    else:
+        dws = [x.new_empty(0) for _ in range(4)]
+    return [dx] + dws + gates
+
+
+@_mixer_train_bwd_op.register_fake
+def _(dy, x, Wi, Wf, Wr, W_out, mask, proj, V, pre, states, W_cat, num_heads, n_lv, need_dx, need_dw):
+    d = x.shape[-1]
+    return ([x.new_empty(x.shape if need_dx else 0)] + [x.new_empty((d, d) if need_dw else 0) for _ in range(4)]
+            + _gate_grads(Wi, d, x.dtype, x.device))
+
+
+def _mixer_setup(ctx, inputs, output):
+    x, W_in, W_x, W_s, Wi, Wf, Wr, bi, bf, br, W_out, mask, num_heads, n_lv = inputs
+    ctx.set_materialize_grads(False)
+    ctx.save_for_backward(x, Wi, Wf, Wr, W_out, mask, *output[1:])
+    ctx.sizes = (num_heads, n_lv)
+
+
+def _mixer_backward(ctx, grads):
+    dy = grads[0]
+    if dy is None:
+        return (None,) * 14
+    need = ctx.needs_input_grad
+    need_dx, need_dw = bool(need[0]), any(need[i] for i in (1, 2, 3, 10))
+    dx, dw_in, dw_x, dw_s, dw_out, *gates = torch.ops.dispatcher.mixer_train_bwd(
+        dy, *ctx.saved_tensors, *ctx.sizes, need_dx, need_dw)
+    g = [dx, dw_in, dw_x, dw_s, *gates, dw_out]
+    return (*[v if n else None for v, n in zip(g, need)], None, None, None)
+
+
+torch.library.register_autograd("dispatcher::mixer_train", _mixer_backward, setup_context=_mixer_setup)
+
+
+def mixer_train(mixer, x, mask, n_lv):
+    """A DispatcherMixer's output (b, T, d), differentiable in x and every parameter (reference
+    dispatcher_hybrid/modeling_dispatcher.py:63-123): one product for the three input projections, the gate path of
+    gate_scan_train, the output projection; one backward, in which the four weight gradients are one launch. See
+    mixer_fits."""
+    (Wi, bi), (Wf, bf), (Wr, br) = mixer._gate_params()
+    return torch.ops.dispatcher.mixer_train(x, mixer.linear_in.weight, mixer.gate_hidden.weight,
+                                            mixer.gate_hidden_src.weight, Wi, Wf, Wr, bi, bf, br, mixer.linear_out.weight,
+                                            mask, mixer.num_heads, n_lv)[0]

@@ -161,21 +161,24 @@ class DispatcherMixer(nn.Module):
         if not x.is_cuda:
             raise RuntimeError("fused gates are enabled but the input is on the CPU; move the model "
                                "to the GPU or call enable_fused_gates(False)")
-        from .fused_gates import (fused_gate_preacts, fused_gate_scan, gate_scan_train, input_projections,
-                                  train_scan_fits)
+        from .fused_gates import fused_gate_preacts, fused_gate_scan, input_projections
         Bb, T = x.shape[0], x.shape[1]
         H, hd = self.num_heads, self.head_dim
         needs_grad = torch.is_grad_enabled() and (
             x.requires_grad or any(p.requires_grad for p in self.parameters()))
         if needs_grad:
+            from . import fused_train as ft
+            if ft.mixer_fits(self, x, mask, n_lv):
+                # the whole layer as one operation with its own backward
+                return ft.mixer_train(self, x, mask, n_lv)
             V0, A, Bs = self.linear_in(x), self.gate_hidden(x), self.gate_hidden_src(x)
         else:
             V0, A, Bs = input_projections(x, self)
         m3 = mask[..., :n_lv] if mask.dim() == 3 else None
         (Wi, bi), (Wf, bf), (Wr, br) = self._gate_params()
-        if needs_grad and train_scan_fits(A, Bs, V0, mask, H, n_lv):
+        if needs_grad and ft.scan_fits(A, Bs, V0, mask, H, n_lv):
             # differentiable: pre-activations and level scan as one operation with its own backward
-            V = gate_scan_train(A, Bs, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, H)
+            V = ft.gate_scan_train(A, Bs, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, H)
         elif needs_grad:
             # the other head widths, lengths and dtypes: fused pre-activations + torch scan
             pre_i, pre_f, pre_r = fused_gate_preacts(A, Bs, Wi, Wf, Wr, bi, bf, br, n_lv, m3)
@@ -526,7 +529,7 @@ class DispatcherHybridForCausalLM(DispatcherPreTrainedModel, GenerationMixin):
         middle of a forward. The fused path needs GPU tensors; returns self.
         """
         if enabled:
-            from . import fused_attention, fused_gates  # noqa: F401  (fail now, not mid-forward)
+            from . import fused_attention, fused_gates, fused_train  # noqa: F401  (fail now, not mid-forward)
         for blk in self.blocks:
             if hasattr(blk, "mixer"):
                 blk.mixer.use_fused_gates = bool(enabled)

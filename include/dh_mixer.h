@@ -110,7 +110,7 @@ int dh_gate_preacts_bwd(int dtype, const void* A, const void* B, int64_t stride_
  * The same backward on the matrix cores, with caller scratch: every sum in fp32 and in a fixed order (no atomics), the
  * gradients of A, B and the readouts in `out_dtype` (DH_F32, or DH_BF16 for bf16 inputs), rounded once.
  *   dP_x      dtype `dtype`, element [b,t,l,h] at b*stride_pb + t*stride_pt + l*stride_pl + h*stride_ph
- *   dA, dB    (b, T, GH); dW_x (levels, H, GH); db_x (levels, H), contiguous; levels >= n_lv, zeros from level n_lv on
+ *   dA, dB    rows of GH at b*stride_gb + t*stride_gt (multiples of 8); dW_x (levels, H, GH); db_x (levels, H), contiguous; levels >= n_lv, zeros from level n_lv on
  *   workspace 16-byte aligned, at least dh_gate_preacts_bwd_workspace_bytes (-1 for refused sizes)
  */
 int64_t dh_gate_preacts_bwd_workspace_bytes(int dtype, int b, int T, int GH, int H, int n_lv);
@@ -119,8 +119,8 @@ int dh_gate_preacts_bwd_ws(int dtype, const void* A, const void* B, int64_t stri
                            int64_t stride_wh, const void* dPi, const void* dPf, const void* dPr,
                            int64_t stride_pb, int64_t stride_pt, int64_t stride_pl, int64_t stride_ph,
                            const void* mask, int64_t stride_mb, int64_t stride_mt, int64_t stride_ml,
-                           int out_dtype, void* dA, void* dB, void* dWi, void* dWf, void* dWr, void* dbi,
-                           void* dbf, void* dbr, int levels, int b, int T, int GH, int H, int n_lv,
+                           int out_dtype, void* dA, void* dB, int64_t stride_gb, int64_t stride_gt, void* dWi,
+                           void* dWf, void* dWr, void* dbi, void* dbf, void* dbr, int levels, int b, int T, int GH, int H, int n_lv,
                            void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
@@ -157,7 +157,7 @@ int dh_level_scan_fwd(int dtype, const void* pre_i, const void* pre_f, const voi
  *             gate and blends the forget gate towards 1
  *   states    (n_lv - 1, b, T, H*hd): the states entering levels 1 .. n_lv - 1, written by the forward, read by the backward
  *   V, dV     the scanned state (contiguous) and its gradient (rows at b*stride_gb + t*stride_gt)
- *   scratch   (b, T, H*hd) of the dtype, needed for n_lv > 6; dV0 (b, T, H*hd) contiguous
+ *   scratch   (b, T, H*hd) of the dtype, needed for n_lv > 6; dV0 rows at b*stride_ob + t*stride_ot
  */
 int dh_level_scan_train_fwd(int dtype, const void* pre_i, const void* pre_f, const void* pre_r, int64_t stride_pb,
                             int64_t stride_pl, int64_t stride_ph, const void* mask, int64_t stride_mb,
@@ -168,8 +168,20 @@ int dh_level_scan_train_bwd(int dtype, const void* pre_i, const void* pre_f, con
                             int64_t stride_pl, int64_t stride_ph, const void* mask, int64_t stride_mb,
                             int64_t stride_mt, int64_t stride_ml, const void* V0, int64_t stride_vb,
                             int64_t stride_vt, const void* states, const void* dV, int64_t stride_gb,
-                            int64_t stride_gt, void* scratch, void* dV0, void* dpre_i, void* dpre_f, void* dpre_r,
-                            int b, int T, int H, int hd, int n_lv, void* stream);
+                            int64_t stride_gt, void* scratch, void* dV0, int64_t stride_ob, int64_t stride_ot,
+                            void* dpre_i, void* dpre_f, void* dpre_r, int b, int T, int H, int hd, int n_lv,
+                            void* stream);
+
+/*
+ * Weight gradients of up to four bias-free linear layers over the same M rows, bf16: dW[s] (N[s], K[s]) contiguous =
+ * dY[s]^T X[s] with X[s] (M, K[s]) rows ldx[s] apart and dY[s] (M, N[s]) rows ldy[s] apart (multiples of 8, 16-byte
+ * aligned, below 2 GiB each); fp32 sums in a fixed order, rounded once. X, ldx, K, dY, ldy, N, dW are host arrays.
+ * workspace: dh_wgrad_gemm_workspace_bytes (0: none needed, -1: refused sizes), 16-byte aligned.
+ */
+int64_t dh_wgrad_gemm_workspace_bytes(int M, int nseg, const int* N, const int* K);
+int dh_wgrad_gemm(int dtype, int M, int nseg, const void* const* X, const int64_t* ldx, const int* K,
+                  const void* const* dY, const int64_t* ldy, const int* N, void* const* dW, void* workspace,
+                  int64_t workspace_bytes, void* stream);
 
 /*
  * The feed-forward block's SwiGLU activation over n elements:

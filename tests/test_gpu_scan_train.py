@@ -41,7 +41,7 @@ CASES = [  # b, T, H, mask kind ("level", "doc", "soft": fractional values)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("b,T,H,kind", CASES)
 def test_gate_scan_train_against_float64(b, T, H, kind, dtype):
-    from dispatcher_hybrid.fused_gates import gate_scan_train
+    from dispatcher_hybrid.fused_train import gate_scan_train
     g = torch.Generator(device=DEV).manual_seed(T + H)
     rn = lambda *s: torch.randn(*s, device=DEV, generator=g)
     d, L = 64 * H, 12
@@ -100,7 +100,7 @@ def test_gate_scan_train_matches_module_fallback():
 def test_gate_scan_train_under_checkpoint_and_autocast():
     """Activation checkpointing recomputes the operation; under autocast (bf16 activations, fp32 weights) the weights'
     gradients come back in fp32."""
-    from dispatcher_hybrid.fused_gates import gate_scan_train
+    from dispatcher_hybrid.fused_train import gate_scan_train
     from torch.utils.checkpoint import checkpoint
     g = torch.Generator(device=DEV).manual_seed(1)
     b, T, H, L = 1, 100, 2, 7
@@ -114,3 +114,73 @@ def test_gate_scan_train_under_checkpoint_and_autocast():
     again = torch.autograd.grad(checkpoint(f, *leaves, use_reentrant=False).float().square().sum(), leaves)
     assert all(p.dtype == x.dtype for p, x in zip(plain, leaves))
     assert all(torch.equal(p, q) for p, q in zip(plain, again))
+
+
+def _mixer(dtype, d=128, max_len=256):
+    from dispatcher_hybrid import DispatcherConfig
+    from dispatcher_hybrid.modeling_dispatcher import DispatcherMixer
+    torch.manual_seed(5)
+    mx = DispatcherMixer(DispatcherConfig(d_model=d, num_heads=d // 64, max_len=max_len, num_layers=1, attn_layers=(),
+                                          vocab_size=64, dim_feedforward=128)).to(DEV, dtype)
+    with torch.no_grad():
+        for n, p in mx.named_parameters():
+            if "bias" not in n:
+                p.normal_(std=0.08)
+    return mx
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5), (torch.bfloat16, 2.5e-2)])
+@pytest.mark.parametrize("b,T", [(1, 1), (2, 65), (3, 256)])
+def test_mixer_train_against_float64_eager(b, T, dtype, tol):
+    """The whole-layer operation against the eager mixer in float64 (tolerances as above)."""
+    mx = _mixer(dtype)
+    ref = _mixer(torch.float64)
+    ref.load_state_dict({n: p.double() for n, p in mx.state_dict().items()})
+    mx.use_fused_gates = True
+    t = torch.arange(T, device=DEV).unsqueeze(1)
+    lag = 1 << torch.arange(8, device=DEV)
+    mask = ((t >= lag) & (lag < T)).to(dtype)
+    x = torch.randn(b, T, 128, device=DEV).to(dtype).requires_grad_()
+    x64 = x.detach().double().requires_grad_()
+    dy = torch.randn(b, T, 128, device=DEV).to(dtype)
+    y, y64 = mx(x, mask), ref(x64, mask.double())
+    y.backward(dy)
+    y64.backward(dy.double())
+    pairs = [("y", y, y64), ("dx", x.grad, x64.grad)]
+    pairs += [(n, p.grad, q.grad) for (n, p), q in zip(mx.named_parameters(), ref.parameters())]
+    for n, a, e in pairs:
+        assert a.dtype == dtype
+        assert (a.double() - e).norm() <= tol * e.norm() + 1e-30, (n, ((a.double() - e).norm() / e.norm()).item())
+
+
+def test_mixer_train_partial_gradients_hooks_and_adapters():
+    """Frozen inputs or weights get no gradient; a hooked or replaced projection keeps being called."""
+    mx = _mixer(torch.float32)
+    mx.use_fused_gates = True
+    t = torch.arange(40, device=DEV).unsqueeze(1)
+    mask = (t >= (1 << torch.arange(8, device=DEV))).float()
+    x = torch.randn(1, 40, 128, device=DEV)
+    full = mx(x, mask)
+    full.sum().backward()
+    want = {n: p.grad.clone() for n, p in mx.named_parameters()}
+    mx.zero_grad()
+    for n, p in mx.named_parameters():
+        p.requires_grad_(n in ("gate_out", "reset_out_bias"))
+    mx(x, mask).sum().backward()
+    assert mx.linear_in.weight.grad is None
+    assert torch.equal(mx.gate_out.grad, want["gate_out"]) and torch.equal(mx.reset_out_bias.grad, want["reset_out_bias"])
+    mx.requires_grad_(True)
+    calls = []
+    handle = mx.gate_hidden.register_forward_hook(lambda m, i, o: calls.append(1))
+    hooked = mx(x, mask)
+    handle.remove()
+    assert calls and (hooked - full).norm() <= 2e-5 * full.norm()
+
+    class Adapter(torch.nn.Linear):
+        def forward(self, h):
+            return 2 * super().forward(h)
+
+    ad = Adapter(128, 128, bias=False).to(DEV)
+    ad.weight = mx.linear_out.weight
+    mx.linear_out = ad
+    assert (mx(x, mask) - 2 * full).norm() <= 4e-5 * full.norm()

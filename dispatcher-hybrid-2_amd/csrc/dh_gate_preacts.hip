@@ -41,9 +41,9 @@ struct FwdArgs {
   const void* Wf;
   const void* Wr;
   int64_t swl, swh;
-  const float* bi;
-  const float* bf;
-  const float* br;
+  const void* bi;               // fp32, or T with bias_t
+  const void* bf;
+  const void* br;
   const void* mask;
   int64_t smb, smt, sml;
   void* oi;
@@ -53,7 +53,13 @@ struct FwdArgs {
   int b, T, GH, H, n_lv;
   int vec_out;                  // outputs take 4-position vector stores (head-major, aligned)
   int activate;                 // write the scan's gates a, f, r instead of pre-activations
+  int bias_t;
 };
+
+template <typename T>
+__device__ __forceinline__ float bias_at(const FwdArgs& a, const void* b, int i) {
+  return a.bias_t ? Elem<T>::load((const T*)b + i) : ((const float*)b)[i];
+}
 
 __device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 
@@ -263,7 +269,7 @@ __global__ __launch_bounds__(kThreads) void gate_preacts_fwd_kernel(FwdArgs a) {
     for (int j = 0; j < LG; ++j) {
       const int l = l0 + j;
       if (l >= a.n_lv || n >= a.H) continue;
-      const float bias[3] = {a.bi[l * a.H + n], a.bf[l * a.H + n], a.br[l * a.H + n]};
+      const float bias[3] = {bias_at<T>(a, a.bi, l * a.H + n), bias_at<T>(a, a.bf, l * a.H + n), bias_at<T>(a, a.br, l * a.H + n)};
       T* outs[3] = {(T*)a.oi, (T*)a.of, (T*)a.orr};
       const int64_t base = (int64_t)b * a.sob + (int64_t)l * a.sol + (int64_t)n * a.soh;
       float v[3][4];
@@ -559,7 +565,7 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
     for (int j = 0; j < LG; ++j) {
       const int l = l0 + j;
       if (l >= a.n_lv || r >= a.H) continue;
-      const float bias[3] = {a.bi[l * a.H + r], a.bf[l * a.H + r], a.br[l * a.H + r]};
+      const float bias[3] = {bias_at<T>(a, a.bi, l * a.H + r), bias_at<T>(a, a.bf, l * a.H + r), bias_at<T>(a, a.br, l * a.H + r)};
       T* outs[3] = {(T*)a.oi, (T*)a.of, (T*)a.orr};
       const int64_t base = (int64_t)b * a.sob + (int64_t)l * a.sol + (int64_t)r * a.soh;
       float v[3][4];
@@ -795,7 +801,7 @@ void dispatch_fwd(const FwdArgs& a, int LG, int KU, dim3 grid, hipStream_t s) {
 
 extern "C" int dh_gate_preacts_fwd(int dtype, const void* A, const void* B, int64_t stride_ab, int64_t stride_at,
                                    const void* Wi, const void* Wf, const void* Wr, int64_t stride_wl,
-                                   int64_t stride_wh, const float* bi, const float* bf, const float* br,
+                                   int64_t stride_wh, const void* bi, const void* bf, const void* br,
                                    const void* mask, int64_t stride_mb, int64_t stride_mt, int64_t stride_ml,
                                    void* out_i, void* out_f, void* out_r, int64_t stride_ob, int64_t stride_ot,
                                    int64_t stride_ol, int64_t stride_oh, int activate, int b, int T, int GH,
@@ -822,7 +828,7 @@ extern "C" int dh_gate_preacts_fwd(int dtype, const void* A, const void* B, int6
                        aligned(out_i, 4 * esz) && aligned(out_f, 4 * esz) && aligned(out_r, 4 * esz);
   FwdArgs a{A, B, stride_ab, stride_at, Wi, Wf, Wr, stride_wl, stride_wh, bi, bf, br, mask, stride_mb, stride_mt,
             stride_ml, out_i, out_f, out_r, stride_ob, stride_ot, stride_ol, stride_oh, b, T, GH, H, n_lv,
-            vec_out ? 1 : 0, activate ? 1 : 0};
+            vec_out ? 1 : 0, activate & 1, (activate >> 1) & 1};
   // level groups: enough workgroups to fill 256 CUs several times over, A reused across <= 4 levels
   const int tiles = (T + kTileT - 1) / kTileT;
   const int64_t tile_wgs = (int64_t)tiles * b;

@@ -25,10 +25,10 @@ Importing this module loads the kernel library and raises ImportError if it is m
 """
 
 import ctypes
-import weakref
 from typing import List, Optional
 
 import torch
+import torch.nn as nn
 
 from . import _hip
 
@@ -55,29 +55,9 @@ def _preacts_launch(A_, B_, Wi_, Wf_, Wr_, bi_, bf_, br_, mask, outs, ostrides, 
         _hip.dtype_code(cd), p(A_), p(B_), A_.stride(0), A_.stride(1),
         p(Wi_), p(Wf_), p(Wr_), Wi_.stride(0), Wi_.stride(1),
         p(bi_), p(bf_), p(br_), p(m_), smb, smt, sml,
-        p(outs[0]), p(outs[1]), p(outs[2]), *ostrides, int(activate),
+        p(outs[0]), p(outs[1]), p(outs[2]), *ostrides, int(activate) | (2 if bi_.dtype == cd else 0),
         b, T, GH, H, n_lv, _hip.stream_handle(A_.device))
     _hip.check(st, what)
-
-
-# fp32 copies of bf16 gate biases (the kernel reads fp32 biases), one per bias tensor, refreshed
-# when the tensor's version counter moves (an in-place update): three cast launches per layer and
-# forward otherwise. A HIP graph captured over a forward keeps the copy it was captured with.
-# (keyed by id, with a weak reference that drops the entry when the tensor goes: a tensor cannot
-# be a WeakKeyDictionary key, whose lookups compare keys with ==)
-_BIAS_F32 = {}
-
-
-def _bias_f32(v, n_lv):
-    if v.dtype == torch.float32 or (v.requires_grad and torch.is_grad_enabled()):
-        return v[:n_lv].contiguous().float()
-    k = id(v)
-    ent = _BIAS_F32.get(k)
-    if ent is None or ent[0]() is not v or ent[1] != v._version or ent[2] != n_lv:
-        ref = weakref.ref(v, lambda _r, k=k: _BIAS_F32.pop(k, None))
-        ent = (ref, v._version, n_lv, v[:n_lv].contiguous().float())
-        _BIAS_F32[k] = ent
-    return ent[3]
 
 
 def _prep_gate_inputs(A, B, Wi, Wf, Wr, bi, bf, br, n_lv):
@@ -85,7 +65,9 @@ def _prep_gate_inputs(A, B, Wi, Wf, Wr, bi, bf, br, n_lv):
     A_ = A.contiguous().to(cd)
     B_ = B.contiguous().to(cd)
     Wi_, Wf_, Wr_ = (w[:n_lv].contiguous().to(cd) for w in (Wi, Wf, Wr))
-    bi_, bf_, br_ = (_bias_f32(v, n_lv) for v in (bi, bf, br))
+    # the kernel reads biases of the compute dtype as they are, others as fp32 copies
+    bd = cd if bi.dtype == bf.dtype == br.dtype == cd else torch.float32
+    bi_, bf_, br_ = (v[:n_lv].contiguous().to(bd) for v in (bi, bf, br))
     return A_, B_, Wi_, Wf_, Wr_, bi_, bf_, br_
 
 
@@ -280,21 +262,17 @@ def fused_level_scan(pre_i, pre_f, pre_r, mask, V0, num_heads, n_lv):
 # ---------------------------------------------------------------------------------------------
 # dispatcher::gate_scan_fwd -- the whole inference gate path in two launches
 # ---------------------------------------------------------------------------------------------
-@torch.library.custom_op("dispatcher::gate_scan_fwd", mutates_args=(), device_types="cuda")
-def _gate_scan_fwd_op(A: torch.Tensor, B: torch.Tensor,
-                      Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
-                      bi: torch.Tensor, bf: torch.Tensor, br: torch.Tensor,
-                      mask: Optional[torch.Tensor], V0: torch.Tensor, num_heads: int,
-                      n_lv: int) -> torch.Tensor:
+def _gate_scan_body(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv):
     b, T, d = V0.shape
     out = torch.empty(b, T, d, device=V0.device, dtype=V0.dtype)
     if b == 0 or T == 0:
         return out
     ins = _prep_gate_inputs(A, B, Wi, Wf, Wr, bi, bf, br, n_lv)
     H = num_heads
-    # activated gates in the head-major (b, H, n_lv, T) layout: unit stride along t for the scan
-    g = torch.empty(3, b, H, n_lv, T, device=V0.device, dtype=ins[0].dtype)
-    gates = [g[i].permute(0, 3, 2, 1) for i in range(3)]              # logical (b, T, n_lv, H)
+    # activated gates in the head-major (b, H, n_lv, T) layout: unit stride along t for the scan, rows padded to 8
+    # positions so they start aligned whatever T is
+    g = torch.empty(3, b, H, n_lv, -(-T // 8) * 8, device=V0.device, dtype=ins[0].dtype)
+    gates = [x.permute(0, 3, 2, 1)[:, :T] for x in g]                 # logical (b, T, n_lv, H)
     _preacts_launch(*ins, mask, gates, gates[0].stride(), 1, n_lv, "dispatcher::gate_scan_fwd")
     cd = ins[0].dtype
     res = out if V0.dtype == cd else torch.empty(b, T, d, device=V0.device, dtype=cd)
@@ -302,6 +280,15 @@ def _gate_scan_fwd_op(A: torch.Tensor, B: torch.Tensor,
     if res is not out:
         out.copy_(res)
     return out
+
+
+@torch.library.custom_op("dispatcher::gate_scan_fwd", mutates_args=(), device_types="cuda")
+def _gate_scan_fwd_op(A: torch.Tensor, B: torch.Tensor,
+                      Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
+                      bi: torch.Tensor, bf: torch.Tensor, br: torch.Tensor,
+                      mask: Optional[torch.Tensor], V0: torch.Tensor, num_heads: int,
+                      n_lv: int) -> torch.Tensor:
+    return _gate_scan_body(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
 
 
 @_gate_scan_fwd_op.register_fake
@@ -317,6 +304,8 @@ def fused_gate_scan(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, num_heads):
     fused_level_scan(*fused_gate_preacts(...), mask, V0, num_heads, n_lv) up to the bf16 rounding
     of the activated gates, which follows the eager path (reference
     dispatcher_hybrid/modeling_dispatcher.py:86-88, 100-121)."""
+    if type(A) is torch.Tensor and not torch.compiler.is_compiling() and not transforms_active():
+        return _gate_scan_body(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
     return torch.ops.dispatcher.gate_scan_fwd(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
 
 
@@ -427,6 +416,60 @@ def project(x, linears, max_rows):
     if rows <= max_rows and projections_fit(x, linears):
         return fused_projections(x, [l.weight for l in linears])
     return [l(x) for l in linears]
+
+
+# whether a torch.func transform (grad, vmap, ...) wraps the tensors: their memory cannot be handed to a kernel directly
+transforms_active = getattr(torch._C, "_are_functorch_transforms_active", lambda: False)
+
+
+def plain_linear(l, dtype, n_in):
+    """A bias-free nn.Linear itself (no subclass, adapter, parametrization or hook that a direct use of its weight would
+    pass by) with a plain contiguous weight of this dtype and input width."""
+    w = l.weight if type(l) is nn.Linear else None
+    return (w is not None and l.bias is None and type(w) in _PLAIN and w.dtype == dtype
+            and w.shape[1] == n_in and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and not (l._forward_hooks or l._forward_pre_hooks or l._backward_hooks or l._backward_pre_hooks))
+
+
+_PLAIN = (torch.Tensor, nn.Parameter)
+
+
+def mixer_layer_fits(mixer, x):
+    """Whether mixer_layer takes this layer and input: few enough rows that both products run on dh_proj_gemm, one dtype
+    throughout, plain bias-free projections, plain eager execution."""
+    if torch.compiler.is_compiling() or transforms_active():
+        return False
+    d, dt = mixer.embed_dim, x.dtype
+    return (x.dim() == 3 and type(x) in _PLAIN and dt in (torch.float32, torch.bfloat16) and x.shape[-1] == d
+            and 0 < x.shape[0] * x.shape[1] <= OUT_GEMM_MAX_ROWS and d % 64 == 0
+            and all(w.dtype == dt and b.dtype == dt and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
+                    and w.shape[-1] == d for w, b in mixer._gate_params())
+            and all(plain_linear(l, dt, d) and l.weight.shape[0] == d
+                    for l in (mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src, mixer.linear_out)))
+
+
+def mixer_layer(mixer, x, mask, n_lv):
+    """A DispatcherMixer's output (b, T, d) in one native call (``dh_mixer_fwd``: the launches of fused_projections,
+    fused_gate_scan and the output projection, with their results). `mask`: the (b, T, L) document mask, or None. Inference
+    only; see mixer_layer_fits."""
+    b, T, d = x.shape
+    dt, H = x.dtype, mixer.num_heads
+    x2 = _rows16(x.reshape(b * T, d), 8)
+    if mask is not None and mask.shape[0] != b:
+        mask = mask.expand(b, -1, -1)
+    m, smb, smt, sml = _mask_view(mask, dt)
+    code = _hip.dtype_code(dt)
+    nbytes = _hip.lib.dh_mixer_fwd_scratch_bytes(code, b, T, d, H, n_lv)
+    scratch = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
+    y = torch.empty(b, T, d, device=x.device, dtype=dt)
+    p = _hip.ptr
+    (Wi, bi), (Wf, bf), (Wr, br) = mixer._gate_params()
+    st = _hip.lib.dh_mixer_fwd(
+        code, p(x2), x2.stride(0), p(mixer.linear_in.weight), p(mixer.gate_hidden.weight), p(mixer.gate_hidden_src.weight),
+        p(Wi), p(Wf), p(Wr), p(bi), p(bf), p(br), p(mixer.linear_out.weight), p(m), smb, smt, sml, p(y), p(scratch),
+        scratch.numel(), b, T, d, H, n_lv, _hip.stream_handle(x.device))
+    _hip.check(st, "dh_mixer_fwd")
+    return y
 
 
 def swiglu_fits(x, gate, up):

@@ -1,7 +1,7 @@
 """Training passes of the fused layers on gfx950 kernels, each one operation with one backward.
 
     dispatcher::gate_scan_train   gate pre-activations + level scan (from the projections A, B, V0)
-    dispatcher::mixer_train       a whole mixer layer: projections, gate path, output projection
+    mixer_train                   a whole mixer layer: projections, gate path, output projection
 
 Both run under ``model.enable_fused_gates()`` when gradients are wanted (DispatcherMixer picks the widest one that fits)
 and replace the reference's eager autograd of the level loop (reference dispatcher_hybrid/modeling_dispatcher.py:86-121)
@@ -20,8 +20,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _hip
-from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch, _preacts_launch, _rows16,
-                          fused_projections)
+from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch,
+                          _preacts_launch, _rows16, fused_projections, plain_linear, transforms_active)
 
 SCAN_MAX_LEN = 4096
 SCAN_MAX_LEVELS = 12
@@ -53,11 +53,12 @@ def _gate_scan_fwd(A, B, W, bias, mask, V0, H, n_lv, what):
     V = torch.empty(b, T, d, device=dev, dtype=cd)
     pre = _gate_rows(b, H, n_lv, T, A)
     states = torch.empty(n_lv - 1, b, T, d, device=dev, dtype=cd)
+    bd = cd if all(v.dtype == cd for v in bias) else torch.float32             # (other biases: fp32 copies)
     W = [_rows16(w[:n_lv].contiguous().to(cd), 8) for w in W]
-    bias = torch.stack(tuple(bias))[:, :n_lv].float().contiguous()             # the kernel reads fp32 biases
+    bias = [v[:n_lv].contiguous().to(bd) for v in bias]
     m = _scan_mask(mask, b, T, n_lv, cd)
     gates = [g[..., :T].permute(0, 3, 2, 1) for g in pre]                      # logical (b, T, n_lv, H)
-    _preacts_launch(A, B, *W, bias[0], bias[1], bias[2], m if mask.dim() == 3 else None, gates, gates[0].stride(), 0,
+    _preacts_launch(A, B, *W, *bias, m if mask.dim() == 3 else None, gates, gates[0].stride(), 0,
                     n_lv, what)
     p = _hip.ptr
     st = _hip.lib.dh_level_scan_train_fwd(
@@ -196,21 +197,15 @@ def weight_grads(pairs):
     return outs
 
 
-def _plain_linear(l, dtype, n_in):
-    """A bias-free nn.Linear itself (no subclass, adapter, parametrization or hook that a direct use of its weight would
-    pass by) with a plain contiguous weight of this dtype and input width."""
-    w = l.weight if type(l) is nn.Linear else None
-    return (w is not None and l.bias is None and type(w) in (torch.Tensor, nn.Parameter) and w.dtype == dtype
-            and w.shape[1] == n_in and w.is_contiguous() and w.data_ptr() % 16 == 0
-            and not (l._forward_hooks or l._forward_pre_hooks or l._backward_hooks or l._backward_pre_hooks))
-
-
 # ---------------------------------------------------------------------------------------------
-# dispatcher::mixer_train
+# a whole mixer layer
 # ---------------------------------------------------------------------------------------------
 def mixer_fits(mixer, x, mask, n_lv):
-    """Whether dispatcher::mixer_train takes this layer and input: one dtype (fp32 or bf16) throughout and no autocast,
-    plain bias-free projections, and the training scan's limits."""
+    """Whether mixer_train takes this layer and input: one dtype (fp32 or bf16) throughout and no autocast, plain bias-free
+    projections, the training scan's limits, and plain eager execution (a compiler gets the layer-by-layer form,
+    whose gate path is one registered operation, and a torch.func transform that operation's refusal)."""
+    if torch.compiler.is_compiling() or transforms_active():
+        return False
     d, H, dt = mixer.embed_dim, mixer.num_heads, x.dtype
     if not (x.dim() == 3 and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
             and dt in (torch.float32, torch.bfloat16) and x.shape[-1] == d
@@ -220,88 +215,54 @@ def mixer_fits(mixer, x, mask, n_lv):
         return False
     if not all(w.dtype == dt and b.dtype == dt for w, b in mixer._gate_params()):
         return False
-    return all(_plain_linear(l, dt, d) and l.weight.shape[0] == d
+    return all(plain_linear(l, dt, d) and l.weight.shape[0] == d
                for l in (mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src, mixer.linear_out))
 
 
-@torch.library.custom_op("dispatcher::mixer_train", mutates_args=(), device_types="cuda")
-def _mixer_train_op(x: torch.Tensor, W_in: torch.Tensor, W_x: torch.Tensor, W_s: torch.Tensor, Wi: torch.Tensor,
-                    Wf: torch.Tensor, Wr: torch.Tensor, bi: torch.Tensor, bf: torch.Tensor, br: torch.Tensor,
-                    W_out: torch.Tensor, mask: torch.Tensor, num_heads: int, n_lv: int) -> List[torch.Tensor]:
-    b, T, d = x.shape
-    x2 = _rows16(x.reshape(b * T, d), 8)
-    W_cat = torch.cat((W_in, W_x, W_s))
-    proj = _linear(x2, W_cat, PROJ_GEMM_MAX_ROWS)                              # rows [V0 | A | B]
-    V0, A, B = proj.view(b, T, 3 * d).split(d, -1)
-    V, pre, states = _gate_scan_fwd(A, B, (Wi, Wf, Wr), (bi, bf, br), mask, V0, num_heads, n_lv, "dispatcher::mixer_train")
-    y = _linear(V.view(b * T, d), W_out, OUT_GEMM_MAX_ROWS)
-    return [y.view(b, T, d), proj, V, pre, states, W_cat]
+class _MixerTrain(torch.autograd.Function):
+    """A mixer layer; see mixer_train. An autograd function rather than a registered
+    operation: the latter's per-call bookkeeping is ~150 us of host time a direction, as much as a small layer's kernels."""
 
+    @staticmethod
+    def forward(ctx, x, W_in, W_x, W_s, Wi, Wf, Wr, bi, bf, br, W_out, mask, num_heads, n_lv):
+        b, T, d = x.shape
+        x2 = _rows16(x.reshape(b * T, d), 8)
+        W_cat = torch.cat((W_in, W_x, W_s))
+        proj = _linear(x2, W_cat, PROJ_GEMM_MAX_ROWS)                          # rows [V0 | A | B]
+        V0, A, B = proj.view(b, T, 3 * d).split(d, -1)
+        V, pre, states = _gate_scan_fwd(A, B, (Wi, Wf, Wr), (bi, bf, br), mask, V0, num_heads, n_lv, "mixer_train")
+        y = _linear(V.view(b * T, d), W_out, OUT_GEMM_MAX_ROWS)
+        ctx.save_for_backward(x, Wi, Wf, Wr, W_out, mask, proj, V, pre, states, W_cat)
+        ctx.sizes = (num_heads, n_lv)
+        return y.view(b, T, d)
 
-@_mixer_train_op.register_fake
-def _(x, W_in, W_x, W_s, Wi, Wf, Wr, bi, bf, br, W_out, mask, num_heads, n_lv):
-    b, T, d = x.shape
-    return [x.new_empty(b, T, d), x.new_empty(b * T, 3 * d), x.new_empty(b, T, d), _gate_rows(b, num_heads, n_lv, T, x),
-            x.new_empty(n_lv - 1, b, T, d), x.new_empty(3 * d, d)]
-
-
-@torch.library.custom_op("dispatcher::mixer_train_bwd", mutates_args=(), device_types="cuda")
-def _mixer_train_bwd_op(dy: torch.Tensor, x: torch.Tensor, Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
-                        W_out: torch.Tensor, mask: torch.Tensor, proj: torch.Tensor, V: torch.Tensor, pre: torch.Tensor,
-                        states: torch.Tensor, W_cat: torch.Tensor, num_heads: int, n_lv: int, need_dx: bool,
-                        need_dw: bool) -> List[torch.Tensor]:
-    b, T, d = x.shape
-    x2, dy2 = _rows16(x.reshape(b * T, d), 8), _rows16(dy.reshape(b * T, d).to(x.dtype), 8)
-    dV = torch.mm(dy2, W_out).view(b, T, d)
-    dproj = torch.empty_like(proj)                                             # rows [dV0 | dA | dB]
-    V0, A, B = proj.view(b, T, 3 * d).split(d, -1)
-    dV0, dA, dB = dproj.view(b, T, 3 * d).split(d, -1)
-    gates = _gate_grads(Wi, d, x.dtype, x.device)
-    _gate_scan_bwd(A, B, (Wi, Wf, Wr), mask, V0, pre, states, dV, dV0, [dA, dB] + gates, num_heads, n_lv,
-                   "dispatcher::mixer_train_bwd")
-    dx = torch.mm(dproj, W_cat).view(b, T, d) if need_dx else x.new_empty(0)
-    if need_dw:
-        dws = weight_grads([(x2, g) for g in dproj.split(d, -1)] + [(V.view(b * T, d), dy2)])
-    else:
-        dws = [x.new_empty(0) for _ in range(4)]
-    return [dx] + dws + gates
-
-
-@_mixer_train_bwd_op.register_fake
-def _(dy, x, Wi, Wf, Wr, W_out, mask, proj, V, pre, states, W_cat, num_heads, n_lv, need_dx, need_dw):
-    d = x.shape[-1]
-    return ([x.new_empty(x.shape if need_dx else 0)] + [x.new_empty((d, d) if need_dw else 0) for _ in range(4)]
-            + _gate_grads(Wi, d, x.dtype, x.device))
-
-
-def _mixer_setup(ctx, inputs, output):
-    x, W_in, W_x, W_s, Wi, Wf, Wr, bi, bf, br, W_out, mask, num_heads, n_lv = inputs
-    ctx.set_materialize_grads(False)
-    ctx.save_for_backward(x, Wi, Wf, Wr, W_out, mask, *output[1:])
-    ctx.sizes = (num_heads, n_lv)
-
-
-def _mixer_backward(ctx, grads):
-    dy = grads[0]
-    if dy is None:
-        return (None,) * 14
-    need = ctx.needs_input_grad
-    need_dx, need_dw = bool(need[0]), any(need[i] for i in (1, 2, 3, 10))
-    dx, dw_in, dw_x, dw_s, dw_out, *gates = torch.ops.dispatcher.mixer_train_bwd(
-        dy, *ctx.saved_tensors, *ctx.sizes, need_dx, need_dw)
-    g = [dx, dw_in, dw_x, dw_s, *gates, dw_out]
-    return (*[v if n else None for v, n in zip(g, need)], None, None, None)
-
-
-torch.library.register_autograd("dispatcher::mixer_train", _mixer_backward, setup_context=_mixer_setup)
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dy):
+        x, Wi, Wf, Wr, W_out, mask, proj, V, pre, states, W_cat = ctx.saved_tensors
+        num_heads, n_lv = ctx.sizes
+        need = ctx.needs_input_grad
+        b, T, d = x.shape
+        x2, dy2 = _rows16(x.reshape(b * T, d), 8), _rows16(dy.reshape(b * T, d), 8)
+        dV = torch.mm(dy2, W_out).view(b, T, d)
+        dproj = torch.empty_like(proj)                                         # rows [dV0 | dA | dB]
+        V0, A, B = proj.view(b, T, 3 * d).split(d, -1)
+        dV0, dA, dB = dproj.view(b, T, 3 * d).split(d, -1)
+        gates = _gate_grads(Wi, d, x.dtype, x.device)
+        _gate_scan_bwd(A, B, (Wi, Wf, Wr), mask, V0, pre, states, dV, dV0, [dA, dB] + gates, num_heads, n_lv, "mixer_train")
+        dx = torch.mm(dproj, W_cat).view(b, T, d) if need[0] else None
+        dw = [None] * 4
+        if any(need[i] for i in (1, 2, 3, 10)):
+            dw = weight_grads([(x2, g) for g in dproj.split(d, -1)] + [(V.view(b * T, d), dy2)])
+        g = [dx, *dw[:3], *gates, dw[3]]
+        return (*[v if n else None for v, n in zip(g, need)], None, None, None)
 
 
 def mixer_train(mixer, x, mask, n_lv):
-    """A DispatcherMixer's output (b, T, d), differentiable in x and every parameter (reference
+    """A DispatcherMixer's output (b, T, d), differentiable (once) in x and every parameter (reference
     dispatcher_hybrid/modeling_dispatcher.py:63-123): one product for the three input projections, the gate path of
     gate_scan_train, the output projection; one backward, in which the four weight gradients are one launch. See
     mixer_fits."""
     (Wi, bi), (Wf, bf), (Wr, br) = mixer._gate_params()
-    return torch.ops.dispatcher.mixer_train(x, mixer.linear_in.weight, mixer.gate_hidden.weight,
-                                            mixer.gate_hidden_src.weight, Wi, Wf, Wr, bi, bf, br, mixer.linear_out.weight,
-                                            mask, mixer.num_heads, n_lv)[0]
+    return _MixerTrain.apply(x, mixer.linear_in.weight, mixer.gate_hidden.weight, mixer.gate_hidden_src.weight, Wi, Wf, Wr,
+                             bi, bf, br, mixer.linear_out.weight, mask, mixer.num_heads, n_lv)

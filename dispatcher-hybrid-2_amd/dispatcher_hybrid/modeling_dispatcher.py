@@ -20,7 +20,6 @@ Two implementations of the mixer, selected per module by `use_fused_gates`:
 """
 
 import math
-import sys
 
 import torch
 import torch.nn as nn
@@ -161,7 +160,8 @@ class DispatcherMixer(nn.Module):
         if not x.is_cuda:
             raise RuntimeError("fused gates are enabled but the input is on the CPU; move the model "
                                "to the GPU or call enable_fused_gates(False)")
-        from .fused_gates import fused_gate_preacts, fused_gate_scan, input_projections
+        from .fused_gates import (fused_gate_preacts, fused_gate_scan, input_projections, mixer_layer,
+                                  mixer_layer_fits)
         Bb, T = x.shape[0], x.shape[1]
         H, hd = self.num_heads, self.head_dim
         needs_grad = torch.is_grad_enabled() and (
@@ -172,6 +172,9 @@ class DispatcherMixer(nn.Module):
                 # the whole layer as one operation with its own backward
                 return ft.mixer_train(self, x, mask, n_lv)
             V0, A, Bs = self.linear_in(x), self.gate_hidden(x), self.gate_hidden_src(x)
+        elif mixer_layer_fits(self, x):
+            # inference on few rows: the whole layer in one native call
+            return mixer_layer(self, x, mask if mask.dim() == 3 else None, n_lv)
         else:
             V0, A, Bs = input_projections(x, self)
         m3 = mask[..., :n_lv] if mask.dim() == 3 else None
@@ -552,11 +555,9 @@ class DispatcherHybridForCausalLM(DispatcherPreTrainedModel, GenerationMixin):
         The first call for a shape runs two warm-up forwards on a side stream and captures one
         forward; every call copies input_ids into the graph's input buffer and replays. The result
         is the graph's output buffer: the next call with the same shape overwrites it (clone it to
-        keep it). The parameters must stay where they are between calls; in-place updates of the
-        weights are seen, but the fused path reads bf16 gate biases through fp32 copies made when a
-        forward runs, so after changing those call release_graphs() to capture again. The path
-        captured is the one active at the first call, so call enable_fused_gates() first for the
-        fused kernels. Bit for bit equal to self(input_ids).logits on that path.
+        keep it). The parameters must stay where they are between calls; in-place updates of them
+        are seen. The path captured is the one active at the first call, so call enable_fused_gates()
+        first for the fused kernels. Bit for bit equal to self(input_ids).logits on that path.
         """
         if not input_ids.is_cuda:
             raise ValueError("graphed_logits needs input_ids on a GPU")
@@ -574,12 +575,8 @@ class DispatcherHybridForCausalLM(DispatcherPreTrainedModel, GenerationMixin):
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph):
                 out = self(static_ids).logits
-            # the graph reads the fp32 gate-bias copies made by the warm-up forwards: keep them alive
-            # even if a later forward replaces them (after a bias update)
-            fg = sys.modules.get(__package__ + ".fused_gates")
-            keep = [e[3] for e in getattr(fg, "_BIAS_F32", {}).values()]
-            entry = graphs[key] = (graph, static_ids, out, keep)
-        graph, static_ids, out, _ = entry
+            entry = graphs[key] = (graph, static_ids, out)
+        graph, static_ids, out = entry
         static_ids.copy_(input_ids)
         graph.replay()
         return out

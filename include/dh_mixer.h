@@ -56,7 +56,7 @@ const char* dh_last_error(void);
  *             contiguous.
  *   Wi,Wf,Wr  (>= n_lv, H, GH): level stride `stride_wl`, head stride `stride_wh` (elements);
  *             innermost contiguous.
- *   bi,bf,br  fp32, (>= n_lv, H) contiguous.
+ *   bi,bf,br  fp32 (or `dtype`, see activate), (>= n_lv, H) contiguous.
  *   mask      nullable; dtype `dtype`, value > 0 means "edge allowed", element [b,t,l] at
  *             b*stride_mb + t*stride_mt + l*stride_ml. The wrap mask t >= 2^l is always applied
  *             in-kernel.
@@ -67,11 +67,12 @@ const char* dh_last_error(void);
  *   activate  0: write the pre-activations (the reference op's output). 1: write the level scan's
  *             gates instead: a = sigmoid(pre_i)*M, f = sigmoid(pre_f)*M + 1 - M, r = sigmoid(pre_r)
  *             with M = [t >= 2^l] * [mask > 0] (bf16: pre-activation and sigmoid rounded, as the
- *             eager path rounds them); dh_level_scan_fwd then runs with `activated`.
+ *             eager path rounds them); dh_level_scan_fwd then runs with `activated`. Plus 2: the biases are of
+ *             `dtype` instead of fp32.
  */
 int dh_gate_preacts_fwd(int dtype, const void* A, const void* B, int64_t stride_ab, int64_t stride_at,
                         const void* Wi, const void* Wf, const void* Wr, int64_t stride_wl,
-                        int64_t stride_wh, const float* bi, const float* bf, const float* br,
+                        int64_t stride_wh, const void* bi, const void* bf, const void* br,
                         const void* mask, int64_t stride_mb, int64_t stride_mt, int64_t stride_ml,
                         void* out_i, void* out_f, void* out_r, int64_t stride_ob, int64_t stride_ot,
                         int64_t stride_ol, int64_t stride_oh, int activate, int b, int T, int GH, int H,
@@ -147,6 +148,21 @@ int dh_level_scan_fwd(int dtype, const void* pre_i, const void* pre_f, const voi
                       const void* mask, int64_t stride_mb, int64_t stride_mt, int64_t stride_ml,
                       const void* V0, int64_t stride_vb, int64_t stride_vt, void* V, int b, int T, int H,
                       int hd, int n_lv, int activated, void* ring, int ring_L, void* stream);
+
+/*
+ * One mixer layer's inference forward (reference dispatcher_hybrid/modeling_dispatcher.py:63-123) as one call: the three
+ * input projections (dh_proj_gemm), the activated gates (dh_gate_preacts_fwd), the level scan (dh_level_scan_fwd) and the
+ * output projection (dh_proj_gemm), with the same results as those calls.
+ *   x         (b, T, d) rows ldx apart; W_in, W_x, W_s, W_out (d, d); Wi/Wf/Wr (>= n_lv, H, d) and bi/bf/br (>= n_lv, H),
+ *             all contiguous and of `dtype`; mask as in dh_gate_preacts_fwd; y (b, T, d) contiguous.
+ *   scratch   at least dh_mixer_fwd_scratch_bytes (-1 for refused sizes), 256-byte aligned.
+ */
+int64_t dh_mixer_fwd_scratch_bytes(int dtype, int b, int T, int d, int H, int n_lv);
+int dh_mixer_fwd(int dtype, const void* x, int64_t ldx, const void* W_in, const void* W_x, const void* W_s,
+                 const void* Wi, const void* Wf, const void* Wr, const void* bi, const void* bf, const void* br,
+                 const void* W_out, const void* mask, int64_t stride_mb, int64_t stride_mt, int64_t stride_ml,
+                 void* y, void* scratch, int64_t scratch_bytes, int b, int T, int d, int H, int n_lv,
+                 void* stream);
 
 /*
  * The level scan and its gradient for training (reference dispatcher_hybrid/modeling_dispatcher.py:86-88, 111-121 under

@@ -184,3 +184,29 @@ def test_mixer_train_partial_gradients_hooks_and_adapters():
     ad.weight = mx.linear_out.weight
     mx.linear_out = ad
     assert (mx(x, mask) - 2 * full).norm() <= 4e-5 * full.norm()
+
+
+def test_mixer_train_under_transforms():
+    """A saved-tensor hook sees what the whole-layer operation keeps; torch.func transforms (which registered operations do
+    not take) and second derivatives are refused, not silently wrong; a compiler gets the layer-by-layer form and the same
+    gradients."""
+    mx = _mixer(torch.float32)
+    mx.use_fused_gates = True
+    t = torch.arange(70, device=DEV).unsqueeze(1)
+    mask = (t >= (1 << torch.arange(8, device=DEV))).float()
+    x = torch.randn(1, 70, 128, device=DEV)
+    xg = x.clone().requires_grad_()
+    want, = torch.autograd.grad(mx(xg, mask).square().sum(), xg)
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda z: mx(z, mask).square().sum())(x)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda z: packed.append(z.numel()) or z.cpu(), lambda z: z.to(DEV)):
+        loss = mx(xg, mask).square().sum()
+    hooked, = torch.autograd.grad(loss, xg)
+    assert packed and torch.equal(hooked, want)
+    g1, = torch.autograd.grad(mx(xg, mask).square().sum(), xg, create_graph=True)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(g1.sum(), xg)
+    compiled = torch.compile(mx, backend="aot_eager", fullgraph=True)
+    traced, = torch.autograd.grad(compiled(xg, mask).square().sum(), xg)
+    assert (traced - want).norm() <= 2e-5 * want.norm()

@@ -17,7 +17,8 @@
 //   strided  levels 6 .. 11 (lags 64 .. 2048): the up to 64 positions t = c (mod 64), closed under these lags
 // The sums over columns (64 lanes) of 64 positions at a time go through a transposing reduction, ~2 instructions a value.
 // Bound: VALU (forward ~4 instructions per state element and level, backward ~11) beside the states' traffic, one write
-// and one read of n_lv x (b, T, d).
+// and one read of n_lv x (b, T, d). Measured on MI355X at d 1024, 12 levels, bf16 (us): b 4, T 4096 forward 65 + 50,
+// backward 96 + 101; b 4, T 1024 25 + 14 and 35 + 22. The torch loop took ~300 launches, 6.2 ms and 2.2 ms.
 #include "dh_common.h"
 
 #include <utility>

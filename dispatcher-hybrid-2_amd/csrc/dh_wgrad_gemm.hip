@@ -9,7 +9,8 @@
 // go into one launch (a mixer's four projections: 256 tiles). With fewer tiles than workgroup slots the rows are split and
 // a second launch adds the ranges' fp32 sums in order and rounds once; the same inputs give the same bits. Consecutive
 // work items (the tiles of one layer and range, which read the same rows) go to one XCD.
-// Bound: LDS (16 fragment reads of 512 B and 8 stores per 16 MFMAs and wave) beside the matrix cores.
+// Bound: LDS (16 fragment reads of 512 B and 8 stores per 16 MFMAs and wave) beside the matrix cores. Measured on MI355X,
+// four 1024 x 1024 gradients: 188 us at 16384 rows (730 TFLOP/s), 53 + 8 at 4096, against 453 and 124 for the library's four.
 #include "dh_common.h"
 
 namespace {

@@ -27,12 +27,9 @@
 // O^T = V^T P^T, whose A operand reads the transposed values from LDS. Workgroups are numbered so
 // consecutive query blocks of one (batch row, head) run on one XCD (round-robin dispatch: block id
 // mod 8), sharing the band's key and value lines in that XCD's L2.
-#include "dh_common.h"
+#include "dh_attn_common.h"
 
 namespace {
-
-typedef __attribute__((__vector_size__(8 * sizeof(short)))) short bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
 
 constexpr int kBQ = 64;          // queries per workgroup
 constexpr int kBK = 64;          // keys per block
@@ -52,49 +49,8 @@ struct WinArgs {
   int64_t cb, ch;               // cache batch / head strides (elements); rows hd apart
   int B, T, H, window, nq, nwork;
   float scale2;                 // 1/sqrt(hd) * log2(e): scores go to the log2 domain
+  float* lse;                   // nullable (B, H, T): log2 of the sum of 2^score, for the backward
 };
-
-__device__ __forceinline__ uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
-__device__ __forceinline__ uint2 ld8(const void* p) { return *reinterpret_cast<const uint2*>(p); }
-__device__ __forceinline__ float lo_f(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float hi_f(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-// bf16 rounding through the compiler's conversion (v_cvt_pk_bf16_f32: round to nearest even, the
-// rounding torch's bf16 ops use); a pair packs in one instruction
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float rnd(float x) { return (float)(__bf16)x; }
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  bf16x2_t v;
-  v.x = (__bf16)lo;
-  v.y = (__bf16)hi;
-  return __builtin_bit_cast(uint32_t, v);
-}
-
-// rope of 8 consecutive elements (4 interleaved pairs) with their 4 cos / sin values; every product
-// and sum rounded to bf16 on its own (torch evaluates them as separate bf16 tensor ops)
-__device__ __forceinline__ uint4 rope8(const uint4& x, const uint2& c, const uint2& s) {
-  const uint32_t xw[4] = {x.x, x.y, x.z, x.w};
-  const float cv[4] = {lo_f(c.x), hi_f(c.x), lo_f(c.y), hi_f(c.y)};
-  const float sv[4] = {lo_f(s.x), hi_f(s.x), lo_f(s.y), hi_f(s.y)};
-  uint32_t o[4];
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    const float e = lo_f(xw[p]), d = hi_f(xw[p]);
-    float r0, r1;
-    {
-#pragma clang fp contract(off)
-      r0 = rnd(rnd(e * cv[p]) - rnd(d * sv[p]));
-      r1 = rnd(rnd(e * sv[p]) + rnd(d * cv[p]));
-    }
-    o[p] = pack2(r0, r1);
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-__device__ __forceinline__ bf16x8 as_bf16x8(const uint4& v) {
-  bf16x8 r;
-  __builtin_memcpy(&r, &v, 16);
-  return r;
-}
 
 // Pre-pass: rope(k) and v of every position into the (B, H, Tmax, hd) buffers the attention reads
 // (the decoder caches, or scratch): each key is rotated once, not by every workgroup whose band
@@ -306,6 +262,7 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
   // ---- output: lane holds query tq, hd columns 16 nt + 4 g + i
   if (tq < a.T) {
     const float inv = 1.f / l;
+    if (a.lse != nullptr && g == 0) a.lse[((int64_t)b * a.H + h) * a.T + tq] = m + __builtin_amdgcn_logf(l);
     bf16_t* yp = a.y + (int64_t)b * a.yb + (int64_t)tq * a.yt + (int64_t)h * HD;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
@@ -316,14 +273,10 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
 
 bool aligned(const void* p, uintptr_t n) { return ((uintptr_t)p % n) == 0; }
 
-}  // namespace
-
-extern "C" int dh_window_attention_fwd(int dtype, const void* q, const void* k, const void* v, int64_t stride_b,
-                                       int64_t stride_t, const void* rope_cos, const void* rope_sin, void* y,
-                                       int64_t y_stride_b, int64_t y_stride_t, void* K_cache, void* V_cache,
-                                       int64_t cache_stride_b, int64_t cache_stride_h, int Tmax, int B, int T, int H,
-                                       int hd, int window, void* stream) {
-  const char* who = "dh_window_attention_fwd";
+int window_attention(const char* who, int dtype, const void* q, const void* k, const void* v, int64_t stride_b,
+                     int64_t stride_t, const void* rope_cos, const void* rope_sin, void* y, int64_t y_stride_b,
+                     int64_t y_stride_t, void* K_cache, void* V_cache, int64_t cache_stride_b, int64_t cache_stride_h,
+                     int Tmax, int B, int T, int H, int hd, int window, float* lse, void* stream) {
   DH_REQUIRE(dtype == DH_BF16, DH_ERR_UNSUPPORTED_DTYPE, "%s: dtype %d (bf16 only)", who, dtype);
   DH_REQUIRE(hd == 32 || hd == 64 || hd == 128, DH_ERR_UNSUPPORTED_SHAPE, "%s: hd=%d not in {32,64,128}", who, hd);
   DH_REQUIRE(B >= 1 && T >= 1 && H >= 1 && window >= 0, DH_ERR_INVALID_ARG, "%s: B=%d T=%d H=%d window=%d", who, B,
@@ -343,7 +296,8 @@ extern "C" int dh_window_attention_fwd(int dtype, const void* q, const void* k, 
   WinArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, stride_b, stride_t,
             (const bf16_t*)rope_cos, (const bf16_t*)rope_sin, (bf16_t*)y, y_stride_b, y_stride_t,
             (bf16_t*)K_cache, (bf16_t*)V_cache, cache_stride_b, cache_stride_h, B, T, H, window, nq, (int)nwork,
-            (float)(1.0 / sqrt((double)hd)) * 1.44269504088896341f};   // torch's fp32 1/sqrt(hd), times log2 e
+            (float)(1.0 / sqrt((double)hd)) * 1.44269504088896341f,    // torch's fp32 1/sqrt(hd), times log2 e
+            lse};
   const int grid = (int)(((nwork + 7) / 8) * 8);
   const int64_t chunks = (int64_t)B * T * H * (hd / 8);
   const int pgrid = (int)((chunks + kThreads - 1) / kThreads);
@@ -359,4 +313,26 @@ extern "C" int dh_window_attention_fwd(int dtype, const void* q, const void* k, 
     window_attn_kernel<128><<<dim3(grid), dim3(kThreads), 0, s>>>(a);
   }
   return dh_check_launch(who);
+}
+
+}  // namespace
+
+extern "C" int dh_window_attention_fwd(int dtype, const void* q, const void* k, const void* v, int64_t stride_b,
+                                       int64_t stride_t, const void* rope_cos, const void* rope_sin, void* y,
+                                       int64_t y_stride_b, int64_t y_stride_t, void* K_cache, void* V_cache,
+                                       int64_t cache_stride_b, int64_t cache_stride_h, int Tmax, int B, int T, int H,
+                                       int hd, int window, void* stream) {
+  return window_attention("dh_window_attention_fwd", dtype, q, k, v, stride_b, stride_t, rope_cos, rope_sin, y, y_stride_b,
+                          y_stride_t, K_cache, V_cache, cache_stride_b, cache_stride_h, Tmax, B, T, H, hd, window, nullptr,
+                          stream);
+}
+
+extern "C" int dh_window_attention_train_fwd(int dtype, const void* q, const void* k, const void* v, int64_t stride_b,
+                                             int64_t stride_t, const void* rope_cos, const void* rope_sin, void* y,
+                                             int64_t y_stride_b, int64_t y_stride_t, void* K_rot, void* V_rows, float* lse,
+                                             int B, int T, int H, int hd, int window, void* stream) {
+  const char* who = "dh_window_attention_train_fwd";
+  DH_REQUIRE(lse, DH_ERR_INVALID_ARG, "%s: null pointer argument", who);
+  return window_attention(who, dtype, q, k, v, stride_b, stride_t, rope_cos, rope_sin, y, y_stride_b, y_stride_t, K_rot,
+                          V_rows, (int64_t)H * T * hd, (int64_t)T * hd, T, B, T, H, hd, window, lse, stream);
 }

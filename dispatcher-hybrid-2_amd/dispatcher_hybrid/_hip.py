@@ -86,6 +86,10 @@ def _load():
                                        vp, i64, vp], i32),
         "dh_window_attention_fwd": ([i32, vp, vp, vp, i64, i64, vp, vp, vp, i64, i64, vp, vp, i64, i64,
                                      i32, i32, i32, i32, i32, i32, vp], i32),
+        "dh_window_attention_train_fwd": ([i32, vp, vp, vp, i64, i64, vp, vp, vp, i64, i64, vp, vp, vp]
+                                           + [i32] * 5 + [vp], i32),
+        "dh_window_attention_bwd": ([i32, vp, i64, i64, vp, vp, vp, i64, i64, vp, i64, i64] + [vp] * 8 + [i64, i64]
+                                    + [i32] * 5 + [vp], i32),
         "dh_decode_scan_out": ([i32] + [vp] * 8 + [i64, vp] + [i32] * 6 + [vp], i32),
         "dh_proj_gemm": ([i32, vp, i64, i32, i32, i32, vp, vp, vp, vp, vp], i32),
         "dh_proj_gemm_swiglu": ([i32, vp, i64, i32, i32, vp, vp, i32, vp, i64, vp], i32),

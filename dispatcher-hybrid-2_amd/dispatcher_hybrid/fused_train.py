@@ -2,11 +2,13 @@
 
     dispatcher::gate_scan_train   gate pre-activations + level scan (from the projections A, B, V0)
     mixer_train                   a whole mixer layer: projections, gate path, output projection
+    attention_train               a whole sliding-window attention layer (bf16, 64-wide heads)
 
-Both run under ``model.enable_fused_gates()`` when gradients are wanted (DispatcherMixer picks the widest one that fits)
-and replace the reference's eager autograd of the level loop (reference dispatcher_hybrid/modeling_dispatcher.py:86-121)
-and its fused gate op's backward (reference dispatcher_hybrid/fused_gates.py:96-173, 225-257). Kernels:
-``dh_gate_preacts_fwd``, ``dh_level_scan_train_fwd`` / ``_bwd``, ``dh_gate_preacts_bwd_ws``, ``dh_wgrad_gemm`` and, for the
+They run under ``model.enable_fused_gates()`` when gradients are wanted (DispatcherMixer picks the widest one that fits)
+and replace the reference's eager autograd of the level loop and the attention (reference
+dispatcher_hybrid/modeling_dispatcher.py:86-121, 163-182) and its fused gate op's backward (reference
+dispatcher_hybrid/fused_gates.py:96-173, 225-257). Kernels: ``dh_gate_preacts_fwd``, ``dh_level_scan_train_fwd`` / ``_bwd``,
+``dh_gate_preacts_bwd_ws``, ``dh_window_attention_train_fwd``, ``dh_window_attention_bwd``, ``dh_wgrad_gemm`` and, for the
 plain products, ``dh_proj_gemm`` or the library.
 
 Importing this module loads the kernel library and raises ImportError if it is missing.
@@ -266,3 +268,82 @@ def mixer_train(mixer, x, mask, n_lv):
     (Wi, bi), (Wf, bf), (Wr, br) = mixer._gate_params()
     return _MixerTrain.apply(x, mixer.linear_in.weight, mixer.gate_hidden.weight, mixer.gate_hidden_src.weight, Wi, Wf, Wr,
                              bi, bf, br, mixer.linear_out.weight, mask, mixer.num_heads, n_lv)
+
+
+# ---------------------------------------------------------------------------------------------
+# a whole attention layer
+# ---------------------------------------------------------------------------------------------
+def attention_fits(attn, x):
+    """Whether attention_train takes this layer and input: bf16 throughout and no autocast, 64-wide heads, plain bias-free
+    projections, plain eager execution."""
+    if torch.compiler.is_compiling() or transforms_active():
+        return False
+    d = attn.embed_dim
+    return (x.dim() == 3 and x.is_cuda and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
+            and x.dtype == torch.bfloat16 and x.shape[-1] == d and attn.head_dim == 64
+            and not torch.is_autocast_enabled("cuda") and x.numel() * 3 * x.element_size() < 2 ** 31
+            and all(plain_linear(l, x.dtype, d) and l.weight.shape[0] == d
+                    for l in (attn.linear_q, attn.linear_k, attn.linear_v, attn.linear_out)))
+
+
+class _AttentionTrain(torch.autograd.Function):
+    """An attention layer; see attention_train."""
+
+    @staticmethod
+    def forward(ctx, x, W_q, W_k, W_v, W_out, cos, sin, num_heads, window):
+        b, T, d = x.shape
+        H, hd = num_heads, d // num_heads
+        x2 = _rows16(x.reshape(b * T, d), 8)
+        W_cat = torch.cat((W_q, W_k, W_v))
+        proj = _linear(x2, W_cat, PROJ_GEMM_MAX_ROWS)                          # rows [q | k | v]
+        q, k, v = proj.view(b, T, 3 * d).split(d, -1)
+        y = torch.empty(b, T, d, device=x.device, dtype=x.dtype)
+        kv = torch.empty(2, b, H, T, hd, device=x.device, dtype=x.dtype)       # rotated keys, values, head-major
+        lse = torch.empty(b, H, T, device=x.device, dtype=torch.float32)
+        p = _hip.ptr
+        st = _hip.lib.dh_window_attention_train_fwd(
+            _hip.dtype_code(x.dtype), p(q), p(k), p(v), q.stride(0), q.stride(1), p(cos), p(sin), p(y), y.stride(0),
+            y.stride(1), p(kv[0]), p(kv[1]), p(lse), b, T, H, hd, window, _hip.stream_handle(x.device))
+        _hip.check(st, "attention_train")
+        out = _linear(y.view(b * T, d), W_out, OUT_GEMM_MAX_ROWS)
+        ctx.save_for_backward(x, W_out, cos, sin, proj, y, kv, lse, W_cat)
+        ctx.sizes = (num_heads, window)
+        return out.view(b, T, d)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dout):
+        x, W_out, cos, sin, proj, y, kv, lse, W_cat = ctx.saved_tensors
+        H, window = ctx.sizes
+        need = ctx.needs_input_grad
+        b, T, d = x.shape
+        hd = d // H
+        x2, do2 = _rows16(x.reshape(b * T, d), 8), _rows16(dout.reshape(b * T, d), 8)
+        dy = torch.mm(do2, W_out).view(b, T, d)
+        dproj = torch.empty_like(proj)                                         # rows [dq | dk | dv]
+        q = proj.view(b, T, 3 * d)[..., :d]
+        dq, dk, dv = dproj.view(b, T, 3 * d).split(d, -1)
+        q_rot = torch.empty(b, H, T, hd, device=x.device, dtype=x.dtype)
+        delta = torch.empty_like(lse)
+        p = _hip.ptr
+        st = _hip.lib.dh_window_attention_bwd(
+            _hip.dtype_code(x.dtype), p(q), q.stride(0), q.stride(1), p(kv[0]), p(kv[1]), p(y), y.stride(0), y.stride(1),
+            p(dy), dy.stride(0), dy.stride(1), p(lse), p(cos), p(sin), p(q_rot), p(delta), p(dq), p(dk), p(dv),
+            dq.stride(0), dq.stride(1), b, T, H, hd, window, _hip.stream_handle(x.device))
+        _hip.check(st, "attention_train")
+        dx = torch.mm(dproj, W_cat).view(b, T, d) if need[0] else None
+        dw = [None] * 4
+        if any(need[1:5]):
+            dw = weight_grads([(x2, g) for g in dproj.split(d, -1)] + [(y.view(b * T, d), do2)])
+        return (*[v if n else None for v, n in zip([dx, *dw], need)], None, None, None, None)
+
+
+def attention_train(attn, x):
+    """A WindowAttention's output (b, T, d), differentiable (once) in x and the four projections (reference
+    dispatcher_hybrid/modeling_dispatcher.py:168-182): scores and probabilities stay in registers in both directions
+    (``dh_window_attention_train_fwd`` / ``dh_window_attention_bwd``; the softmax's log-sum is kept in fp32), one product for
+    q, k, v and one launch for the four weight gradients. See attention_fits."""
+    T = x.shape[1]
+    cos, sin = attn.rope_tables(T, x.device, x.dtype)
+    return _AttentionTrain.apply(x, attn.linear_q.weight, attn.linear_k.weight, attn.linear_v.weight, attn.linear_out.weight,
+                                 cos, sin, attn.num_heads, attn.band(T))

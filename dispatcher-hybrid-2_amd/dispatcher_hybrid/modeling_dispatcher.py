@@ -276,6 +276,11 @@ class WindowAttention(nn.Module):
                 cos, sin = self.rope_tables(T, x.device, x.dtype)
                 y = fa.window_attention(q, k, v, cos, sin, self.num_heads, self.band(T))
                 return project(y, [self.linear_out], OUT_GEMM_MAX_ROWS)[0]
+        elif self.use_fused and x.is_cuda and torch.is_grad_enabled() and (
+                x.requires_grad or any(p.requires_grad for p in self.parameters())):
+            from . import fused_train as ft
+            if ft.attention_fits(self, x):
+                return ft.attention_train(self, x)
         return self._forward_eager(x)
 
     def band(self, T):

@@ -348,6 +348,24 @@ int dh_window_attention_fwd(int dtype, const void* q, const void* k, const void*
                             int hd, int window, void* stream);
 
 /*
+ * The same attention in training (bf16): the forward also writes lse (B, H, T), log2 of each query's sum of
+ * 2^(score log2 e / sqrt(hd)); K_rot and V_rows (B, H, T, hd) contiguous are kept for the backward.
+ * The backward (hd 64) takes the projection rows q, the output y and its gradient dy (rows of H*hd), fills the scratch
+ * Q_rot (B, H, T, hd) and delta (B, H, T), and writes the gradients of the projections q, k, v before rope. All row strides
+ * are multiples of 8 elements.
+ */
+int dh_window_attention_train_fwd(int dtype, const void* q, const void* k, const void* v, int64_t stride_b,
+                                  int64_t stride_t, const void* rope_cos, const void* rope_sin, void* y,
+                                  int64_t y_stride_b, int64_t y_stride_t, void* K_rot, void* V_rows, float* lse,
+                                  int B, int T, int H, int hd, int window, void* stream);
+int dh_window_attention_bwd(int dtype, const void* q, int64_t stride_b, int64_t stride_t, const void* K_rot,
+                            const void* V_rows, const void* y, int64_t y_stride_b, int64_t y_stride_t,
+                            const void* dy, int64_t dy_stride_b, int64_t dy_stride_t, const float* lse,
+                            const void* rope_cos, const void* rope_sin, void* Q_rot, float* delta, void* dq,
+                            void* dk, void* dv, int64_t d_stride_b, int64_t d_stride_t, int B, int T, int H,
+                            int hd, int window, void* stream);
+
+/*
  * One decode step of a windowed RoPE attention layer: rotation of the new query and key at the
  * device position t, the cache write of (k', v) at t, the scores over the window [lo, t]
  * (lo = max(0, t+1-window), window 0 = the whole prefix), softmax and the value average, as ONE

@@ -89,9 +89,6 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 // result and the compiler's hazard pass does not look into inline assembly. The hot loop feeds it
 // v_max results only; everything else rounds with round_bf16_sw.
 __device__ __forceinline__ float round_bf16_sw(float x) { return bf16_to_f32(f32_to_bf16(x)); }
-// the same through the compiler's own conversion (v_cvt_pk_bf16_f32 + shift; round to nearest
-// even, NaN stays NaN), usable on transcendental results
-__device__ __forceinline__ float round_bf16_cc(float x) { return (float)(__bf16)x; }
 __device__ __forceinline__ float round_bf16(float x) {
   float r;
   asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(r) : "v"(x));
@@ -315,7 +312,8 @@ __global__ __launch_bounds__(kThreads) void gate_preacts_fwd_kernel(FwdArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// bf16 forward with the weights staged in LDS (H <= 16).
+// Forward with the weights staged in LDS (H <= 16). Written for bf16, where the sizes below hold; fp32 differs in the MFMA and
+// in a chunk being 32 k elements.
 //
 // The kernel above streams every weight fragment from the cache hierarchy into every wave: per
 // k-step a wave reads 3 KB of weights per level for 1 KB of activations, and at C5 sizes
@@ -345,18 +343,19 @@ template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
   static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
-constexpr int kLdsKC = 64;                      // k elements per LDS weight chunk (2 MFMA k-steps)
-constexpr int kLdsRow = kLdsKC * 2 + 16;         // padded LDS row: 144 bytes
+constexpr int kLdsKB = 128;                     // k bytes per LDS weight chunk (2 steps of 64: 64 bf16 / 32 fp32 elements)
+constexpr int kLdsRow = kLdsKB + 16;             // padded LDS row: 144 bytes
 
 // occupancy by register footprint: (levels x row blocks) accumulators plus two chunks of fragments
 template <int LG, int MB> struct LdsOcc { static constexpr int value = LG * MB >= 4 ? 2 : 3; };
 
-template <int LG, int MB, bool HAS_MASK>
+template <typename M, int LG, int MB, bool HAS_MASK>
 __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preacts_fwd_lds_kernel(FwdArgs a) {
-  typedef bf16_t T;
+  typedef typename M::T T;
+  constexpr int VE = 16 / (int)sizeof(T);        // elements of a 16-byte piece
   constexpr int P = 64 * MB;                     // positions per workgroup
   constexpr int WBYTES = LG * 3 * 16 * kLdsRow;  // one LDS weight buffer
-  constexpr int PIECES = LG * 3 * 16 * (kLdsKC / 8);   // 16-byte pieces of one chunk
+  constexpr int PIECES = LG * 3 * 16 * (kLdsKB / 16);   // 16-byte pieces of one chunk
   constexpr int PPT = (PIECES + kThreads - 1) / kThreads;
   __shared__ __align__(16) unsigned char wl[2][WBYTES];
   const int tid = threadIdx.x;
@@ -386,7 +385,7 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
     const int t = tbase + 16 * mb + crow;
     const bool t_ok = t < a.T;
     const int tc = t_ok ? t : a.T - 1;
-    aoff[mb] = (uint32_t)(((int64_t)tc * a.sat + cpiece * 8) * (int64_t)sizeof(T));
+    aoff[mb] = (uint32_t)(((int64_t)tc * a.sat + cpiece * VE) * (int64_t)sizeof(T));
 #pragma unroll
     for (int j = 0; j < LG; ++j) {
       const int lv = min(l0 + j, a.n_lv - 1);
@@ -396,7 +395,7 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
       const int src = tc - (1 << lv);
       const bool keep = t_ok && src >= 0 && l0 + j < a.n_lv && mv > 0.f;
       // a row without a source reads past the descriptor's range, which returns zeros (B = 0)
-      boff[mb][j] = keep ? (uint32_t)(((int64_t)src * a.sat + cpiece * 8) * (int64_t)sizeof(T)) : 0x80000000u;
+      boff[mb][j] = keep ? (uint32_t)(((int64_t)src * a.sat + cpiece * VE) * (int64_t)sizeof(T)) : 0x80000000u;
     }
   }
   auto to_mfma = [&](const uint4& v) {
@@ -419,12 +418,12 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
     const int jx = min(2 * i + (wave_u >> 1), 3 * LG - 1);   // = q >> 7 (uniform)
     const int j = jx / 3;
     const int lv = min(l0 + j, a.n_lv - 1), nc = min(n, a.H - 1);
-    wsrc[i] = (uint32_t)(((int64_t)lv * a.swl + (int64_t)nc * a.swh + c * 8) * (int64_t)sizeof(T));
+    wsrc[i] = (uint32_t)(((int64_t)lv * a.swl + (int64_t)nc * a.swh + c * VE) * (int64_t)sizeof(T));
     wdst[i] = (uint32_t)((jx * 16 + n) * kLdsRow + c * 16);
   }
   uint4 wst[PPT];
-  auto w_fetch = [&](int k0) {
-    const uint32_t kb = (uint32_t)(k0 * (int)sizeof(T));
+  auto w_fetch = [&](int kbyte) {
+    const uint32_t kb = (uint32_t)kbyte;
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
       const int jx = min(2 * i + (wave_u >> 1), 3 * LG - 1);
@@ -451,10 +450,10 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
   // block. Two chunk buffers in ping-pong: the next chunk's fragments are in flight during the
   // whole current chunk (the loads' latency under load is several k-steps of arithmetic).
   uint4 xA[2][MB], xB[2][MB][LG], yA[2][MB], yB[2][MB][LG];
-  auto fetch = [&](int k0, uint4 (&fA)[2][MB], uint4 (&fB)[2][MB][LG]) {
+  auto fetch = [&](int kbyte, uint4 (&fA)[2][MB], uint4 (&fB)[2][MB][LG]) {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
-      const uint32_t kb = (uint32_t)((k0 + 32 * kk) * (int)sizeof(T));
+      const uint32_t kb = (uint32_t)(kbyte + 64 * kk);
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
         fA[kk][mb] = bld16(rA, aoff[mb], kb);
@@ -467,9 +466,9 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
   auto compute = [&](const uint4 (&fA)[2][MB], const uint4 (&fB)[2][MB][LG], int buf) {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
-      float af[MB][8];
+      float af[MB][M::KL];
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) MathBf16::unpack_a(to_mfma(fA[kk][mb]), af[mb]);
+      for (int mb = 0; mb < MB; ++mb) M::unpack_a(to_mfma(fA[kk][mb]), af[mb]);
 #pragma unroll
       for (int j = 0; j < LG; ++j) {
         uint4 w[3];
@@ -477,18 +476,18 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
         for (int x = 0; x < 3; ++x)
           w[x] = *reinterpret_cast<const uint4*>(&wl[buf][((j * 3 + x) * 16 + r) * kLdsRow + kk * 64 + g * 16]);
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) MathBf16::mma3(acc[mb][j], af[mb], to_mfma(fB[kk][mb][j]), w);
+        for (int mb = 0; mb < MB; ++mb) M::mma3(acc[mb][j], af[mb], to_mfma(fB[kk][mb][j]), w);
       }
     }
   };
-  const int nchunk_ = a.GH / kLdsKC;
+  const int nchunk_ = a.GH * (int)sizeof(T) / kLdsKB;
   // chunk c: request chunk c+1 (weights and fragments), compute chunk c, store the weights of c+1
   auto chunk = [&](int c, const uint4 (&cA)[2][MB], const uint4 (&cB)[2][MB][LG], uint4 (&nA)[2][MB],
                    uint4 (&nB)[2][MB][LG]) {
     const bool more = c + 1 < nchunk_;                   // uniform
     if (more) {
-      w_fetch((c + 1) * kLdsKC);
-      fetch((c + 1) * kLdsKC, nA, nB);
+      w_fetch((c + 1) * kLdsKB);
+      fetch((c + 1) * kLdsKB, nA, nB);
     }
     compute(cA, cB, c & 1);
     if (more) w_store((c + 1) & 1);
@@ -503,8 +502,8 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
     // into the set chunk c - 1 used, and writes the weights of chunk c + 1 to LDS.
     constexpr int NS = kSets;
     uint4 sA[NS][2][MB], sB[NS][2][MB][LG], sW[NS][PPT];
-    auto w_fetch3 = [&](int k0, uint4 (&ws)[PPT]) {
-      const uint32_t kb = (uint32_t)(k0 * (int)sizeof(T));
+    auto w_fetch3 = [&](int kbyte, uint4 (&ws)[PPT]) {
+      const uint32_t kb = (uint32_t)kbyte;
 #pragma unroll
       for (int i = 0; i < PPT; ++i) {
         const int jx = min(2 * i + (wave_u >> 1), 3 * LG - 1);
@@ -522,8 +521,8 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
       constexpr int u = decltype(uc)::value;             // c % NS
       constexpr int uf = (u + NS - 1) % NS, un = (u + 1) % NS;
       if (c + NS - 1 < nchunk_) {                        // uniform
-        w_fetch3((c + NS - 1) * kLdsKC, sW[uf]);
-        fetch((c + NS - 1) * kLdsKC, sA[uf], sB[uf]);
+        w_fetch3((c + NS - 1) * kLdsKB, sW[uf]);
+        fetch((c + NS - 1) * kLdsKB, sA[uf], sB[uf]);
       }
       compute(sA[u], sB[u], c & 1);
       if (c + 1 < nchunk_) w_store3((c + 1) & 1, sW[un]);
@@ -532,8 +531,8 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
     static_for<NS - 1>([&](auto uc) {
       constexpr int u = decltype(uc)::value;
       if (u < nchunk_) {
-        w_fetch3(u * kLdsKC, sW[u]);
-        fetch(u * kLdsKC, sA[u], sB[u]);
+        w_fetch3(u * kLdsKB, sW[u]);
+        fetch(u * kLdsKB, sA[u], sB[u]);
       }
     });
     w_store3(0, sW[0]);
@@ -586,10 +585,9 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float m = (tb + i >= (1 << l) && mval[i] > 0.f) ? 1.f : 0.f;
-          // compiler-emitted bf16 rounding (hardware conversion, its hazards handled)
-          const float si = round_bf16_cc(dh_sigmoid(round_bf16_cc(v[0][i])));
-          const float sf = round_bf16_cc(dh_sigmoid(round_bf16_cc(v[1][i])));
-          const float sr = round_bf16_cc(dh_sigmoid(round_bf16_cc(v[2][i])));
+          const float si = M::rnd(dh_sigmoid(M::rnd(v[0][i])));
+          const float sf = M::rnd(dh_sigmoid(M::rnd(v[1][i])));
+          const float sr = M::rnd(dh_sigmoid(M::rnd(v[2][i])));
           v[0][i] = si * m;
           v[1][i] = sf * m + (1.f - m);
           v[2][i] = sr;
@@ -598,11 +596,11 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
 #pragma unroll
       for (int x = 0; x < 3; ++x) {
         if (vec) {
-          MathBf16::store4(outs[x] + base + tb, v[x]);
+          M::store4(outs[x] + base + tb, v[x]);
         } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (tb + i < a.T) outs[x][base + (int64_t)(tb + i) * a.sot] = MathBf16::out(v[x][i]);
+            if (tb + i < a.T) outs[x][base + (int64_t)(tb + i) * a.sot] = M::out(v[x][i]);
         }
       }
     }
@@ -767,14 +765,14 @@ void launch_fwd(const FwdArgs& a, dim3 grid, hipStream_t s) {
     gate_preacts_fwd_kernel<M, LG, KU, false><<<grid, dim3(kThreads), 0, s>>>(a);
 }
 
-template <int LG, int MB>
+template <typename M, int LG, int MB>
 void launch_fwd_lds(const FwdArgs& a, hipStream_t s) {
   constexpr int P = 64 * MB;
   dim3 grid((a.T + P - 1) / P, (a.n_lv + LG - 1) / LG, a.b);
   if (a.mask)
-    gate_preacts_fwd_lds_kernel<LG, MB, true><<<grid, dim3(kThreads), 0, s>>>(a);
+    gate_preacts_fwd_lds_kernel<M, LG, MB, true><<<grid, dim3(kThreads), 0, s>>>(a);
   else
-    gate_preacts_fwd_lds_kernel<LG, MB, false><<<grid, dim3(kThreads), 0, s>>>(a);
+    gate_preacts_fwd_lds_kernel<M, LG, MB, false><<<grid, dim3(kThreads), 0, s>>>(a);
 }
 
 // Tile per workgroup (measured on MI355X at the released widths): two levels x 64 positions once
@@ -783,10 +781,11 @@ void launch_fwd_lds(const FwdArgs& a, hipStream_t s) {
 // the most workgroups for short prefills. Handing each XCD whole batch rows (a tile's level groups
 // and its lagged B rows then share one L2) measured the same, 136 us, and so did rounding the hidden
 // tile once instead of at the eager path's two points (the launch is not bound by that VALU work).
+template <typename M>
 void dispatch_fwd_lds(const FwdArgs& a, hipStream_t s) {
   const int64_t wgs21 = (int64_t)((a.T + 63) / 64) * ((a.n_lv + 1) / 2) * a.b;
-  if (wgs21 >= 1024) launch_fwd_lds<2, 1>(a, s);
-  else launch_fwd_lds<1, 1>(a, s);
+  if (wgs21 >= 1024) launch_fwd_lds<M, 2, 1>(a, s);
+  else launch_fwd_lds<M, 1, 1>(a, s);
 }
 
 template <typename M>
@@ -842,8 +841,10 @@ extern "C" int dh_gate_preacts_fwd(int dtype, const void* A, const void* B, int6
   if (KU == 2 && LG == 1) KU = 1;                            // no <1, 2> instantiation
   dim3 grid(tiles, ngroups, b);
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == DH_BF16 && H <= 16)
-    dispatch_fwd_lds(a, s);
+  if (H <= 16 && dtype == DH_BF16)
+    dispatch_fwd_lds<MathBf16>(a, s);
+  else if (H <= 16)
+    dispatch_fwd_lds<MathF32>(a, s);
   else if (dtype == DH_BF16)
     dispatch_fwd<MathBf16>(a, LG, KU, grid, s);
   else

@@ -4,33 +4,36 @@
 // B = gate_hidden_src(x) -- three GEMMs over the same rows, done here as one launch over the
 // concatenated N = N_0 + N_1 + N_2 columns). fp32 accumulation; bf16 outputs rounded once.
 //
-// Work decomposition: a workgroup (4 wave64s, a 2 x 2 grid) computes a square output tile of
-// 32 * WT rows and columns; each wave a quadrant of WT x WT MFMA tiles of 16 x 16
-// (v_mfma_f32_16x16x32_bf16; fp32 models use v_mfma_f32_16x16x4f32). Two tile sizes:
-//   WT = 4: 128 x 128 tiles, for launches with too few 256 x 256 tiles to fill the 256 CUs;
-//   WT = 8: 256 x 256 tiles (bf16), for many rows: each wave's 128 x 128 quadrant reads 512 LDS bytes
-//           per k for 32 KFLOP, half the LDS traffic per MFMA of the 128 x 128 tile, whose 64 x 64
-//           quadrants need the LDS at its full read rate to keep the MFMA pipe busy.
-// K advances in tiles of 128 bytes per row (64 bf16 / 32 fp32): both operand tiles are staged in LDS
-// with a 16-byte row pad (conflict-free 16-byte fragment reads), double-buffered, the next tile's
-// global loads in flight in registers while the current one is multiplied; one barrier per K tile.
+// Two kernels. bf16 launches whose operands allow it take the ping-pong kernel further down (LDS filled by the DMA path).
+// The rest -- fp32 (v_mfma_f32_16x16x4f32) and unaligned bf16 -- take proj_gemm_kernel: a workgroup (4 wave64s, a 2 x 2 grid)
+// computes an output tile of 32 TM rows x 32 TN columns, each wave TM x TN MFMA tiles of 16 x 16. K advances in tiles of 128
+// bytes per row (64 bf16 / 32 fp32): both operand tiles are staged in LDS with a 16-byte row pad (conflict-free 16-byte
+// fragment reads), double-buffered, the next D tiles' global loads in flight in registers while the current one is
+// multiplied; one barrier per K tile.
 // The weight tile is the MFMA's A operand and the activation tile its B operand, so the accumulator
 // of a lane holds four consecutive output columns of one output row: the epilogue writes 8 (bf16) or
 // 16 (fp32) contiguous bytes per lane and MFMA tile.
-// Block order is XCD-aware: with round-robin dispatch over the 8 XCDs, block id % 8 picks the XCD,
-// and every column tile of a row tile goes to the same XCD, so the row tile's activations are
-// fetched once into that XCD's L2.
+// Block order is XCD-aware (tile_of): a row tile's column tiles go to one XCD, so the row tile's activations are fetched
+// once into that XCD's L2.
 #include "dh_common.h"
+
+#include <utility>
 
 namespace {
 
-constexpr int kBM = 128;                  // output rows (activation rows) per workgroup
-constexpr int kBN = 128;                  // output columns (weight rows) per workgroup
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
 constexpr int kThreads = 256;
 constexpr int kRowBytes = 128;            // K bytes of a staged row
 constexpr int kPad = 16;
 constexpr int kRS = kRowBytes + kPad;     // LDS row stride
-constexpr int kTileBytes = 128 * kRS;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -59,6 +62,17 @@ __device__ __forceinline__ int seg_of(const GemmArgs& a, int n, int& local) {
 template <typename P>
 __device__ __forceinline__ P pick(int s, P p0, P p1, P p2) {
   return s == 0 ? p0 : (s == 1 ? p1 : p2);
+}
+
+// Tile (mt, nt) of workgroup id: XCD id % 8 (round-robin dispatch) takes a contiguous eighth of the tiles in row-tile-major
+// order, so a row tile's column tiles share the activations in one XCD's L2 and every XCD has work, also with fewer than
+// eight row tiles (row tiles x, x + 8, ... per XCD left XCDs idle there: fp32 M = 128, N = 3072 40.5 -> 24 us).
+__device__ __forceinline__ bool tile_of(const GemmArgs& a, int id, int& mt, int& nt) {
+  const int total = a.mtiles * a.ntiles, per = (total + 7) >> 3;
+  const int lin = (id & 7) * per + (id >> 3);
+  mt = lin / a.ntiles;
+  nt = lin - mt * a.ntiles;
+  return (id >> 3) < per && lin < total;
 }
 
 template <typename T> struct Frag;
@@ -93,100 +107,111 @@ template <> struct Frag<float> {
   }
 };
 
-template <typename T>
+// TM x TN MFMA tiles of 16 x 16 per wave: output tiles of 32 TM rows x 32 TN columns; D: K tiles requested ahead, each in
+// registers of its own
+template <typename T, int TM, int TN, int D>
 __global__ __launch_bounds__(kThreads) void proj_gemm_kernel(GemmArgs a) {
-  __shared__ __align__(16) unsigned char smem[2][2][kTileBytes];   // [buffer][weights | activations]
+  constexpr int BM = 32 * TM, BN = 32 * TN;
+  __shared__ __align__(16) unsigned char sw[2][BN * kRS], sx[2][BM * kRS];
   typedef Frag<T> F;
   constexpr int VE = F::VE;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1;             // the wave's 64 x 64 quadrant
+  const int wm = wave & 1, wn = wave >> 1;             // the wave's quadrant
 
-  // tile of this workgroup: XCD x = id % 8 takes row tiles x, x + 8, ..., each with all its
-  // column tiles in a row
-  const int id = blockIdx.x;
-  const int xcd = id & 7, slot = id >> 3;
-  const int mt = (slot / a.ntiles) * 8 + xcd, nt = slot % a.ntiles;
-  if (mt >= a.mtiles) return;                          // uniform
-  const int m0 = mt * kBM, n0 = nt * kBN;
+  int mt, nt;
+  if (!tile_of(a, blockIdx.x, mt, nt)) return;         // uniform
+  const int m0 = mt * BM, n0 = nt * BN;
 
   // global -> LDS mapping: chunk c = tid + 256 q is row c / 8, 16-byte chunk c % 8 of the row
-  const T* xp[4];
-  const T* wp[4];
+  const T* xp[TM];
+  const T* wp[TN];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+  for (int q = 0; q < TM; ++q) {
+    const int c = tid + kThreads * q;
+    const int m = min(m0 + (c >> 3), a.M - 1);
+    xp[q] = (const T*)a.X + (int64_t)m * a.ldx + (c & 7) * VE;
+  }
+#pragma unroll
+  for (int q = 0; q < TN; ++q) {
     const int c = tid + kThreads * q;
     const int row = c >> 3, cc = c & 7;
-    const int m = min(m0 + row, a.M - 1);
-    xp[q] = (const T*)a.X + (int64_t)m * a.ldx + cc * VE;
     int loc;
     const int n = min(n0 + row, a.Ntot - 1);
     const int s = seg_of(a, n, loc);
     wp[q] = (const T*)pick(s, a.W[0], a.W[1], a.W[2]) + (int64_t)loc * a.K + cc * VE;
   }
-  uint4 px[4], pw[4];
-  auto fetch = [&](int kt) {
+  uint4 rx[D][TM], rw[D][TN];
+  auto fetch = [&](int kt, uint4 (&px)[TM], uint4 (&pw)[TN]) {
     const int k0 = kt * (kRowBytes / (int)sizeof(T));
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      pw[q] = ld16(wp[q] + k0);
-      px[q] = ld16(xp[q] + k0);
-    }
-  };
-  auto stage = [&](int buf) {
+    for (int q = 0; q < TN; ++q) pw[q] = ld16(wp[q] + k0);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int c = tid + kThreads * q;
-      const int off = (c >> 3) * kRS + (c & 7) * 16;
-      *reinterpret_cast<uint4*>(&smem[buf][0][off]) = pw[q];
-      *reinterpret_cast<uint4*>(&smem[buf][1][off]) = px[q];
-    }
+    for (int q = 0; q < TM; ++q) px[q] = ld16(xp[q] + k0);
+  };
+  auto stage = [&](int buf, const uint4 (&px)[TM], const uint4 (&pw)[TN]) {
+    const int off = (tid >> 3) * kRS + (tid & 7) * 16;   // 32 rows further per q
+#pragma unroll
+    for (int q = 0; q < TN; ++q) *reinterpret_cast<uint4*>(&sw[buf][off + 32 * q * kRS]) = pw[q];
+#pragma unroll
+    for (int q = 0; q < TM; ++q) *reinterpret_cast<uint4*>(&sx[buf][off + 32 * q * kRS]) = px[q];
   };
 
-  f32x4 acc[4][4];
+  f32x4 acc[TN][TM];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < TN; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < TM; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int nk = a.K / (kRowBytes / (int)sizeof(T));
-  fetch(0);
-  stage(0);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
+  // K tile kt passes through register set kt mod D: requested D tiles ahead, written to LDS one tile ahead
+  auto step = [&](int kt, auto uc) {
+    constexpr int u = decltype(uc)::value;
     const int cur = kt & 1;
-    if (kt + 1 < nk) fetch(kt + 1);                    // in flight during the multiply
+    if (kt + D < nk) fetch(kt + D, rx[u], rw[u]);      // uniform; set u was staged in the last step
 #pragma unroll
     for (int ks = 0; ks < F::KSTEPS; ++ks) {
-      uint4 wf[4], xf[4];
+      uint4 wf[TN], xf[TM];
       const int kb = ks * 64 + g * 16;                 // byte offset of this lane's k chunk
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        wf[j] = *reinterpret_cast<const uint4*>(&smem[cur][0][(wn * 64 + j * 16 + r) * kRS + kb]);
+      for (int j = 0; j < TN; ++j)
+        wf[j] = *reinterpret_cast<const uint4*>(&sw[cur][(wn * 16 * TN + j * 16 + r) * kRS + kb]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        xf[i] = *reinterpret_cast<const uint4*>(&smem[cur][1][(wm * 64 + i * 16 + r) * kRS + kb]);
+      for (int i = 0; i < TM; ++i)
+        xf[i] = *reinterpret_cast<const uint4*>(&sx[cur][(wm * 16 * TM + i * 16 + r) * kRS + kb]);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) F::mma(acc[j][i], wf[j], xf[i]);
+        for (int i = 0; i < TM; ++i) F::mma(acc[j][i], wf[j], xf[i]);
     }
-    if (kt + 1 < nk) stage(cur ^ 1);
+    constexpr int un = (u + 1) % D;
+    if (kt + 1 < nk) stage(cur ^ 1, rx[un], rw[un]);
     __syncthreads();
-  }
+  };
+  static_for<D>([&](auto uc) {
+    constexpr int u = decltype(uc)::value;
+    if (u < nk) fetch(u, rx[u], rw[u]);
+  });
+  stage(0, rx[0], rw[0]);
+  __syncthreads();
+  int kt = 0;
+  for (; kt + D <= nk; kt += D) static_for<D>([&](auto uc) { step(kt + decltype(uc)::value, uc); });
+  static_for<D>([&](auto uc) {
+    if (kt + decltype(uc)::value < nk) step(kt + decltype(uc)::value, uc);
+  });
 
-  // ---- epilogue: acc[j][i] = out[m][n .. n+3], m = m0 + wm*64 + i*16 + r, n = n0 + wn*64 + j*16 + 4g
+  // ---- epilogue: acc[j][i] = out[m][n .. n+3], m = m0 + 16 (wm TM + i) + r, n = n0 + 16 (wn TN + j) + 4g
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int n = n0 + wn * 64 + j * 16 + 4 * g;
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wn * 16 * TN + j * 16 + 4 * g;
     int loc;
     const int s = seg_of(a, n, loc);
     T* o = (T*)pick(s, a.out[0], a.out[1], a.out[2]);
     const int64_t ld = pick(s, a.ldo[0], a.ldo[1], a.ldo[2]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + wm * 64 + i * 16 + r;
+    for (int i = 0; i < TM; ++i) {
+      const int m = m0 + wm * 16 * TM + i * 16 + r;
       if (m < a.M && n < a.Ntot) F::store4(o + (int64_t)m * ld + loc, acc[j][i]);
     }
   }
@@ -327,7 +352,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void proj_gemm_pp_kernel(GemmArgs a
   const int r = lane & 15, g = lane >> 4;
   const int wm = wave % WGM, wn = wave / WGM;
   const int nk = a.K / 64;
-  const int nvirt = ((a.mtiles + 7) / 8) * 8 * a.ntiles;
+  const int nvirt = (a.mtiles * a.ntiles + 7) / 8 * 8;
 
   // fragment byte offsets within a stage: row R = quadrant base + 16 j + r, chunk 4 ks + g
   const int fw = (wn * 16 * TN + r) * kRowBytes, fx = (wm * 16 * TM + r) * kRowBytes;
@@ -362,9 +387,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void proj_gemm_pp_kernel(GemmArgs a
   uint4 aw[TN], ax[TM], bw[TN], bx[TM];                // step-0 and step-1 operand sets
   int pm0 = -1, pn0 = 0;                               // the tile whose output acc holds
   for (int id = blockIdx.x; id < nvirt; id += gridDim.x) {
-    const int xcd = id & 7, slot = id >> 3;
-    const int mt = (slot / a.ntiles) * 8 + xcd, nt = slot % a.ntiles;
-    if (mt >= a.mtiles) continue;                      // uniform
+    int mt, nt;
+    if (!tile_of(a, id, mt, nt)) continue;             // uniform
     const int m0 = mt * BM, n0 = nt * BN;
 #pragma unroll
     for (int q = 0; q < GX; ++q) {
@@ -445,7 +469,7 @@ int launch_pp_tiles(GemmArgs& a, hipStream_t s, const char* who) {
   constexpr int BM = 32 * TM, BN = 32 * TN;
   a.mtiles = (a.M + BM - 1) / BM;
   a.ntiles = (a.Ntot + BN - 1) / BN;
-  const int64_t nvirt = (int64_t)((a.mtiles + 7) / 8) * 8 * a.ntiles;
+  const int64_t nvirt = ((int64_t)a.mtiles * a.ntiles + 7) / 8 * 8;
   DH_REQUIRE(nvirt < (1ll << 31), DH_ERR_UNSUPPORTED_SHAPE, "%s: M=%d too large", who, a.M);
   proj_gemm_pp_kernel<TM, TN, 2, 2, SWI, S><<<dim3((unsigned)nvirt), dim3(256), 0, s>>>(a);
   return dh_check_launch(who);
@@ -476,13 +500,30 @@ constexpr int64_t kWideGrid = 256;        // persistent workgroups: one per CU (
 // per CU the extra LDS costs occupancy (M = 1024 N = 3072: 12.6 / 14.3 / 16.3).
 // Every form sums the same products in the same k order: outputs are bit-identical across forms
 // and stage counts.
+//
+// The persistent form's last round: with a few tiles more than a multiple of the 256 CUs, most CUs idle while a few compute
+// one more 256 x 256 tile (28-30 us at K = 1024). When less than a quarter of a round is left over, the whole rounds' rows go
+// first and the remaining rows take whatever form fits them, as a second launch (M = 3000, N = 2 x 2816, 264 tiles: 60.8 ->
+// 44.8 us; with 96 tiles left over, M = 4096, the split measured 62.8 against 61.2).
 template <bool SWI>
 int launch_wide(GemmArgs& a, hipStream_t s, const char* who) {
   const int M = a.M, N = a.Ntot;
   if (tiles_of(M, N, 256, 256) >= kWideMinTiles) {
+    const int nt = (N + 255) / 256, mt = (M + 255) / 256;
+    const int64_t rounds = (int64_t)mt * nt / kWideGrid, left = (int64_t)mt * nt - rounds * kWideGrid;
+    const int whole = (int)(rounds * kWideGrid / nt);              // row tiles within the whole rounds
+    if (rounds >= 1 && left > 0 && left < kWideGrid / 4 && whole >= 1) {
+      GemmArgs head = a, tail = a;
+      head.M = whole * 256;
+      tail.M = M - head.M;
+      tail.X = (const bf16_t*)a.X + (int64_t)head.M * a.ldx;
+      for (int i = 0; i < (SWI ? 1 : a.nseg); ++i) tail.out[i] = (bf16_t*)a.out[i] + (int64_t)head.M * a.ldo[i];
+      const int st = launch_wide<SWI>(head, s, who);
+      return st ? st : launch_wide<SWI>(tail, s, who);
+    }
     a.mtiles = (M + 255) / 256;
     a.ntiles = (N + 255) / 256;
-    const int64_t nvirt = (int64_t)((a.mtiles + 7) / 8) * 8 * a.ntiles;
+    const int64_t nvirt = ((int64_t)a.mtiles * a.ntiles + 7) / 8 * 8;
     DH_REQUIRE(nvirt < (1ll << 31), DH_ERR_UNSUPPORTED_SHAPE, "%s: M=%d too large", who, M);
     const unsigned grid = (unsigned)(nvirt < kWideGrid ? nvirt : kWideGrid);
     proj_gemm_pp_kernel<8, 4, 2, 4, SWI, 2><<<dim3(grid), dim3(512), 0, s>>>(a);
@@ -495,6 +536,31 @@ int launch_wide(GemmArgs& a, hipStream_t s, const char* who) {
   if (tiles_of(M, N, 64, 128) >= 768) return launch_pp_tiles<2, 4, SWI>(a, s, who);
   if (tiles_of(M, N, 128, 64) >= 512) return launch_pp_tiles<4, 2, SWI>(a, s, who);
   return launch_pp_tiles<4, 4, SWI>(a, s, who);
+}
+
+// The register-staged kernel, one workgroup per tile of 32 TM x 32 TN.
+template <typename T, int TM, int TN, int D>
+int launch_staged(GemmArgs& a, hipStream_t s, const char* who) {
+  a.mtiles = (a.M + 32 * TM - 1) / (32 * TM);
+  a.ntiles = (a.Ntot + 32 * TN - 1) / (32 * TN);
+  const int64_t grid = ((int64_t)a.mtiles * a.ntiles + 7) / 8 * 8;
+  DH_REQUIRE(grid < (1ll << 31), DH_ERR_UNSUPPORTED_SHAPE, "%s: M=%d too large", who, a.M);
+  proj_gemm_kernel<T, TM, TN, D><<<dim3((unsigned)grid), dim3(kThreads), 0, s>>>(a);
+  return dh_check_launch(who);
+}
+
+// fp32 tile: the form with the least ceil(tiles / 256 CUs) rounds times its time a round (K = 1024 on MI355X, us: 64 x 32
+// 9.3, 64 x 64 18, 128 x 128 65, and ~5.5 / 5.5 / 8 once). A short launch of 128 x 128 tiles leaves CUs idle and each busy
+// one takes the tile's full time: N = 1024, us, 64 x 32 / 64 x 64 / 128 x 128: M = 128 14.7 / 22.9 / 71.5, M = 1024 23.5 /
+// 23.9 / 73.2, M = 1501 32.8 / 39.5 / 73.5, M = 3002 68.8 / 57.6 / 74.4, M = 4096 81.2 / 75.6 / 74.9; N = 3072: M = 128 16.4 /
+// 23.5 / 72.0, M = 1501 92.5 / 93.1 / 133.7, M = 3002 176 / 164 / 201 (128 x 128 tiles alone: 209), M = 8192 465 / 431 / 397.
+// Every form sums the same products in the same k order.
+int launch_f32(GemmArgs& a, hipStream_t s, const char* who) {
+  auto rounds = [&](int bm, int bn) { return (tiles_of(a.M, a.Ntot, bm, bn) + 255) / 256; };
+  const int64_t c21 = 93 * rounds(64, 32) + 55, c22 = 180 * rounds(64, 64) + 55, c44 = 650 * rounds(128, 128) + 80;
+  if (c44 <= c22 && c44 <= c21) return launch_staged<float, 4, 4, 2>(a, s, who);
+  if (c22 <= c21) return launch_staged<float, 2, 2, 2>(a, s, who);
+  return launch_staged<float, 2, 1, 2>(a, s, who);
 }
 
 }  // namespace
@@ -538,15 +604,8 @@ extern "C" int dh_proj_gemm(int dtype, const void* X, int64_t ldx, int M, int K,
   for (int i = 0; i < nseg; ++i)
     wide = wide && N[i] % 8 == 0 && (int64_t)N[i] * K * esz < (1ll << 31) && ldo[i] % 8 == 0 && aligned(out[i], 16);
   if (wide) return launch_wide<false>(a, s, who);
-  a.mtiles = (M + kBM - 1) / kBM;
-  a.ntiles = (total + kBN - 1) / kBN;
-  const int64_t grid = (int64_t)((a.mtiles + 7) / 8) * 8 * a.ntiles;
-  DH_REQUIRE(grid < (1ll << 31), DH_ERR_UNSUPPORTED_SHAPE, "%s: M=%d too large", who, M);
-  if (dtype == DH_BF16)
-    proj_gemm_kernel<bf16_t><<<dim3((unsigned)grid), dim3(kThreads), 0, s>>>(a);
-  else
-    proj_gemm_kernel<float><<<dim3((unsigned)grid), dim3(kThreads), 0, s>>>(a);
-  return dh_check_launch(who);
+  if (dtype == DH_BF16) return launch_staged<bf16_t, 4, 4, 1>(a, s, who);
+  return launch_f32(a, s, who);
 }
 
 // out[m, f] = round(round(silu(round(X[m] . Wg[f]))) * round(X[m] . Wu[f])): a SwiGLU layer's

@@ -403,9 +403,16 @@ def input_projections(x, mixer):
 # projection (the mixer's and attention's linear_out) 6.7 / 8.9 at 1024, 9.1 / 10.4 at 2048,
 # 12.9 / 13.0 at 4096, and the SwiGLU down projection (1024 x 2816) 12.1 / 14.0 at 1024, 19.8 / 18.8
 # at 2048 (the launches of at most 512 tiles keep two or three K tiles in flight).
+# fp32: the 1024 x 1024 output projection 23.9 / 36.7 / 57.6 / 75.6 us at 1024 / 2048 / 3002 / 4096 rows against 20.6 / 36.7
+# / 68.2 / 63.8 for the library.
 QKV_GEMM_MAX_ROWS = 4096
 OUT_GEMM_MAX_ROWS = 2048
+OUT_GEMM_MAX_ROWS_F32 = 3072
 DOWN_GEMM_MAX_ROWS = 1024
+
+
+def out_max_rows(dtype):
+    return OUT_GEMM_MAX_ROWS if dtype == torch.bfloat16 else OUT_GEMM_MAX_ROWS_F32
 
 
 def project(x, linears, max_rows):
@@ -441,7 +448,7 @@ def mixer_layer_fits(mixer, x):
         return False
     d, dt = mixer.embed_dim, x.dtype
     return (x.dim() == 3 and type(x) in _PLAIN and dt in (torch.float32, torch.bfloat16) and x.shape[-1] == d
-            and 0 < x.shape[0] * x.shape[1] <= OUT_GEMM_MAX_ROWS and d % 64 == 0
+            and 0 < x.shape[0] * x.shape[1] <= out_max_rows(dt) and d % 64 == 0
             and all(w.dtype == dt and b.dtype == dt and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
                     and w.shape[-1] == d for w, b in mixer._gate_params())
             and all(plain_linear(l, dt, d) and l.weight.shape[0] == d

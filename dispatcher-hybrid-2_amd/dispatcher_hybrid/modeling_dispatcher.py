@@ -192,8 +192,8 @@ class DispatcherMixer(nn.Module):
         else:
             # inference: activated gates written head-major, then the level scan (two launches)
             V = fused_gate_scan(A, Bs, Wi, Wf, Wr, bi, bf, br, n_lv, m3, V0, H)
-            from .fused_gates import OUT_GEMM_MAX_ROWS, project
-            return project(V, [self.linear_out], OUT_GEMM_MAX_ROWS)[0]
+            from .fused_gates import out_max_rows, project
+            return project(V, [self.linear_out], out_max_rows(V.dtype))[0]
         return self.linear_out(V)
 
 

@@ -111,8 +111,8 @@ struct MathBf16 {
       af[2 * j + 1] = __uint_as_float(aw[j] & 0xffff0000u);
     }
   }
-  __device__ __forceinline__ static void mma3(f32x4 (&acc)[3], const float (&af)[8], const uint4& bv,
-                                              const uint4 (&w)[3]) {
+  // relu(a + b)^2 of a fragment, rounded where the eager path rounds
+  __device__ __forceinline__ static uint4 hidden(const float (&af)[8], const uint4& bv) {
     const uint32_t bw[4] = {bv.x, bv.y, bv.z, bv.w};
     uint32_t hw[4];
 #pragma unroll
@@ -122,8 +122,13 @@ struct MathBf16 {
       const float x1 = round_bf16(fmaxf(af[2 * j + 1] + __uint_as_float(bw[j] & 0xffff0000u), 0.f));
       hw[j] = pack_bf16x2(x0 * x0, x1 * x1);
     }
+    return make_uint4(hw[0], hw[1], hw[2], hw[3]);
+  }
+  __device__ __forceinline__ static void mma3(f32x4 (&acc)[3], const float (&af)[8], const uint4& bv,
+                                              const uint4 (&w)[3]) {
+    const uint4 hv = hidden(af, bv);
     bf16x8 hid, wi, wf, wr;
-    __builtin_memcpy(&hid, hw, 16);
+    __builtin_memcpy(&hid, &hv, 16);
     __builtin_memcpy(&wi, &w[0], 16);
     __builtin_memcpy(&wf, &w[1], 16);
     __builtin_memcpy(&wr, &w[2], 16);
@@ -171,6 +176,55 @@ struct MathF32 {
     *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
   }
 };
+
+// The outputs of one MFMA tile: lane (head n, lane group g) holds positions tb .. tb + 3 = 4 g .. of the three gates.
+template <typename M, bool HAS_MASK>
+__device__ __forceinline__ void write_gates(const FwdArgs& a, const f32x4 (&acc)[3], int b, int l, int n, int tb) {
+  typedef typename M::T T;
+  if (l >= a.n_lv || n >= a.H) return;
+  const float bias[3] = {bias_at<T>(a, a.bi, l * a.H + n), bias_at<T>(a, a.bf, l * a.H + n), bias_at<T>(a, a.br, l * a.H + n)};
+  T* outs[3] = {(T*)a.oi, (T*)a.of, (T*)a.orr};
+  const int64_t base = (int64_t)b * a.sob + (int64_t)l * a.sol + (int64_t)n * a.soh;
+  float v[3][4];
+#pragma unroll
+  for (int x = 0; x < 3; ++x)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[x][i] = acc[x][i] + bias[x];
+  if (a.activate) {
+    // a = sigmoid(pre_i) * M, f = sigmoid(pre_f) * M + 1 - M, r = sigmoid(pre_r), rounded where
+    // the eager bf16 path rounds (pre-activation, sigmoid output); M = [t >= 2^l] * [mask > 0]
+    float mval[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      mval[i] = 1.f;
+      if (HAS_MASK) {
+        const int to = min(tb + i, a.T - 1);
+        mval[i] = Elem<T>::load((const T*)a.mask + (int64_t)b * a.smb + (int64_t)to * a.smt + (int64_t)l * a.sml);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float m = (tb + i >= (1 << l) && mval[i] > 0.f) ? 1.f : 0.f;
+      const float si = M::rnd(dh_sigmoid(M::rnd(v[0][i])));
+      const float sf = M::rnd(dh_sigmoid(M::rnd(v[1][i])));
+      const float sr = M::rnd(dh_sigmoid(M::rnd(v[2][i])));
+      v[0][i] = si * m;
+      v[1][i] = sf * m + (1.f - m);
+      v[2][i] = sr;
+    }
+  }
+  const bool vec = a.vec_out && tb + 3 < a.T;
+#pragma unroll
+  for (int x = 0; x < 3; ++x) {
+    if (vec) {
+      M::store4(outs[x] + base + tb, v[x]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (tb + i < a.T) outs[x][base + (int64_t)(tb + i) * a.sot] = M::out(v[x][i]);
+    }
+  }
+}
 
 template <typename M, int LG, int KU, bool HAS_MASK>
 __global__ __launch_bounds__(kThreads) void gate_preacts_fwd_kernel(FwdArgs a) {
@@ -261,53 +315,8 @@ __global__ __launch_bounds__(kThreads) void gate_preacts_fwd_kernel(FwdArgs a) {
     }
     // C fragment: column (head) lane%16, rows 4*(lane/16) + i
     const int tb = blockIdx.x * kTileT + wave * 16 + g * 4;
-    const bool vec = a.vec_out && tb + 3 < a.T;
 #pragma unroll
-    for (int j = 0; j < LG; ++j) {
-      const int l = l0 + j;
-      if (l >= a.n_lv || n >= a.H) continue;
-      const float bias[3] = {bias_at<T>(a, a.bi, l * a.H + n), bias_at<T>(a, a.bf, l * a.H + n), bias_at<T>(a, a.br, l * a.H + n)};
-      T* outs[3] = {(T*)a.oi, (T*)a.of, (T*)a.orr};
-      const int64_t base = (int64_t)b * a.sob + (int64_t)l * a.sol + (int64_t)n * a.soh;
-      float v[3][4];
-#pragma unroll
-      for (int x = 0; x < 3; ++x)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[x][i] = acc[j][x][i] + bias[x];
-      if (a.activate) {
-        // a = sigmoid(pre_i) * M, f = sigmoid(pre_f) * M + 1 - M, r = sigmoid(pre_r), rounded where
-        // the eager bf16 path rounds (pre-activation, sigmoid output); M = [t >= 2^l] * [mask > 0]
-        float mval[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          mval[i] = 1.f;
-          if (HAS_MASK) {
-            const int to = min(tb + i, a.T - 1);
-            mval[i] = Elem<T>::load((const T*)a.mask + (int64_t)b * a.smb + (int64_t)to * a.smt + (int64_t)l * a.sml);
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float m = (tb + i >= (1 << l) && mval[i] > 0.f) ? 1.f : 0.f;
-          const float si = M::rnd(dh_sigmoid(M::rnd(v[0][i])));
-          const float sf = M::rnd(dh_sigmoid(M::rnd(v[1][i])));
-          const float sr = M::rnd(dh_sigmoid(M::rnd(v[2][i])));
-          v[0][i] = si * m;
-          v[1][i] = sf * m + (1.f - m);
-          v[2][i] = sr;
-        }
-      }
-#pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        if (vec) {
-          M::store4(outs[x] + base + tb, v[x]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (tb + i < a.T) outs[x][base + (int64_t)(tb + i) * a.sot] = M::out(v[x][i]);
-        }
-      }
-    }
+    for (int j = 0; j < LG; ++j) write_gates<M, HAS_MASK>(a, acc[j], b, l0 + j, n, tb);
   }
 }
 
@@ -349,16 +358,22 @@ constexpr int kLdsRow = kLdsKB + 16;             // padded LDS row: 144 bytes
 // occupancy by register footprint: (levels x row blocks) accumulators plus two chunks of fragments
 template <int LG, int MB> struct LdsOcc { static constexpr int value = LG * MB >= 4 ? 2 : 3; };
 
-template <typename M, int LG, int MB, bool HAS_MASK>
-__global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preacts_fwd_lds_kernel(FwdArgs a) {
+// KS > 1 (one-level tiles): KS groups of 4 waves share the tile, group q taking the q-th part of the K chunks (its own weight
+// buffers); the groups' sums are added in order at the end. A short prefill has about one workgroup per CU, whose 4 waves (one
+// per SIMD) leave every LDS, cross-lane and memory round trip exposed; 16 waves cover them with each other.
+template <typename M, int LG, int MB, int KS, bool HAS_MASK>
+__global__ __launch_bounds__(kThreads * KS, (KS > 1 ? KS : LdsOcc<LG, MB>::value)) void gate_preacts_fwd_lds_kernel(FwdArgs a) {
+  static_assert(KS == 1 || (LG == 1 && MB == 1), "K is split for one-level tiles");
   typedef typename M::T T;
   constexpr int VE = 16 / (int)sizeof(T);        // elements of a 16-byte piece
   constexpr int P = 64 * MB;                     // positions per workgroup
   constexpr int WBYTES = LG * 3 * 16 * kLdsRow;  // one LDS weight buffer
   constexpr int PIECES = LG * 3 * 16 * (kLdsKB / 16);   // 16-byte pieces of one chunk
   constexpr int PPT = (PIECES + kThreads - 1) / kThreads;
-  __shared__ __align__(16) unsigned char wl[2][WBYTES];
-  const int tid = threadIdx.x;
+  __shared__ __align__(16) unsigned char wl_[KS][2][WBYTES];
+  const int tid = threadIdx.x & (kThreads - 1);        // within the wave group
+  const int grp = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
+  auto& wl = wl_[grp];
   const int lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
   const int b = blockIdx.z;
@@ -480,7 +495,8 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
       }
     }
   };
-  const int nchunk_ = a.GH * (int)sizeof(T) / kLdsKB;
+  const int nchunk_ = a.GH * (int)sizeof(T) / kLdsKB / KS;     // of this group; the host checks divisibility
+  const int kbase = grp * nchunk_ * kLdsKB;
   // chunk c: request chunk c+1 (weights and fragments), compute chunk c, store the weights of c+1
   auto chunk = [&](int c, const uint4 (&cA)[2][MB], const uint4 (&cB)[2][MB][LG], uint4 (&nA)[2][MB],
                    uint4 (&nB)[2][MB][LG]) {
@@ -521,8 +537,8 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
       constexpr int u = decltype(uc)::value;             // c % NS
       constexpr int uf = (u + NS - 1) % NS, un = (u + 1) % NS;
       if (c + NS - 1 < nchunk_) {                        // uniform
-        w_fetch3((c + NS - 1) * kLdsKB, sW[uf]);
-        fetch((c + NS - 1) * kLdsKB, sA[uf], sB[uf]);
+        w_fetch3(kbase + (c + NS - 1) * kLdsKB, sW[uf]);
+        fetch(kbase + (c + NS - 1) * kLdsKB, sA[uf], sB[uf]);
       }
       compute(sA[u], sB[u], c & 1);
       if (c + 1 < nchunk_) w_store3((c + 1) & 1, sW[un]);
@@ -531,8 +547,8 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
     static_for<NS - 1>([&](auto uc) {
       constexpr int u = decltype(uc)::value;
       if (u < nchunk_) {
-        w_fetch3(u * kLdsKB, sW[u]);
-        fetch(u * kLdsKB, sA[u], sB[u]);
+        w_fetch3(kbase + u * kLdsKB, sW[u]);
+        fetch(kbase + u * kLdsKB, sA[u], sB[u]);
       }
     });
     w_store3(0, sW[0]);
@@ -555,56 +571,121 @@ __global__ __launch_bounds__(kThreads, (LdsOcc<LG, MB>::value)) void gate_preact
     if (c < nchunk_) chunk(c, xA, xB, yA, yB);
   }
 
+  if constexpr (KS > 1) {
+    // the other groups hand their sums over through the weight buffers (12 floats per lane; 36 KB of 54)
+    static_assert((KS - 1) * 3 * kThreads * 16 <= KS * 2 * WBYTES, "the sums fit the weight buffers");
+    f32x4* sums = reinterpret_cast<f32x4*>(&wl_[0][0][0]);
+    if (grp > 0)
+#pragma unroll
+      for (int x = 0; x < 3; ++x) sums[((grp - 1) * 3 + x) * kThreads + tid] = acc[0][0][x];
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int q = 0; q < KS - 1; ++q)
+#pragma unroll
+      for (int x = 0; x < 3; ++x) acc[0][0][x] += sums[(q * 3 + x) * kThreads + tid];
+  }
+
   // ---- epilogue: C fragment column (head) r, rows 4g + i of row block mb
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int tb = tbase + 16 * mb + g * 4;
-    const bool vec = a.vec_out && tb + 3 < a.T;
+  for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-    for (int j = 0; j < LG; ++j) {
-      const int l = l0 + j;
-      if (l >= a.n_lv || r >= a.H) continue;
-      const float bias[3] = {bias_at<T>(a, a.bi, l * a.H + r), bias_at<T>(a, a.bf, l * a.H + r), bias_at<T>(a, a.br, l * a.H + r)};
-      T* outs[3] = {(T*)a.oi, (T*)a.of, (T*)a.orr};
-      const int64_t base = (int64_t)b * a.sob + (int64_t)l * a.sol + (int64_t)r * a.soh;
-      float v[3][4];
+    for (int j = 0; j < LG; ++j) write_gates<M, HAS_MASK>(a, acc[mb][j], b, l0 + j, r, tbase + 16 * mb + g * 4);
+}
+
+// ---------------------------------------------------------------------------------------------
+// bf16 forward in one shot, for launches of at most one (64-position tile, level) per CU (H <= 16, GH = 256 NC <= 1024).
+//
+// With nothing else on a CU, the chunked kernel's time is its chain of 16 chunk round trips. Here 16 waves request the whole
+// tile at once: the level's weights go to LDS entire (3 x 16 rows, 99 KB at GH = 1024, rows padded by 16 bytes so the 16 rows
+// a fragment read takes fall on distinct banks), and wave (row group w, quarter q) loads a quarter of K of its 16 rows and
+// forms that quarter of the hidden tile in registers. Then the quarters multiply one after the other, the accumulators
+// handed over through LDS: the same products in the same k order as the chunked kernel, hence the same bits (a split with
+// the quarters' sums added up was 4 us faster than the chunked kernel, too, but moved bf16 results).
+// ---------------------------------------------------------------------------------------------
+template <int NC, bool HAS_MASK>
+__global__ __launch_bounds__(1024) void gate_preacts_once_kernel(FwdArgs a) {
+  typedef bf16_t T;
+  constexpr int kRow = NC * 512 + 16;                        // padded LDS row: GH bf16 and 16 bytes
+  constexpr int PIECES = 48 * NC * 32, PPT = (PIECES + 1023) / 1024;
+  __shared__ __align__(16) unsigned char wl[48 * kRow];
+  __shared__ f32x4 hand[3][256];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), rw = wave & 3, q = wave >> 2;
+  const int r = lane & 15, g = lane >> 4;
+  const int b = blockIdx.z, l = blockIdx.y;
+  const int tbase = blockIdx.x * 64 + rw * 16;
+  const uint32_t row_bytes = (uint32_t)((int64_t)a.T * a.sat * 2);
+  const __amdgpu_buffer_rsrc_t rA = buf_rsrc((const T*)a.A + (int64_t)b * a.sab, row_bytes);
+  const __amdgpu_buffer_rsrc_t rB = buf_rsrc((const T*)a.B + (int64_t)b * a.sab, row_bytes);
+
+  // activations in the coalesced order (see the chunked kernel), masked rows of B past the range
+  const int t = tbase + (lane >> 2), tc = min(t, a.T - 1), src = tc - (1 << l), cpiece = lane & 3;
+  float mv = 1.f;
+  if (HAS_MASK) mv = Elem<T>::load((const T*)a.mask + (int64_t)b * a.smb + (int64_t)tc * a.smt + (int64_t)l * a.sml);
+  const bool keep = t < a.T && src >= 0 && mv > 0.f;
+  const uint32_t aoff = (uint32_t)(((int64_t)tc * a.sat + cpiece * 8) * 2);
+  const uint32_t boff = keep ? (uint32_t)(((int64_t)src * a.sat + cpiece * 8) * 2) : 0x80000000u;
+  uint4 fa[2 * NC], fb[2 * NC];
 #pragma unroll
-      for (int x = 0; x < 3; ++x)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[x][i] = acc[mb][j][x][i] + bias[x];
-      if (a.activate) {
-        float mval[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          mval[i] = 1.f;
-          if (HAS_MASK) {
-            const int to = min(tb + i, a.T - 1);
-            mval[i] = Elem<T>::load((const T*)a.mask + (int64_t)b * a.smb + (int64_t)to * a.smt + (int64_t)l * a.sml);
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float m = (tb + i >= (1 << l) && mval[i] > 0.f) ? 1.f : 0.f;
-          const float si = M::rnd(dh_sigmoid(M::rnd(v[0][i])));
-          const float sf = M::rnd(dh_sigmoid(M::rnd(v[1][i])));
-          const float sr = M::rnd(dh_sigmoid(M::rnd(v[2][i])));
-          v[0][i] = si * m;
-          v[1][i] = sf * m + (1.f - m);
-          v[2][i] = sr;
-        }
-      }
-#pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        if (vec) {
-          M::store4(outs[x] + base + tb, v[x]);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (tb + i < a.T) outs[x][base + (int64_t)(tb + i) * a.sot] = M::out(v[x][i]);
-        }
-      }
-    }
+  for (int s = 0; s < 2 * NC; ++s) {
+    const uint32_t kb = (uint32_t)((q * 2 * NC + s) * 64);
+    fa[s] = bld16(rA, aoff, kb);
+    fb[s] = bld16(rB, boff, kb);
   }
+  uint4 wv[PPT];
+#pragma unroll
+  for (int i = 0; i < PPT; ++i) {
+    const int p = min(tid + i * 1024, PIECES - 1), row = p / (NC * 32), c = p - row * (NC * 32);
+    const int x = row >> 4, h = min(row & 15, a.H - 1);
+    const T* w = (const T*)(x == 0 ? a.Wi : x == 1 ? a.Wf : a.Wr);
+    wv[i] = ld16(w + (int64_t)l * a.swl + (int64_t)h * a.swh + c * 8);
+  }
+  // the hidden quarter: MFMA A-operand fragments of 32 k each
+  const int bperm = 4 * (4 * r + g);
+  auto to_mfma = [&](const uint4& v) {
+    return make_uint4((uint32_t)__builtin_amdgcn_ds_bpermute(bperm, (int)v.x),
+                      (uint32_t)__builtin_amdgcn_ds_bpermute(bperm, (int)v.y),
+                      (uint32_t)__builtin_amdgcn_ds_bpermute(bperm, (int)v.z),
+                      (uint32_t)__builtin_amdgcn_ds_bpermute(bperm, (int)v.w));
+  };
+  uint4 hid[2 * NC];
+#pragma unroll
+  for (int s = 0; s < 2 * NC; ++s) {
+    float af[8];
+    MathBf16::unpack_a(to_mfma(fa[s]), af);
+    hid[s] = MathBf16::hidden(af, to_mfma(fb[s]));
+  }
+#pragma unroll
+  for (int i = 0; i < PPT; ++i) {
+    const int p = tid + i * 1024, row = p / (NC * 32), c = p - row * (NC * 32);
+    if (p < PIECES) *reinterpret_cast<uint4*>(&wl[row * kRow + c * 16]) = wv[i];
+  }
+  __syncthreads();
+  f32x4 acc[3];
+#pragma unroll
+  for (int x = 0; x < 3; ++x) acc[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int turn = 0; turn < 4; ++turn) {
+    if (q == turn) {                                         // uniform over a wave
+      if (turn > 0)
+#pragma unroll
+        for (int x = 0; x < 3; ++x) acc[x] = hand[x][rw * 64 + lane];
+#pragma unroll
+      for (int s = 0; s < 2 * NC; ++s)
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+          const uint4 w = *reinterpret_cast<const uint4*>(&wl[(x * 16 + r) * kRow + (q * 2 * NC + s) * 64 + g * 16]);
+          acc[x] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, hid[s]), __builtin_bit_cast(bf16x8, w),
+                                                           acc[x], 0, 0, 0);
+        }
+      if (turn < 3)
+#pragma unroll
+        for (int x = 0; x < 3; ++x) hand[x][rw * 64 + lane] = acc[x];
+    }
+    __syncthreads();
+  }
+  if (q == 3) write_gates<MathBf16, HAS_MASK>(a, acc, b, l, r, tbase + g * 4);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -765,27 +846,52 @@ void launch_fwd(const FwdArgs& a, dim3 grid, hipStream_t s) {
     gate_preacts_fwd_kernel<M, LG, KU, false><<<grid, dim3(kThreads), 0, s>>>(a);
 }
 
-template <typename M, int LG, int MB>
+template <typename M, int LG, int MB, int KS>
 void launch_fwd_lds(const FwdArgs& a, hipStream_t s) {
   constexpr int P = 64 * MB;
   dim3 grid((a.T + P - 1) / P, (a.n_lv + LG - 1) / LG, a.b);
   if (a.mask)
-    gate_preacts_fwd_lds_kernel<M, LG, MB, true><<<grid, dim3(kThreads), 0, s>>>(a);
+    gate_preacts_fwd_lds_kernel<M, LG, MB, KS, true><<<grid, dim3(kThreads * KS), 0, s>>>(a);
   else
-    gate_preacts_fwd_lds_kernel<M, LG, MB, false><<<grid, dim3(kThreads), 0, s>>>(a);
+    gate_preacts_fwd_lds_kernel<M, LG, MB, KS, false><<<grid, dim3(kThreads * KS), 0, s>>>(a);
 }
 
 // Tile per workgroup (measured on MI355X at the released widths): two levels x 64 positions once
 // the launch has >= 1024 workgroups (b = 8, T = 4096: 135 us, against 143 / 155 / 224 for three /
 // four / six levels -- fewer waves per SIMD -- and 169 for 2 x 128), else one level x 64 positions,
-// the most workgroups for short prefills. Handing each XCD whole batch rows (a tile's level groups
+// the most workgroups for short prefills. With at most one of those per CU, bf16 takes the one-shot kernel (b = 1, us, chunked /
+// one-shot: T = 24 13.5 / 9.1, T = 200 14.9 / 9.6, T = 1024, 176 workgroups, 15.3 / 11.1; past one per CU its 111 KB of LDS
+// leave no second workgroup) and fp32 splits K over four wave groups, with at most 448 workgroups over two (one / two / four
+// groups: T = 200 30.4 / 23.9 / 21.2, T = 1024 31.0 / 24.8 / 22.5, T = 2048, 384 workgroups, 40.0 / 36.9 / 41.5, T = 3840, 720,
+// 55.4 / 58.1 / 66.3). Handing each XCD whole batch rows (a tile's level groups
 // and its lagged B rows then share one L2) measured the same, 136 us, and so did rounding the hidden
 // tile once instead of at the eager path's two points (the launch is not bound by that VALU work).
+template <int NC>
+void launch_once(const FwdArgs& a, hipStream_t s) {
+  const dim3 grid((a.T + 63) / 64, a.n_lv, a.b);
+  if (a.mask) gate_preacts_once_kernel<NC, true><<<grid, dim3(1024), 0, s>>>(a);
+  else gate_preacts_once_kernel<NC, false><<<grid, dim3(1024), 0, s>>>(a);
+}
+
 template <typename M>
 void dispatch_fwd_lds(const FwdArgs& a, hipStream_t s) {
   const int64_t wgs21 = (int64_t)((a.T + 63) / 64) * ((a.n_lv + 1) / 2) * a.b;
-  if (wgs21 >= 1024) launch_fwd_lds<M, 2, 1>(a, s);
-  else launch_fwd_lds<M, 1, 1>(a, s);
+  const int64_t wgs1 = (int64_t)((a.T + 63) / 64) * a.n_lv * a.b;
+  const int nch = a.GH * (int)sizeof(typename M::T) / kLdsKB;
+  if constexpr (sizeof(typename M::T) == 2) {
+    if (wgs1 <= 256 && a.GH <= 1024 && a.GH % 256 == 0) {
+      if (a.GH == 1024) launch_once<4>(a, s);
+      else if (a.GH == 768) launch_once<3>(a, s);
+      else if (a.GH == 512) launch_once<2>(a, s);
+      else launch_once<1>(a, s);
+      return;
+    }
+  } else {
+    if (wgs1 <= 256 && nch % 4 == 0) return launch_fwd_lds<M, 1, 1, 4>(a, s);
+    if (wgs1 <= 448 && nch % 2 == 0) return launch_fwd_lds<M, 1, 1, 2>(a, s);
+  }
+  if (wgs21 >= 1024) launch_fwd_lds<M, 2, 1, 1>(a, s);
+  else launch_fwd_lds<M, 1, 1, 1>(a, s);
 }
 
 template <typename M>

@@ -29,6 +29,8 @@ from typing import List, Optional
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _hip
 
@@ -304,7 +306,7 @@ def fused_gate_scan(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, num_heads):
     fused_level_scan(*fused_gate_preacts(...), mask, V0, num_heads, n_lv) up to the bf16 rounding
     of the activated gates, which follows the eager path (reference
     dispatcher_hybrid/modeling_dispatcher.py:86-88, 100-121)."""
-    if type(A) is torch.Tensor and not torch.compiler.is_compiling() and not transforms_active():
+    if type(A) is torch.Tensor and plain_eager():
         return _gate_scan_body(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
     return torch.ops.dispatcher.gate_scan_fwd(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
 
@@ -412,7 +414,10 @@ DOWN_GEMM_MAX_ROWS = 1024
 
 
 def out_max_rows(dtype):
-    return OUT_GEMM_MAX_ROWS if dtype == torch.bfloat16 else OUT_GEMM_MAX_ROWS_F32
+    # (under autocast the library call casts to the autocast dtype: the line between the two stays where it was)
+    if dtype == torch.bfloat16 or torch.is_autocast_enabled("cuda"):
+        return OUT_GEMM_MAX_ROWS
+    return OUT_GEMM_MAX_ROWS_F32
 
 
 def project(x, linears, max_rows):
@@ -425,17 +430,21 @@ def project(x, linears, max_rows):
     return [l(x) for l in linears]
 
 
-# whether a torch.func transform (grad, vmap, ...) wraps the tensors: their memory cannot be handed to a kernel directly
-transforms_active = getattr(torch._C, "_are_functorch_transforms_active", lambda: False)
+def plain_eager():
+    """Whether kernels may be launched without a registered operation around them: no compiler, tracer, torch.func transform
+    (grad, vmap, ...), forward-mode level or dispatch mode looks at the tensors' operations."""
+    return not (torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active() or torch.jit.is_tracing()
+                or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0)
 
 
 def plain_linear(l, dtype, n_in):
-    """A bias-free nn.Linear itself (no subclass, adapter, parametrization or hook that a direct use of its weight would
-    pass by) with a plain contiguous weight of this dtype and input width."""
+    """A bias-free nn.Linear itself (no subclass, adapter, parametrization, replaced forward or hook that a direct use of its
+    weight would pass by) with a plain contiguous weight of this dtype and input width."""
     w = l.weight if type(l) is nn.Linear else None
     return (w is not None and l.bias is None and type(w) in _PLAIN and w.dtype == dtype
             and w.shape[1] == n_in and w.is_contiguous() and w.data_ptr() % 16 == 0
-            and not (l._forward_hooks or l._forward_pre_hooks or l._backward_hooks or l._backward_pre_hooks))
+            and not (l._forward_hooks or l._forward_pre_hooks or l._backward_hooks or l._backward_pre_hooks
+                     or "forward" in l.__dict__ or _has_any_global_hook()))
 
 
 _PLAIN = (torch.Tensor, nn.Parameter)
@@ -444,7 +453,7 @@ _PLAIN = (torch.Tensor, nn.Parameter)
 def mixer_layer_fits(mixer, x):
     """Whether mixer_layer takes this layer and input: few enough rows that both products run on dh_proj_gemm, one dtype
     throughout, plain bias-free projections, plain eager execution."""
-    if torch.compiler.is_compiling() or transforms_active():
+    if not plain_eager():
         return False
     d, dt = mixer.embed_dim, x.dtype
     return (x.dim() == 3 and type(x) in _PLAIN and dt in (torch.float32, torch.bfloat16) and x.shape[-1] == d

@@ -23,7 +23,7 @@ import torch.nn.functional as F
 
 from . import _hip
 from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch,
-                          _preacts_launch, _rows16, fused_projections, plain_linear, transforms_active)
+                          _preacts_launch, _rows16, fused_projections, plain_eager, plain_linear)
 
 SCAN_MAX_LEN = 4096
 SCAN_MAX_LEVELS = 12
@@ -206,7 +206,7 @@ def mixer_fits(mixer, x, mask, n_lv):
     """Whether mixer_train takes this layer and input: one dtype (fp32 or bf16) throughout and no autocast, plain bias-free
     projections, the training scan's limits, and plain eager execution (a compiler gets the layer-by-layer form,
     whose gate path is one registered operation, and a torch.func transform that operation's refusal)."""
-    if torch.compiler.is_compiling() or transforms_active():
+    if not plain_eager():
         return False
     d, H, dt = mixer.embed_dim, mixer.num_heads, x.dtype
     if not (x.dim() == 3 and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
@@ -276,7 +276,7 @@ def mixer_train(mixer, x, mask, n_lv):
 def attention_fits(attn, x):
     """Whether attention_train takes this layer and input: bf16 throughout and no autocast, 64-wide heads, plain bias-free
     projections, plain eager execution."""
-    if torch.compiler.is_compiling() or transforms_active():
+    if not plain_eager():
         return False
     d = attn.embed_dim
     return (x.dim() == 3 and x.is_cuda and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
@@ -284,6 +284,22 @@ def attention_fits(attn, x):
             and not torch.is_autocast_enabled("cuda") and x.numel() * 3 * x.element_size() < 2 ** 31
             and all(plain_linear(l, x.dtype, d) and l.weight.shape[0] == d
                     for l in (attn.linear_q, attn.linear_k, attn.linear_v, attn.linear_out)))
+
+
+def _attention_grads(inputs, need, dout, cos, sin, H, window):
+    """The gradients of an attention layer's (x, W_q, W_k, W_v, W_out) as torch operations that autograd can differentiate
+    again; in fp32 (a batched bf16 product with a transposed operand is not used)."""
+    from .modeling_dispatcher import causal_window_attention, rope_rotate
+    inputs = [t.view_as(t) for t in inputs]                                    # (tied weights: a gradient for each use)
+    x, *W = (t.float() for t in inputs)
+    b, T, d = x.shape
+    q, k, v = (F.linear(x, w).view(b, T, H, d // H).transpose(1, 2) for w in W[:3])
+    q, k = (rope_rotate(t, cos.float(), sin.float()) for t in (q, k))
+    y = causal_window_attention(q, k, v, window).transpose(1, 2).reshape(b, T, d)
+    out = F.linear(y, W[3]).to(inputs[0].dtype)
+    wanted = [t for t, n in zip(inputs, need) if n]
+    g = iter(torch.autograd.grad(out, wanted, dout, create_graph=True))
+    return [next(g) if n else None for n in need[:5]]
 
 
 class _AttentionTrain(torch.autograd.Function):
@@ -306,16 +322,18 @@ class _AttentionTrain(torch.autograd.Function):
             y.stride(1), p(kv[0]), p(kv[1]), p(lse), b, T, H, hd, window, _hip.stream_handle(x.device))
         _hip.check(st, "attention_train")
         out = _linear(y.view(b * T, d), W_out, OUT_GEMM_MAX_ROWS)
-        ctx.save_for_backward(x, W_out, cos, sin, proj, y, kv, lse, W_cat)
+        ctx.save_for_backward(x, W_q, W_k, W_v, W_out, cos, sin, proj, y, kv, lse, W_cat)
         ctx.sizes = (num_heads, window)
         return out.view(b, T, d)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, dout):
-        x, W_out, cos, sin, proj, y, kv, lse, W_cat = ctx.saved_tensors
+        x, W_q, W_k, W_v, W_out, cos, sin, proj, y, kv, lse, W_cat = ctx.saved_tensors
         H, window = ctx.sizes
         need = ctx.needs_input_grad
+        if torch.is_grad_enabled():                                            # create_graph: gradients of these are wanted
+            g = _attention_grads((x, W_q, W_k, W_v, W_out), need, dout, cos, sin, H, window)
+            return (*g, None, None, None, None)
         b, T, d = x.shape
         hd = d // H
         x2, do2 = _rows16(x.reshape(b * T, d), 8), _rows16(dout.reshape(b * T, d), 8)
@@ -339,8 +357,8 @@ class _AttentionTrain(torch.autograd.Function):
 
 
 def attention_train(attn, x):
-    """A WindowAttention's output (b, T, d), differentiable (once) in x and the four projections (reference
-    dispatcher_hybrid/modeling_dispatcher.py:168-182): scores and probabilities stay in registers in both directions
+    """A WindowAttention's output (b, T, d), differentiable in x and the four projections (reference
+    dispatcher_hybrid/modeling_dispatcher.py:168-182; under create_graph through torch operations): scores and probabilities stay in registers in both directions
     (``dh_window_attention_train_fwd`` / ``dh_window_attention_bwd``; the softmax's log-sum is kept in fp32), one product for
     q, k, v and one launch for the four weight gradients. See attention_fits."""
     T = x.shape[1]

@@ -6,7 +6,7 @@
 //   delta[t] = sum_c dO[t,c] O[t,c]
 //   dV[s] = sum_t P[t,s] dO[t]      dS[t,s] = P[t,s] (dO[t] . V[s] - delta[t])
 //   dQ'[t] = sum_s dS[t,s] K'[s] / sqrt(hd)      dK'[s] = sum_t dS[t,s] Q'[t] / sqrt(hd)      (primes: rotated)
-// and dQ, dK rotated back. Three launches: a pre-pass (rotated queries head-major, delta), then one kernel in two forms.
+// and dQ, dK rotated back. Two launches: a pre-pass (rotated queries head-major, delta), then one kernel in two forms.
 //
 // Work decomposition: a workgroup of 4 waves owns 64 rows of one (batch row, head) -- queries for dQ, keys for dK and dV --
 // and walks the 64-row blocks of the other side inside the band; wave w owns rows 16 w .. + 15, their two operand fragments
@@ -16,7 +16,7 @@
 // transposed, are read with ds_read_tr16_b64 from the same LDS tiles. So nothing is transposed in registers and no value
 // crosses a wave.
 // Bound: VALU (~9 instructions per score and form) beside 3 (dQ) and 4 (dK, dV) MFMA products. Measured on MI355X at B 2,
-// T 2048, window 1024, 16 heads: dK and dV 61 us, dQ 43, pre-pass 9 (58 GFLOP with the forward's), where the blockwise torch
+// T 2048, window 1024, 16 heads: 90 us and the pre-pass 9 (58 GFLOP with the forward's), where the blockwise torch
 // attention took ~390 launches and 4 ms for the two directions.
 #include "dh_attn_common.h"
 
@@ -78,16 +78,18 @@ __global__ __launch_bounds__(kThreads) void attn_bwd_prep(BwdArgs a) {
   if (c == 0) a.delta[hm] = s;
 }
 
-// KV: dK and dV of 64 keys, else dQ of 64 queries
+struct BwdLds {
+  __align__(16) unsigned char tile[2][2][kB * kRow];                     // [buffer][keys | queries, values | dO]
+  __align__(16) float stat[2][2][kB];                                    // KV: log2-sum-exp and delta of the block's queries
+};
+
+// KV: dK and dV of 64 keys, else dQ of 64 queries; item w = block of 64 rows of one (batch row, head)
 template <bool KV>
-__global__ __launch_bounds__(kThreads, 3) void attn_bwd_kernel(BwdArgs a) {
-  __shared__ __align__(16) unsigned char tile[2][2][kB * kRow];          // [buffer][keys | queries, values | dO]
-  __shared__ __align__(16) float stat[2][2][kB];                         // KV: log2-sum-exp and delta of the block's queries
+__device__ __forceinline__ void attn_bwd_rows(const BwdArgs& a, BwdLds& lds, int w) {
+  auto& tile = lds.tile;
+  auto& stat = lds.stat;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int per = (a.nwork + 7) >> 3;                                    // consecutive items (blocks of one head) on one XCD
-  const int w = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if (w >= a.nwork) return;
   const int blk = w % a.nblk, bh = w / a.nblk, h = bh % a.H, b = bh / a.H;
   const int own0 = blk * kB;
   const int town = own0 + wave * 16 + r;                                 // this lane's row
@@ -236,6 +238,21 @@ __global__ __launch_bounds__(kThreads, 3) void attn_bwd_kernel(BwdArgs a) {
   }
 }
 
+// Both forms in one launch, the key blocks (more products each) first: two launches end in a round of their own each, and a
+// short sequence fills the CUs with neither (B 2, T 2048, window 1024, 16 heads: 59 + 41 us -> 90).
+__global__ __launch_bounds__(kThreads, 3) void attn_bwd_kernel(BwdArgs a) {
+  __shared__ BwdLds lds;
+  const int per = (a.nwork + 7) >> 3;                                    // consecutive items (blocks of one head) on one XCD
+  const int i = blockIdx.x >> 3;
+  const bool kv = i < per;
+  const int w = (blockIdx.x & 7) * per + (kv ? i : i - per);
+  if (w >= a.nwork) return;
+  if (kv)
+    attn_bwd_rows<true>(a, lds, w);
+  else
+    attn_bwd_rows<false>(a, lds, w);
+}
+
 bool aligned(const void* p, uintptr_t n) { return ((uintptr_t)p % n) == 0; }
 
 }  // namespace
@@ -271,7 +288,6 @@ extern "C" int dh_window_attention_bwd(int dtype, const void* q, int64_t stride_
   hipStream_t s = (hipStream_t)stream;
   const unsigned grid = (unsigned)((nwork + 7) / 8 * 8);
   attn_bwd_prep<<<dim3((unsigned)((chunks + kThreads - 1) / kThreads)), kThreads, 0, s>>>(a);
-  attn_bwd_kernel<true><<<dim3(grid), kThreads, 0, s>>>(a);
-  attn_bwd_kernel<false><<<dim3(grid), kThreads, 0, s>>>(a);
+  attn_bwd_kernel<<<dim3(2 * grid), kThreads, 0, s>>>(a);
   return dh_check_launch(who);
 }

@@ -11,7 +11,9 @@ DEV = "cuda"
 @pytest.mark.parametrize("M,shapes", [
     (1, [(8, 8)]), (63, [(64, 64), (136, 72)]), (64, [(128, 128)]), (65, [(120, 264)]), (511, [(1024, 64)]),
     (1024, [(128, 128), (256, 64), (8, 1000), (512, 136)]),        # split rows, four layers, ragged tiles
-    (3001, [(1024, 1024)] * 4), (5000, [(64, 64)])])
+    (3001, [(1024, 1024)] * 4), (5000, [(64, 64)]),
+    (6143, [(136, 256)]), (6144, [(136, 256), (8, 512)]), (6145, [(1024, 256)]),
+    (8001, [(256, 1024)] * 4), (6200, [(64, 264)])])
 def test_weight_grads_against_float64(M, shapes):
     from dispatcher_hybrid.fused_train import weight_grads
     g = torch.Generator(device=DEV).manual_seed(M)

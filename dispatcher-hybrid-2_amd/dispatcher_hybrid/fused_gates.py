@@ -398,26 +398,30 @@ def input_projections(x, mixer):
     return tuple(l(x) for l in lins)
 
 
-# Rows up to which one dh_proj_gemm launch beats the library, measured on MI355X in captured graphs
-# (bf16; us, ours against the library): an attention layer's q, k, v (three 1024-wide nn.Linear
-# GEMMs, K = 1024) 13.3 / 23.8 at 1024 rows, 19.6 / 29.7 at 2048, 30.0 / 37.4 at 4096, 60 / 59 at
-# 8192; over 18 distinct weights per graph, as in the forward, a single 1024 x 1024 output
-# projection (the mixer's and attention's linear_out) 6.7 / 8.9 at 1024, 9.1 / 10.4 at 2048,
-# 12.9 / 13.0 at 4096, and the SwiGLU down projection (1024 x 2816) 12.1 / 14.0 at 1024, 19.8 / 18.8
-# at 2048 (the launches of at most 512 tiles keep two or three K tiles in flight).
+# Rows up to which one dh_proj_gemm launch beats the library, measured on MI355X in captured graphs over 18 distinct weights,
+# as in the forward (bf16; us, ours against the library): an attention layer's q, k, v (three 1024-wide nn.Linear GEMMs,
+# K = 1024) 21.4 / 32.5 at 2048 rows, 30.2 / 40.0 at 4096, 33.6 / 46.7 at 5120, 44.9 / 51.7 at 6002, 58.2 / 62.9 at 8192; a
+# single 1024 x 1024 output projection (the mixer's and attention's linear_out) 6.7 / 8.9 at 1024, 9.3 / 10.7 at 2048,
+# 11.4 / 11.5 at 3000, 13.1 / 14.1 at 4096, 15.9 / 14.8 at 4608; the SwiGLU down projection (1024 x 2816) 12.1 / 14.0 at
+# 1024, 20.4 / 19.7 at 2048, 25.5 / 22.9 at 3000.
 # fp32: the 1024 x 1024 output projection 23.9 / 36.7 / 57.6 / 75.6 us at 1024 / 2048 / 3002 / 4096 rows against 20.6 / 36.7
 # / 68.2 / 63.8 for the library.
-QKV_GEMM_MAX_ROWS = 4096
-OUT_GEMM_MAX_ROWS = 2048
+QKV_GEMM_MAX_ROWS = 8192
+OUT_GEMM_MAX_ROWS = 4096
 OUT_GEMM_MAX_ROWS_F32 = 3072
 DOWN_GEMM_MAX_ROWS = 1024
 
 
+# (under autocast the library call casts to the autocast dtype and dh_proj_gemm does not: the line between the two stays at
+# half of what the unrestricted bf16 limits are)
 def out_max_rows(dtype):
-    # (under autocast the library call casts to the autocast dtype: the line between the two stays where it was)
-    if dtype == torch.bfloat16 or torch.is_autocast_enabled("cuda"):
-        return OUT_GEMM_MAX_ROWS
-    return OUT_GEMM_MAX_ROWS_F32
+    if torch.is_autocast_enabled("cuda"):
+        return OUT_GEMM_MAX_ROWS // 2
+    return OUT_GEMM_MAX_ROWS if dtype == torch.bfloat16 else OUT_GEMM_MAX_ROWS_F32
+
+
+def qkv_max_rows():
+    return QKV_GEMM_MAX_ROWS // 2 if torch.is_autocast_enabled("cuda") else QKV_GEMM_MAX_ROWS
 
 
 def project(x, linears, max_rows):

@@ -269,13 +269,13 @@ class WindowAttention(nn.Module):
         if self.use_fused and not torch.is_grad_enabled() and x.is_cuda:
             from . import fused_attention as fa
             if fa.supported(x.dtype, self.head_dim):
-                from .fused_gates import OUT_GEMM_MAX_ROWS, QKV_GEMM_MAX_ROWS, project
-                # q, k, v as one GEMM launch (up to QKV_GEMM_MAX_ROWS rows); RoPE, banded scores,
+                from .fused_gates import out_max_rows, project, qkv_max_rows
+                # q, k, v as one GEMM launch (up to qkv_max_rows rows); RoPE, banded scores,
                 # softmax and the value average in one launch, (B, T, d) in/out
-                q, k, v = project(x, [self.linear_q, self.linear_k, self.linear_v], QKV_GEMM_MAX_ROWS)
+                q, k, v = project(x, [self.linear_q, self.linear_k, self.linear_v], qkv_max_rows())
                 cos, sin = self.rope_tables(T, x.device, x.dtype)
                 y = fa.window_attention(q, k, v, cos, sin, self.num_heads, self.band(T))
-                return project(y, [self.linear_out], OUT_GEMM_MAX_ROWS)[0]
+                return project(y, [self.linear_out], out_max_rows(y.dtype))[0]
         elif self.use_fused and x.is_cuda and torch.is_grad_enabled() and (
                 x.requires_grad or any(p.requires_grad for p in self.parameters())):
             from . import fused_train as ft

@@ -15,8 +15,8 @@
 //   gate_bwd_w       dW and db: contractions over positions, split over row ranges
 //   gate_bwd_reduce  the ranges' partial sums, added in order and rounded once to the gradients' dtype
 //
-// Measured on MI355X (16 heads, 12 levels, GH 1024; us): bf16 b 4, T 4096: pack 30 + ab 166 + w 93 + reduce 6, where the
-// atomic kernel of dh_gate_preacts_bwd takes 8361; b 4, T 1024: 15 + 48 + 29 + 5 against 5115; fp32 b 1, T 777: 105
+// Measured on MI355X (16 heads, 12 levels, GH 1024; us): bf16 b 4, T 4096: pack 15 + ab 166 + w 93 + reduce 6, where the
+// atomic kernel of dh_gate_preacts_bwd takes 8361; b 4, T 1024: 8 + 44 + 28 + 6 against 5115; fp32 b 1, T 777: 105
 // against 3944.
 #include "dh_common.h"
 
@@ -83,6 +83,7 @@ struct PackArgs {
   void* p1;
   uint4* p2;
   uint32_t* ok;
+  bool wide;                    // dP rows contiguous along t, starting on 16-byte boundaries
   Dims d;
 };
 
@@ -95,42 +96,79 @@ __global__ __launch_bounds__(256) void gate_bwd_pack(PackArgs a) {
   T* tile = (T*)raw;                                         // [3 H][RS]
   const Dims& d = a.d;
   const int b = blockIdx.z, l = blockIdx.y, t0 = blockIdx.x * kPackRows, tid = threadIdx.x;
-  const int n = 3 * d.H * kPackRows;
-  for (int e = tid; e < n; e += 256) {
-    // consecutive threads follow the layout's unit stride: along t (head-major) or along h
-    int x, h, i;
-    if (a.st == 1) {
-      i = e & (kPackRows - 1);
-      const int q = e / kPackRows;
-      x = q / d.H;
-      h = q - x * d.H;
-    } else {
-      const int q = e / d.H;
-      h = e - q * d.H;
-      x = q / kPackRows;
-      i = q & (kPackRows - 1);
-    }
-    const T* p = (const T*)(x == 0 ? a.dP[0] : x == 1 ? a.dP[1] : a.dP[2]);
-    T v = 0;
-    if (t0 + i < d.T) v = p[(int64_t)b * a.sb + (int64_t)(t0 + i) * a.st + (int64_t)l * a.sl + (int64_t)h * a.sh];
-    tile[(x * d.H + h) * RS + i] = v;
-  }
-  if (l == 0 && tid < kPackRows && t0 + tid < d.T) {
-    // bit j: level j reaches t from t - 2^j (low half); level j carries t to t + 2^j (high half)
-    const int t = t0 + tid;
+  __shared__ uint32_t part[4][kPackRows];
+  if (l == 0) {
+    // bit j: level j reaches t from t - 2^j (low half); level j carries t to t + 2^j (high half). A thread takes every
+    // fourth level of a position and has its 8 mask values in flight together
+    const int i = tid & (kPackRows - 1), t = t0 + i, q = tid / kPackRows;
     uint32_t bits = 0;
-    for (int j = 0; j < d.n_lv; ++j) {
-      const int lag = 1 << j;
-      auto on = [&](int tt) {
-        return a.mask == nullptr ||
-               Elem<T>::load((const T*)a.mask + (int64_t)b * a.smb + (int64_t)tt * a.smt + (int64_t)j * a.sml) > 0.f;
+    float in[4], out[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = min(q + 4 * u, d.n_lv - 1);
+      auto at = [&](int tt) {
+        return a.mask == nullptr ? 1.f
+                                 : Elem<T>::load((const T*)a.mask + (int64_t)b * a.smb + (int64_t)min(tt, d.T - 1) * a.smt +
+                                                 (int64_t)j * a.sml);
       };
-      if (t >= lag && on(t)) bits |= 1u << j;
-      if (t + lag < d.T && on(t + lag)) bits |= 1u << (16 + j);
+      in[u] = at(t);
+      out[u] = at(t + (1 << j));
     }
-    a.ok[(int64_t)b * d.T + t] = bits;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = q + 4 * u;
+      if (j >= d.n_lv) continue;
+      if (t >= (1 << j) && in[u] > 0.f) bits |= 1u << j;
+      if (t + (1 << j) < d.T && out[u] > 0.f) bits |= 1u << (16 + j);
+    }
+    part[q][i] = bits;
+  }
+  if (a.wide) {
+    // rows contiguous along t and 16-byte aligned: a 16-byte piece per thread (with the mask loads above in flight together,
+    // b 4, T 4096: 26 us with single elements -> 15)
+    constexpr int V = 16 / (int)sizeof(T), CPR = kPackRows / V;
+    for (int e = tid; e < 3 * d.H * CPR; e += 256) {
+      const int row = e / CPR, i = (e % CPR) * V, t = t0 + i;            // row = x H + h
+      const int x = row < d.H ? 0 : row < 2 * d.H ? 1 : 2, h = row - x * d.H;
+      const T* p = (const T*)(x == 0 ? a.dP[0] : x == 1 ? a.dP[1] : a.dP[2]) + (int64_t)b * a.sb + (int64_t)l * a.sl +
+                   (int64_t)h * a.sh + t;
+      T v[V];
+      if (t + V <= d.T) {
+        const uint4 u = *reinterpret_cast<const uint4*>(p);
+        __builtin_memcpy(v, &u, 16);
+      } else {
+#pragma unroll
+        for (int k = 0; k < V; ++k) v[k] = t + k < d.T ? p[k] : (T)0;
+      }
+      uint4 u;
+      __builtin_memcpy(&u, v, 16);
+      *reinterpret_cast<uint4*>(&tile[row * RS + i]) = u;
+    }
+  } else {
+    const int n = 3 * d.H * kPackRows;
+    for (int e = tid; e < n; e += 256) {
+      // consecutive threads follow the layout's unit stride: along t (head-major) or along h
+      int x, h, i;
+      if (a.st == 1) {
+        i = e & (kPackRows - 1);
+        const int q = e / kPackRows;
+        x = q / d.H;
+        h = q - x * d.H;
+      } else {
+        const int q = e / d.H;
+        h = e - q * d.H;
+        x = q / kPackRows;
+        i = q & (kPackRows - 1);
+      }
+      const T* p = (const T*)(x == 0 ? a.dP[0] : x == 1 ? a.dP[1] : a.dP[2]);
+      T v = 0;
+      if (t0 + i < d.T) v = p[(int64_t)b * a.sb + (int64_t)(t0 + i) * a.st + (int64_t)l * a.sl + (int64_t)h * a.sh];
+      tile[(x * d.H + h) * RS + i] = v;
+    }
   }
   __syncthreads();
+  if (l == 0 && tid < kPackRows && t0 + tid < d.T)
+    a.ok[(int64_t)b * d.T + t0 + tid] = part[0][tid] | part[1][tid] | part[2][tid] | part[3][tid];
   for (int nt = 0; nt < d.NT; ++nt) {
     const int64_t pair = (int64_t)b * d.NP + l * d.NT + nt;
     {
@@ -766,8 +804,10 @@ extern "C" int dh_gate_preacts_bwd_ws(int dtype, const void* A, const void* B, i
   unsigned char* ws = (unsigned char*)workspace;
   const int nsplit = splits_of(d);
   const int64_t blocks = (int64_t)d.b * d.NBK;
+  const bool wide = stride_pt == 1 && aligned(dPi, 16) && aligned(dPf, 16) && aligned(dPr, 16) &&
+                    stride_pb % vec == 0 && stride_pl % vec == 0 && stride_ph % vec == 0;
   PackArgs pa{{dPi, dPf, dPr}, stride_pb, stride_pt, stride_pl, stride_ph, mask, stride_mb, stride_mt, stride_ml,
-              ws + sp.p1, (uint4*)(ws + sp.p2), (uint32_t*)(ws + sp.ok), d};
+              ws + sp.p1, (uint4*)(ws + sp.p2), (uint32_t*)(ws + sp.ok), wide, d};
   AbArgs aa{A, B, stride_ab, stride_at, {Wi, Wf, Wr}, stride_wl, stride_wh, ws + sp.p1, (const uint32_t*)(ws + sp.ok),
             dA, dB, stride_gb, stride_gt, d};
   WArgs wa{A, B, stride_ab, stride_at, (const uint4*)(ws + sp.p2), (const uint32_t*)(ws + sp.ok), (float*)(ws + sp.part),

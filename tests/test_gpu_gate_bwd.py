@@ -48,6 +48,7 @@ CASES = [  # b, T, GH, H, n_lv, mask, layout
     (3, 64, 128, 16, 7, True, "op"),
     (2, 130, 1024, 16, 8, True, "head"),
     (1, 515, 256, 64, 10, True, "op"),          # 40 (level, head group) pairs: the weights pass through LDS in chunks
+    (1, 5, 64, 2, 3, True, "rows"), (2, 64, 64, 16, 6, True, "rows"), (2, 131, 64, 17, 16, True, "rows"),
     (2, 515, 64, 3, 16, False, "head"),          # levels whose lag exceeds the length
 ]
 
@@ -64,6 +65,11 @@ def test_gate_backward_against_float64(b, T, GH, H, n_lv, masked, layout, dtype)
     mask = (torch.rand(b, T, L, device=DEV, generator=g) < 0.8).to(dtype) if masked else None
     if layout == "head":
         dP = [rn(b, H, n_lv, T).to(dtype).permute(0, 3, 2, 1) for _ in range(3)]
+    elif layout == "rows":                                        # head-major rows padded to 8, the padding not a number
+        dP = [torch.full((b, H, n_lv, -(-T // 8) * 8), float("nan"), device=DEV, dtype=dtype) for _ in range(3)]
+        for p in dP:
+            p[..., :T] = rn(b, H, n_lv, T).to(dtype)
+        dP = [p[..., :T].permute(0, 3, 2, 1) for p in dP]
     elif layout == "expanded":                                    # one value for all positions: stride 0 along t
         dP = [rn(b, 1, n_lv, H).to(dtype).expand(b, T, n_lv, H) for _ in range(3)]
     else:

@@ -17,15 +17,16 @@
 // (each block of 64 keys is 64 contiguous rows of one head).
 //
 // Work decomposition: a workgroup of 4 waves owns 64 queries of one (batch row, head); wave w owns
-// queries q0 + 16w .. +15. The key blocks of the band (64 keys each) are staged in LDS -- keys
-// row-major with rows padded to hd*2 + 16 bytes; values transposed (hd rows of 64 keys, padded to
-// 136 bytes) -- double-buffered, the next block's global loads in flight during the current
-// block. Scores are computed transposed, S^T = K Q^T (v_mfma_f32_16x16x32_bf16, A = key
-// rows from LDS, B = the wave's rotated query fragments held in registers), so the C fragment puts
-// one query per lane column: the running max, sum and rescale stay per lane (plus two cross-group
-// shuffles per reduction), and the probabilities are already in the B-operand layout of
-// O^T = V^T P^T, whose A operand reads the transposed values from LDS. Workgroups are numbered so
-// consecutive query blocks of one (batch row, head) run on one XCD (round-robin dispatch: block id
+// queries q0 + 16w .. +15. The key blocks of the band (64 keys each) are staged row-major in padded LDS rows, keys and values
+// alike, double-buffered, the next block's global loads in flight during the current block. Scores are computed transposed,
+// S^T = K Q^T (v_mfma_f32_16x16x32_bf16, A = key rows from LDS, B = the wave's rotated query fragments held in registers),
+// so the C fragment puts one query per lane column: the running max (exchanged between the four lanes of a query by
+// permlane swaps), this lane's part of the sum and the rescale stay in registers, and the probabilities are already in
+// the B-operand layout of O^T = V^T P^T, whose A operand is read transposed from the value rows (ds_read_tr16_b64).
+// Bound: VALU (the 16 exponentials a block and lane cost as much as its 16 MFMA products). Measured on MI355X at B 2, T 3001,
+// window 1024, 16 heads of 64: 59 us; with the values transposed through 4-byte LDS writes, LDS shuffles for both
+// reductions and a rescale per block 66 us.
+// Workgroups are numbered so consecutive query blocks of one (batch row, head) run on one XCD (round-robin dispatch: block id
 // mod 8), sharing the band's key and value lines in that XCD's L2.
 #include "dh_attn_common.h"
 
@@ -34,6 +35,10 @@ namespace {
 constexpr int kBQ = 64;          // queries per workgroup
 constexpr int kBK = 64;          // keys per block
 constexpr int kThreads = 256;
+
+typedef short v4i16 __attribute__((ext_vector_type(4)));
+typedef short v8i16 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) v4i16* lds4;
 
 struct WinArgs {
   const bf16_t* q;
@@ -74,20 +79,31 @@ __global__ __launch_bounds__(kThreads) void rope_kv_kernel(WinArgs a) {
   *reinterpret_cast<uint4*>(a.vc + dst) = ld16(a.v + src);
 }
 
+// over the four 16-lane groups that share a query (lanes r, r + 16, r + 32, r + 48), in all of them; no LDS round trip
+__device__ __forceinline__ float across_groups_max(float x) {
+  const auto u = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(u[0]), __uint_as_float(u[1]));
+  const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(v[0]), __uint_as_float(v[1]));
+}
+__device__ __forceinline__ float across_groups_sum(float x) {
+  const auto u = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(u[0]) + __uint_as_float(u[1]);
+  const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(v[0]) + __uint_as_float(v[1]);
+}
+
 template <int HD>
 __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
   constexpr int KROW = HD * 2 + 16;              // padded key row (bytes)
-  constexpr int VROW = kBK * 2 + 8;              // padded transposed-value row (bytes)
+  constexpr int VROW = HD * 2 + (HD == 64 ? 16 : 32);   // padded value row: four rows start 8 banks or more apart
   constexpr int KS = HD / 32;                    // MFMA k-steps over hd
   constexpr int NT = HD / 16;                    // hd tiles of the output
   constexpr int CPR = HD / 8;                    // 16-byte chunks per row
   constexpr int LPT = kBK * CPR / kThreads;      // key (and value) chunks per thread per block
   static_assert(LPT >= 1 && kBK * CPR % kThreads == 0, "block shape");
-  // with two or more chunks a thread takes pairs of consecutive keys at one column, so the
-  // transposed values are written as 4-byte (key, key + 1) words
-  constexpr bool PAIRS = LPT % 2 == 0;
   __shared__ __align__(16) unsigned char ks[2][kBK * KROW];
-  __shared__ __align__(16) unsigned char vt[2][HD * VROW];
+  __shared__ __align__(16) unsigned char vs[2][kBK * VROW];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
@@ -103,55 +119,23 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
   const bf16_t* kp = a.kc + (int64_t)b * a.cb + (int64_t)h * a.ch;    // rotated keys, rows of hd
   const bf16_t* vp = a.vc + (int64_t)b * a.cb + (int64_t)h * a.ch;
 
-  // ---- K/V block staging. Chunk i of the thread -> (key, 16-byte column): without pairs chunk
-  // index tid + 256 i -> key idx / CPR, column idx % CPR; with pairs, pair tid + 256 (i / 2) ->
-  // keys 2 (idx / CPR) + (i & 1), column idx % CPR
-  auto chunk_of = [&](int i, int& key, int& c) {
-    if constexpr (PAIRS) {
-      const int idx = tid + (i >> 1) * kThreads;
-      key = 2 * (idx / CPR) + (i & 1);
-      c = idx % CPR;
-    } else {
-      const int idx = tid + i * kThreads;
-      key = idx / CPR;
-      c = idx % CPR;
-    }
-  };
+  // ---- K/V block staging: chunk index tid + 256 i -> key idx / CPR, 16-byte column idx % CPR
   uint4 kraw[LPT], vraw[LPT];
   auto kv_fetch = [&](int kb) {
 #pragma unroll
     for (int i = 0; i < LPT; ++i) {
-      int key, c;
-      chunk_of(i, key, c);
+      const int idx = tid + i * kThreads, key = idx / CPR, c = idx % CPR;
       const int t = min(kb * kBK + key, a.T - 1);
       kraw[i] = ld16(kp + (int64_t)t * HD + 8 * c);
       vraw[i] = ld16(vp + (int64_t)t * HD + 8 * c);
     }
   };
-  auto kv_store = [&](int buf, int kb) {
-    (void)kb;
+  auto kv_store = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < LPT; ++i) {
-      int key, c;
-      chunk_of(i, key, c);
+      const int idx = tid + i * kThreads, key = idx / CPR, c = idx % CPR;
       *reinterpret_cast<uint4*>(&ks[buf][key * KROW + c * 16]) = kraw[i];
-      const uint32_t vw[4] = {vraw[i].x, vraw[i].y, vraw[i].z, vraw[i].w};
-      if constexpr (PAIRS) {
-        if (i & 1) {                               // chunk i - 1 holds key - 1 at the same column
-          const uint32_t uw[4] = {vraw[i - 1].x, vraw[i - 1].y, vraw[i - 1].z, vraw[i - 1].w};
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const uint32_t lo = (e & 1) ? (uw[e >> 1] >> 16) : (uw[e >> 1] & 0xffffu);
-            const uint32_t hi = (e & 1) ? (vw[e >> 1] & 0xffff0000u) : (vw[e >> 1] << 16);
-            *reinterpret_cast<uint32_t*>(&vt[buf][(8 * c + e) * VROW + (key - 1) * 2]) = lo | hi;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          *reinterpret_cast<bf16_t*>(&vt[buf][(8 * c + e) * VROW + key * 2]) =
-              (bf16_t)((e & 1) ? (vw[e >> 1] >> 16) : (vw[e >> 1] & 0xffffu));
-      }
+      *reinterpret_cast<uint4*>(&vs[buf][key * VROW + c * 16]) = vraw[i];
     }
   };
 
@@ -173,10 +157,10 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
   f32x4 o[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) o[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -1e30f, l = 0.f;                      // running max (finite floor) and sum of this query
+  float m = -1e30f, l = 0.f;                      // running max (finite floor); this lane's part of the running sum
 
   kv_fetch(kb_lo);
-  kv_store(0, kb_lo);
+  kv_store(0);
   __syncthreads();
   for (int kb = kb_lo; kb <= kb_hi; ++kb) {
     const int buf = (kb - kb_lo) & 1;
@@ -194,48 +178,42 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
         sT[tau] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[s], sT[tau], 0, 0, 0);
       }
     }
-    // scores in the log2 domain (scale * log2 e folded in; softmax via 2^x). A block strictly below
+    // softmax via 2^x: scale * log2 e is folded into the exponent's multiply-add. A block strictly below
     // the diagonal and wholly inside every query's window needs no mask (all blocks but the band's
     // first and last): a uniform branch.
     const bool interior = kb < qb && (a.window == 0 || q0 + kBQ - 1 - kb * kBK < a.window);
     float p[16];
     float mx = -INFINITY;
-    if (interior) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) p[j] = sT[j >> 2][j & 3];
+    if (!interior) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        p[j] = sT[j >> 2][j & 3] * a.scale2;
-        mx = fmaxf(mx, p[j]);
+        const int key = kb * kBK + (j >> 2) * 16 + 4 * g + (j & 3);
+        const bool ok = key <= tq && key < a.T && (a.window == 0 || tq - key < a.window);
+        p[j] = ok ? p[j] : -INFINITY;
       }
-    } else {
-#pragma unroll
-      for (int tau = 0; tau < 4; ++tau)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = kb * kBK + tau * 16 + 4 * g + i;
-          const bool ok = key <= tq && key < a.T && (a.window == 0 || tq - key < a.window);
-          const float sc = sT[tau][i] * a.scale2;
-          p[tau * 4 + i] = ok ? sc : -INFINITY;
-          mx = fmaxf(mx, p[tau * 4 + i]);
-        }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16));
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float mn = fmaxf(m, mx);
-    const float alpha = __builtin_amdgcn_exp2f(m - mn);
-    m = mn;
-    float ps = 0.f;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) mx = fmaxf(mx, p[j]);
+    mx = across_groups_max(mx) * a.scale2;        // scale2 > 0
+    // the running max moves only when it falls 2^8 behind (the weights stay below 2^8, exact in fp32 and bf16 alike), so
+    // the output is rarely rescaled
+    if (__builtin_amdgcn_ballot_w64(mx > m + 8.f)) {
+      const float mn = fmaxf(m, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[nt][i] *= alpha;
+    }
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-      p[j] = __builtin_amdgcn_exp2f(p[j] - mn);   // masked: 2^-inf = 0
-      ps += p[j];
+      p[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[j], a.scale2, -m));   // masked: 2^-inf = 0
+      l += p[j];
     }
-    ps += __shfl_xor(ps, 16);
-    ps += __shfl_xor(ps, 32);
-    l = l * alpha + ps;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[nt][i] *= alpha;
 
     // ---- O^T += V^T P^T over the two 32-key steps; key order within a step: the lane group's
     // four keys of tile 2kk, then its four keys of tile 2kk + 1 (the same order on both operands)
@@ -248,18 +226,19 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
       const bf16x8 pf = as_bf16x8(pw);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        const unsigned char* vrow = &vt[buf][(nt * 16 + r) * VROW];
-        const uint2 v0 = *reinterpret_cast<const uint2*>(vrow + (32 * kk + 4 * g) * 2);
-        const uint2 v1 = *reinterpret_cast<const uint2*>(vrow + (32 * kk + 16 + 4 * g) * 2);
-        o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(make_uint4(v0.x, v0.y, v1.x, v1.y)), pf,
-                                                        o[nt], 0, 0, 0);
+        const unsigned char* src = &vs[buf][(32 * kk + 4 * g + (r >> 2)) * VROW + nt * 32 + (r & 3) * 8];
+        const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(src));
+        const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(src + 16 * VROW));
+        const v8i16 vf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        o[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vf), pf, o[nt], 0, 0, 0);
       }
     }
-    if (more) kv_store(buf ^ 1, kb + 1);
+    if (more) kv_store(buf ^ 1);
     __syncthreads();
   }
 
   // ---- output: lane holds query tq, hd columns 16 nt + 4 g + i
+  l = across_groups_sum(l);
   if (tq < a.T) {
     const float inv = 1.f / l;
     if (a.lse != nullptr && g == 0) a.lse[((int64_t)b * a.H + h) * a.T + tq] = m + __builtin_amdgcn_logf(l);

@@ -8,7 +8,7 @@
 // rounded (so the cache rows below are the eager prefill's bit for bit); scores stay fp32 (the
 // eager path rounds them to bf16 first: the kernel is the more accurate of the two), softmax in
 // fp32, probabilities rounded to bf16 for the value product, output rounded once. The softmax is
-// evaluated online over key blocks (running max and sum, the output rescaled per block), so it
+// evaluated online over key blocks (running max and sum, the output rescaled when the max moves), so it
 // normalises at the end where the eager path normalises first: outputs agree to bf16 rounding,
 // not bit for bit.
 // Two launches: a pre-pass writes rope(k) and v of every position to (B, H, Tmax, hd) buffers --

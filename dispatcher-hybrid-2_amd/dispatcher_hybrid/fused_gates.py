@@ -368,10 +368,9 @@ def fused_projections(x, weights):
 
 
 def projections_fit(x, linears):
-    """True when dh_proj_gemm takes x . W^T for these bias-free nn.Linear layers: CUDA input, weights
-    of x's dtype, K a multiple of 64 (bf16) / 32 (fp32), output widths multiples of 4."""
-    return (x.is_cuda and len(linears) <= 3 and all(l.bias is None for l in linears)
-            and all(l.weight.dtype == x.dtype and l.weight.is_contiguous() for l in linears)
+    """True when dh_proj_gemm gives what calling these layers gives: plain bias-free nn.Linear layers (plain_linear), CUDA
+    input, weights of x's dtype, K a multiple of 64 (bf16) / 32 (fp32), output widths multiples of 4."""
+    return (x.is_cuda and len(linears) <= 3 and all(plain_linear(l, x.dtype, x.shape[-1]) for l in linears)
             and x.shape[-1] % (64 if x.dtype == torch.bfloat16 else 32) == 0
             and all(l.weight.shape[0] % 4 == 0 for l in linears))
 
@@ -425,9 +424,8 @@ def qkv_max_rows():
 
 
 def project(x, linears, max_rows):
-    """[l(x) for l in linears] (bias-free nn.Linear layers over the same input) as one dh_proj_gemm
-    launch when x has at most max_rows rows and the kernel takes the shapes (projections_fit), else
-    the library calls. Inference only."""
+    """[l(x) for l in linears] (layers over the same input) as one dh_proj_gemm launch when x has at most max_rows rows and
+    the kernel takes them (projections_fit), else the layers' own calls. Inference only."""
     rows = x.numel() // max(x.shape[-1], 1)
     if rows <= max_rows and projections_fit(x, linears):
         return fused_projections(x, [l.weight for l in linears])
@@ -493,15 +491,11 @@ def mixer_layer(mixer, x, mask, n_lv):
 
 
 def swiglu_fits(x, gate, up):
-    """True when dh_proj_gemm_swiglu takes silu(gate(x)) * up(x) for these bias-free nn.Linear
-    layers: a bf16 CUDA input with 16-byte aligned rows, bf16 contiguous weights of one shape, K a
-    multiple of 64 and N of 8."""
+    """True when dh_proj_gemm_swiglu gives silu(gate(x)) * up(x) for these layers: plain bias-free nn.Linear layers
+    (plain_linear), a bf16 CUDA input, bf16 weights of one shape, K a multiple of 64 and N of 8."""
     K = x.shape[-1]
-    return (x.is_cuda and x.dtype == torch.bfloat16 and gate.bias is None and up.bias is None
-            and gate.weight.dtype == up.weight.dtype == torch.bfloat16
-            and gate.weight.shape == up.weight.shape and gate.weight.shape[1] == K
-            and gate.weight.is_contiguous() and up.weight.is_contiguous()
-            and K % 64 == 0 and gate.weight.shape[0] % 8 == 0)
+    return (x.is_cuda and x.dtype == torch.bfloat16 and plain_linear(gate, x.dtype, K) and plain_linear(up, x.dtype, K)
+            and gate.weight.shape == up.weight.shape and K % 64 == 0 and gate.weight.shape[0] % 8 == 0)
 
 
 def fused_swiglu(x, w_gate, w_up):

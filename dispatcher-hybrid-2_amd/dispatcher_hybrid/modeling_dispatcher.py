@@ -320,12 +320,16 @@ class SwiGLU(nn.Module):
     def forward(self, h):
         if (self.use_fused and h.is_cuda and not torch.is_grad_enabled()
                 and h.dtype in (torch.float32, torch.bfloat16)):                   # dh_silu_mul's dtypes
-            from .fused_gates import DOWN_GEMM_MAX_ROWS, fused_swiglu, project, silu_mul, swiglu_fits
+            from .fused_gates import DOWN_GEMM_MAX_ROWS, fused_swiglu, plain_linear, project, silu_mul, swiglu_fits
             if swiglu_fits(h, self.linear_gate, self.linear_up):
                 a = fused_swiglu(h, self.linear_gate.weight, self.linear_up.weight)
             else:
-                g = self.linear_gate(h)
-                a = silu_mul(g, self.linear_up(h), out=g)
+                g, u = self.linear_gate(h), self.linear_up(h)
+                if g.shape == u.shape and g.dtype == u.dtype and g.dtype in (torch.float32, torch.bfloat16):
+                    # (a hook may have kept the gate's output)
+                    a = silu_mul(g, u, out=g if plain_linear(self.linear_gate, h.dtype, h.shape[-1]) else None)
+                else:
+                    a = F.silu(g) * u
             # (bf16: the shapes it was measured on; fp32 stays on the library)
             return project(a, [self.linear_down], DOWN_GEMM_MAX_ROWS if a.dtype == torch.bfloat16 else 0)[0]
         return self.linear_down(F.silu(self.linear_gate(h)) * self.linear_up(h))

@@ -1,0 +1,74 @@
+"""The fused inference layers call a projection that something stands around (a hook, an adapter, a replaced forward) at every
+row count: with one that doubles its result, the layer's output is what the torch path gives. Tolerance (2-norm relative):
+each projection, the layer's inner results and its output are rounded to bf16 (2^-9) on either path, at most ~12 roundings a
+path: 24 of them in quadrature 1e-2; fp32 sums of at most 1024 products and 12 levels 2e-5."""
+
+import pytest
+import torch
+import torch.nn as nn
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+class Doubled(nn.Linear):
+    def forward(self, h):
+        return 2 * super().forward(h)
+
+
+def _around(l, kind):
+    if kind == "hook":
+        l.register_forward_hook(lambda m, i, o: 2 * o)
+    elif kind == "replaced":
+        l.forward = lambda h: 2 * nn.Linear.forward(l, h)
+    else:
+        ad = Doubled(l.in_features, l.out_features, bias=False).to(l.weight)
+        ad.weight = l.weight
+        return ad
+    return l
+
+
+def _layer(cls, dtype, d=256):
+    import dispatcher_hybrid.modeling_dispatcher as md
+    from dispatcher_hybrid import DispatcherConfig
+    torch.manual_seed(11)
+    layer = getattr(md, cls)(DispatcherConfig(d_model=d, num_heads=d // 64, max_len=4096, attn_window=128, num_layers=1,
+                                              vocab_size=64, dim_feedforward=2 * d)).to(DEV, dtype)
+    with torch.no_grad():
+        for n, p in layer.named_parameters():
+            if "bias" not in n:
+                p.normal_(std=0.05)
+    return layer.eval()
+
+
+CASES = [  # layer, projection, dtype, b, T: whole-layer call, one launch, and the ranges where only some products are
+    ("DispatcherMixer", "linear_out", torch.bfloat16, 1, 200), ("DispatcherMixer", "linear_out", torch.bfloat16, 1, 3000),
+    ("DispatcherMixer", "gate_hidden", torch.bfloat16, 2, 3000), ("DispatcherMixer", "linear_out", torch.float32, 2, 1400),
+    ("WindowAttention", "linear_q", torch.bfloat16, 2, 3000), ("WindowAttention", "linear_out", torch.bfloat16, 1, 3000),
+    ("WindowAttention", "linear_v", torch.bfloat16, 1, 100), ("SwiGLU", "linear_gate", torch.bfloat16, 1, 100),
+    ("SwiGLU", "linear_down", torch.bfloat16, 1, 100), ("SwiGLU", "linear_up", torch.float32, 1, 100)]
+
+
+@pytest.mark.parametrize("kind", ["hook", "replaced", "adapter"])
+@pytest.mark.parametrize("cls,proj,dtype,b,T", CASES)
+def test_inference_calls_what_stands_around_a_projection(cls, proj, dtype, b, T, kind):
+    layer = _layer(cls, dtype)
+    setattr(layer, proj, _around(getattr(layer, proj), kind))
+    x = torch.randn(b, T, 256, device=DEV).to(dtype)
+    t = torch.arange(T, device=DEV).unsqueeze(1)
+    args = (x, (t >= (1 << torch.arange(12, device=DEV))).to(dtype)) if cls == "DispatcherMixer" else (x,)
+    with torch.no_grad():
+        want = layer(*args)
+        layer.use_fused_gates = layer.use_fused = True
+        got = layer(*args)
+    assert (got.double() - want.double()).norm() <= (1e-2 if dtype == torch.bfloat16 else 2e-5) * want.double().norm()
+
+
+def test_a_hook_keeps_the_gate_it_was_given():
+    layer = _layer("SwiGLU", torch.bfloat16)
+    kept = []
+    layer.linear_gate.register_forward_hook(lambda m, i, o: kept.append((o, o.clone())) and None)
+    layer.use_fused = True
+    with torch.no_grad():
+        layer(torch.randn(1, 70, 256, device=DEV).bfloat16())
+    assert torch.equal(*kept[0])

@@ -106,9 +106,12 @@ def _(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask):
 # dispatcher::gate_preacts_bwd
 # ---------------------------------------------------------------------------------------------
 def _rows16(t, n):
-    """t with unit-stride rows whose starts are 16-byte aligned (n elements to 16 bytes), copied if it is not."""
-    t = t if t.stride(-1) == 1 and all(s % n == 0 for s in t.stride()[:-1]) else t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+    """t with unit-stride rows whose starts are 16-byte aligned (n elements to 16 bytes) and lie at least a row apart; any
+    other layout (broadcast or overlapping rows, columns of a wider tensor, an odd offset) copied."""
+    w = t.shape[-1]
+    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % n == 0 and s >= w for s in t.stride()[:-1]):
+        return t
+    return t.clone(memory_format=torch.contiguous_format)
 
 
 def _preacts_bwd_launch(A, B, Wi, Wf, Wr, dP, mask, outs, n_lv, levels, what):
@@ -346,9 +349,7 @@ def fused_projections(x, weights):
     weights: up to three (N_s, K) tensors of x's dtype. Inference only (no autograd)."""
     _hip.require_gpu(x, "fused_projections")
     K = x.shape[-1]
-    x2 = x.reshape(-1, K)
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
+    x2 = _rows16(x.reshape(-1, K), 16 // x.element_size())
     M = x2.shape[0]
     n = len(weights)
     for w in weights:
@@ -506,9 +507,7 @@ def fused_swiglu(x, w_gate, w_up):
     (N, K) bf16. Returns (..., N). Inference only (no autograd)."""
     _hip.require_gpu(x, "fused_swiglu")
     K = x.shape[-1]
-    x2 = x.reshape(-1, K)
-    if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
-        x2 = x2.clone(memory_format=torch.contiguous_format)      # a fresh, aligned copy
+    x2 = _rows16(x.reshape(-1, K), 8)
     N = w_gate.shape[0]
     if (x.dtype != torch.bfloat16 or w_gate.dtype != torch.bfloat16 or w_up.dtype != torch.bfloat16
             or w_gate.shape != (N, K) or w_up.shape != (N, K) or not w_gate.is_contiguous()

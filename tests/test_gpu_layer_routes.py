@@ -72,3 +72,44 @@ def test_a_hook_keeps_the_gate_it_was_given():
     with torch.no_grad():
         layer(torch.randn(1, 70, 256, device=DEV).bfloat16())
     assert torch.equal(*kept[0])
+
+
+def _inputs(layer, cls, x):
+    if cls != "DispatcherMixer":
+        return (x,)
+    t = torch.arange(x.shape[1], device=DEV).unsqueeze(1)
+    return x, (t >= (1 << torch.arange(12, device=DEV))).to(x.dtype)
+
+
+@pytest.mark.parametrize("cls,dtype", [("DispatcherMixer", torch.bfloat16), ("DispatcherMixer", torch.float32),
+                                       ("WindowAttention", torch.bfloat16)])
+def test_broadcast_gradients_and_inputs_in_training(cls, dtype):
+    """A gradient or an input whose rows are one row in memory gives what its dense copy gives, bit for bit."""
+    layer = _layer(cls, dtype)
+    layer.use_fused_gates = layer.use_fused = True
+    w = torch.randn(256, device=DEV).to(dtype)
+
+    def grads(x, dy):
+        x = x.detach().requires_grad_()
+        layer.zero_grad()
+        layer(*_inputs(layer, cls, x)).backward(dy)
+        return [x.grad, *[p.grad for p in layer.parameters()]]
+
+    x = torch.randn(2, 70, 256, device=DEV).to(dtype)
+    for dy in (w.expand(2, 70, 256), torch.randn(2, 1, 256, device=DEV).to(dtype).expand(2, 70, 256)):
+        for a, e in zip(grads(x, dy), grads(x, dy.contiguous())):
+            assert torch.equal(a, e)
+    row = w.clone().requires_grad_()
+    y = layer(*_inputs(layer, cls, row.expand(2, 70, 256)))
+    y.sum((0, 1)).square().sum().backward()
+    assert torch.equal(y.detach(), layer(*_inputs(layer, cls, row.detach().expand(2, 70, 256).contiguous())).detach())
+    assert row.grad.isfinite().all()
+
+
+@pytest.mark.parametrize("cls,T", [("DispatcherMixer", 100), ("WindowAttention", 2500), ("SwiGLU", 100)])
+def test_broadcast_inputs_in_inference(cls, T):
+    layer = _layer(cls, torch.bfloat16)
+    layer.use_fused_gates = layer.use_fused = True
+    x = torch.randn(256, device=DEV).bfloat16().expand(2, T, 256)
+    with torch.no_grad():
+        assert torch.equal(layer(*_inputs(layer, cls, x)), layer(*_inputs(layer, cls, x.contiguous())))

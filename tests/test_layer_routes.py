@@ -1,4 +1,5 @@
-"""Which projections the fused inference layers multiply by their weights directly, and which they call, on the CPU."""
+"""What the fused layers hand to the kernels, on the CPU: the projections they multiply by directly and those they call, and
+the layouts of their operands."""
 
 from types import SimpleNamespace
 
@@ -42,3 +43,18 @@ def test_only_plain_projections_are_multiplied_directly(kind):
     assert not fg.projections_fit(x, [make(), NOT_PLAIN[kind](make())])
     assert not fg.swiglu_fits(x, NOT_PLAIN[kind](make()), make())
     assert not fg.swiglu_fits(x, make(), NOT_PLAIN[kind](make()))
+
+
+def test_rows_a_kernel_cannot_read_are_copied():
+    """Row operands of the products and their gradients: unit stride, rows at least a row apart, 16-byte aligned."""
+    from dispatcher_hybrid.fused_gates import _rows16
+    base = torch.arange(40 * 72, dtype=torch.float32).bfloat16().view(40, 72)
+    kept = [base, base[:, :64], base[:, 8:72], base[::2], base.view(5, 8, 72)]
+    copied = [base[0].expand(40, 72), base[:5, None].expand(5, 8, 72)[:, :, :64].reshape(5, 8, 64).transpose(0, 1),
+              base[None, 0].expand(8, 40, 72), base[:, 1:65], base.view(-1)[1:65].view(1, 64), base.t(),
+              base.view(-1)[:8 * 40 + 64].as_strided((41, 64), (8, 1)), base[:1, :66].as_strided((1, 64), (66, 1))]
+    for t in kept:
+        assert _rows16(t, 8).data_ptr() == t.data_ptr()
+    for t in copied:
+        r = _rows16(t, 8)
+        assert torch.equal(r, t) and r.is_contiguous() and r.stride(-2) == t.shape[-1] and r.data_ptr() % 16 == 0

@@ -160,3 +160,11 @@ def require_gpu(t, what):
     if not t.is_cuda:
         raise RuntimeError(f"{what}: tensors must be on the GPU (got device {t.device}); "
                            "the fused paths have no CPU implementation")
+
+
+def same_gpu(what, x, *others):
+    """Raise unless x is on a GPU and the other tensors (None allowed) are on the same one: a kernel gets bare pointers."""
+    require_gpu(x, what)
+    for t in others:
+        if t is not None and t.get_device() != x.get_device():
+            raise RuntimeError(f"{what}: all tensors must be on one device (got {x.device} and {t.device})")

@@ -39,10 +39,15 @@ def _compute_dtype(x):
     return torch.float32 if x.dtype == torch.float32 else torch.bfloat16
 
 
-def _mask_view(mask, cd):
-    """(b, T, n_lv) mask in dtype `cd` and its element strides (any layout; no copy if already cd)."""
+def _mask_view(mask, cd, b, T, n_lv):
+    """(b, T, >= n_lv) mask in dtype `cd` and its element strides (any layout; no copy if already cd). Sizes that neither
+    match nor broadcast raise: the kernels read b x T x n_lv elements by these strides."""
     if mask is None:
         return None, 0, 0, 0
+    if mask.dim() != 3:
+        raise ValueError(f"document mask: (b, T, levels) expected, got {tuple(mask.shape)}")
+    if mask.shape[0] != b or mask.shape[1] != T or mask.shape[2] < n_lv:
+        mask = mask.expand(b, T, n_lv)
     m = mask.to(cd)
     return m, m.stride(0), m.stride(1), m.stride(2)
 
@@ -51,7 +56,8 @@ def _preacts_launch(A_, B_, Wi_, Wf_, Wr_, bi_, bf_, br_, mask, outs, ostrides, 
     b, T, GH = A_.shape
     H = Wi_.shape[1]
     cd = A_.dtype
-    m_, smb, smt, sml = _mask_view(mask, cd)
+    _hip.same_gpu(what, A_, B_, Wi_, Wf_, Wr_, bi_, bf_, br_, mask)
+    m_, smb, smt, sml = _mask_view(mask, cd, b, T, n_lv)
     p = _hip.ptr
     st = _hip.lib.dh_gate_preacts_fwd(
         _hip.dtype_code(cd), p(A_), p(B_), A_.stride(0), A_.stride(1),
@@ -128,7 +134,8 @@ def _preacts_bwd_launch(A, B, Wi, Wf, Wr, dP, mask, outs, n_lv, levels, what):
     Wi_, Wf_, Wr_ = (_rows16(w[:n_lv].contiguous().to(cd), vec) for w in (Wi, Wf, Wr))
     if not (dP[0].stride() == dP[1].stride() == dP[2].stride()):
         dP = [g.contiguous() for g in dP]
-    m_, smb, smt, sml = _mask_view(mask, cd)
+    _hip.same_gpu(what, A_, B_, Wi_, Wf_, Wr_, *dP, mask)
+    m_, smb, smt, sml = _mask_view(mask, cd, b, T, n_lv)
     p = _hip.ptr
     code = _hip.dtype_code(cd)
     nbytes = _hip.lib.dh_gate_preacts_bwd_workspace_bytes(code, b, T, GH, H, n_lv)
@@ -239,7 +246,8 @@ def _scan_launch(pre_i, pre_f, pre_r, mask, V0, out, num_heads, n_lv, activated,
     pi, pf, pr = (g.to(cd) for g in (pre_i, pre_f, pre_r))       # keeps each tensor's layout
     if not (pi.stride() == pf.stride() == pr.stride()):
         pi, pf, pr = pi.contiguous(), pf.contiguous(), pr.contiguous()
-    m_, smb, smt, sml = _mask_view(mask, cd)
+    _hip.same_gpu(what, V0_, pi, pf, pr, mask)
+    m_, smb, smt, sml = _mask_view(mask, cd, b, T, n_lv)
     p = _hip.ptr
     st = _hip.lib.dh_level_scan_fwd(
         _hip.dtype_code(cd), p(pi), p(pf), p(pr), *pi.stride(), p(m_), smb, smt, sml,
@@ -309,7 +317,7 @@ def fused_gate_scan(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, num_heads):
     fused_level_scan(*fused_gate_preacts(...), mask, V0, num_heads, n_lv) up to the bf16 rounding
     of the activated gates, which follows the eager path (reference
     dispatcher_hybrid/modeling_dispatcher.py:86-88, 100-121)."""
-    if type(A) is torch.Tensor and plain_eager():
+    if type(A) is torch.Tensor and A.is_cuda and plain_eager():
         return _gate_scan_body(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
     return torch.ops.dispatcher.gate_scan_fwd(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
 
@@ -355,6 +363,7 @@ def fused_projections(x, weights):
     for w in weights:
         if w.dtype != x.dtype or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
             raise ValueError("fused_projections: weights must be contiguous (N, K) tensors of x's dtype")
+    _hip.same_gpu("fused_projections", x, *weights)
     outs = [torch.empty(*x.shape[:-1], w.shape[0], device=x.device, dtype=x.dtype) for w in weights]
     if M == 0:
         return outs
@@ -371,7 +380,7 @@ def fused_projections(x, weights):
 def projections_fit(x, linears):
     """True when dh_proj_gemm gives what calling these layers gives: plain bias-free nn.Linear layers (plain_linear), CUDA
     input, weights of x's dtype, K a multiple of 64 (bf16) / 32 (fp32), output widths multiples of 4."""
-    return (x.is_cuda and len(linears) <= 3 and all(plain_linear(l, x.dtype, x.shape[-1]) for l in linears)
+    return (x.is_cuda and len(linears) <= 3 and all(plain_linear(l, x.dtype, x.shape[-1], x.device) for l in linears)
             and x.shape[-1] % (64 if x.dtype == torch.bfloat16 else 32) == 0
             and all(l.weight.shape[0] % 4 == 0 for l in linears))
 
@@ -440,53 +449,73 @@ def plain_eager():
                 or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0)
 
 
-def plain_linear(l, dtype, n_in):
-    """A bias-free nn.Linear itself (no subclass, adapter, parametrization, replaced forward or hook that a direct use of its
-    weight would pass by) with a plain contiguous weight of this dtype and input width."""
+def plain_weight(l, dtype, n_in, device=None):
+    """The weight of a bias-free nn.Linear itself (no subclass, adapter, parametrization, replaced forward or hook of its own
+    that a direct use of the weight would pass by) if it is a plain contiguous tensor of this dtype and input width, on this
+    device if one is given; else None."""
     w = l.weight if type(l) is nn.Linear else None
-    return (w is not None and l.bias is None and type(w) in _PLAIN and w.dtype == dtype
-            and w.shape[1] == n_in and w.is_contiguous() and w.data_ptr() % 16 == 0
+    if (w is not None and l.bias is None and type(w) in _PLAIN and w.dtype == dtype
+            and w.shape[1] == n_in and w.is_contiguous() and w.data_ptr() % 16 == 0 and device in (None, w.device)
             and not (l._forward_hooks or l._forward_pre_hooks or l._backward_hooks or l._backward_pre_hooks
-                     or "forward" in l.__dict__ or _has_any_global_hook()))
+                     or "forward" in l.__dict__)):
+        return w
+    return None
+
+
+def plain_linear(l, dtype, n_in, device=None):
+    """Whether x . weight^T is all that calling this layer does (plain_weight, and no hook on every module)."""
+    return plain_weight(l, dtype, n_in, device) is not None and not _has_any_global_hook()
+
+
+def plain_mixer_weights(mixer, dtype, device):
+    """(gate parameters, projection weights in, x, s, out) of a mixer layer whose (d, d) projections are plain (plain_linear)
+    and whose parameters share this dtype and device; else None."""
+    d, gates = mixer.embed_dim, mixer._gate_params()
+    if _has_any_global_hook() or not all(w.dtype == dtype and b.dtype == dtype and w.device == device and b.device == device
+                                         for w, b in gates):
+        return None
+    lins = [plain_weight(l, dtype, d, device)
+            for l in (mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src, mixer.linear_out)]
+    return None if any(w is None or w.shape[0] != d for w in lins) else (gates, lins)
 
 
 _PLAIN = (torch.Tensor, nn.Parameter)
 
 
 def mixer_layer_fits(mixer, x):
-    """Whether mixer_layer takes this layer and input: few enough rows that both products run on dh_proj_gemm, one dtype
-    throughout, plain bias-free projections, plain eager execution."""
+    """The weights mixer_layer takes (plain_mixer_weights) if it takes this layer and input, else None: few enough rows that
+    both products run on dh_proj_gemm, one dtype and device throughout, plain bias-free projections, plain eager execution."""
     if not plain_eager():
-        return False
+        return None
     d, dt = mixer.embed_dim, x.dtype
-    return (x.dim() == 3 and type(x) in _PLAIN and dt in (torch.float32, torch.bfloat16) and x.shape[-1] == d
-            and 0 < x.shape[0] * x.shape[1] <= out_max_rows(dt) and d % 64 == 0
-            and all(w.dtype == dt and b.dtype == dt and w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0
-                    and w.shape[-1] == d for w, b in mixer._gate_params())
-            and all(plain_linear(l, dt, d) and l.weight.shape[0] == d
-                    for l in (mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src, mixer.linear_out)))
+    if not (x.dim() == 3 and type(x) in _PLAIN and dt in (torch.float32, torch.bfloat16) and x.shape[-1] == d
+            and 0 < x.shape[0] * x.shape[1] <= out_max_rows(dt) and d % 64 == 0):
+        return None
+    weights = plain_mixer_weights(mixer, dt, x.device)
+    if weights is None or not all(w.is_contiguous() and b.is_contiguous() and w.data_ptr() % 16 == 0 and w.shape[-1] == d
+                                  for w, b in weights[0]):
+        return None
+    return weights
 
 
-def mixer_layer(mixer, x, mask, n_lv):
+def mixer_layer(mixer, x, mask, n_lv, weights):
     """A DispatcherMixer's output (b, T, d) in one native call (``dh_mixer_fwd``: the launches of fused_projections,
-    fused_gate_scan and the output projection, with their results). `mask`: the (b, T, L) document mask, or None. Inference
-    only; see mixer_layer_fits."""
+    fused_gate_scan and the output projection, with their results). `mask`: the (b, T, L) document mask, or None; `weights`
+    as mixer_layer_fits returns them. Inference only."""
     b, T, d = x.shape
     dt, H = x.dtype, mixer.num_heads
     x2 = _rows16(x.reshape(b * T, d), 8)
-    if mask is not None and mask.shape[0] != b:
-        mask = mask.expand(b, -1, -1)
-    m, smb, smt, sml = _mask_view(mask, dt)
+    _hip.same_gpu("mixer_layer", x2, mask)
+    m, smb, smt, sml = _mask_view(mask, dt, b, T, n_lv)
     code = _hip.dtype_code(dt)
     nbytes = _hip.lib.dh_mixer_fwd_scratch_bytes(code, b, T, d, H, n_lv)
     scratch = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
     y = torch.empty(b, T, d, device=x.device, dtype=dt)
     p = _hip.ptr
-    (Wi, bi), (Wf, bf), (Wr, br) = mixer._gate_params()
+    ((Wi, bi), (Wf, bf), (Wr, br)), (W_in, W_x, W_s, W_out) = weights
     st = _hip.lib.dh_mixer_fwd(
-        code, p(x2), x2.stride(0), p(mixer.linear_in.weight), p(mixer.gate_hidden.weight), p(mixer.gate_hidden_src.weight),
-        p(Wi), p(Wf), p(Wr), p(bi), p(bf), p(br), p(mixer.linear_out.weight), p(m), smb, smt, sml, p(y), p(scratch),
-        scratch.numel(), b, T, d, H, n_lv, _hip.stream_handle(x.device))
+        code, p(x2), x2.stride(0), p(W_in), p(W_x), p(W_s), p(Wi), p(Wf), p(Wr), p(bi), p(bf), p(br), p(W_out), p(m), smb,
+        smt, sml, p(y), p(scratch), scratch.numel(), b, T, d, H, n_lv, _hip.stream_handle(x.device))
     _hip.check(st, "dh_mixer_fwd")
     return y
 
@@ -495,7 +524,8 @@ def swiglu_fits(x, gate, up):
     """True when dh_proj_gemm_swiglu gives silu(gate(x)) * up(x) for these layers: plain bias-free nn.Linear layers
     (plain_linear), a bf16 CUDA input, bf16 weights of one shape, K a multiple of 64 and N of 8."""
     K = x.shape[-1]
-    return (x.is_cuda and x.dtype == torch.bfloat16 and plain_linear(gate, x.dtype, K) and plain_linear(up, x.dtype, K)
+    return (x.is_cuda and x.dtype == torch.bfloat16 and plain_linear(gate, x.dtype, K, x.device)
+            and plain_linear(up, x.dtype, K, x.device)
             and gate.weight.shape == up.weight.shape and K % 64 == 0 and gate.weight.shape[0] % 8 == 0)
 
 
@@ -509,6 +539,7 @@ def fused_swiglu(x, w_gate, w_up):
     K = x.shape[-1]
     x2 = _rows16(x.reshape(-1, K), 8)
     N = w_gate.shape[0]
+    _hip.same_gpu("fused_swiglu", x, w_gate, w_up)
     if (x.dtype != torch.bfloat16 or w_gate.dtype != torch.bfloat16 or w_up.dtype != torch.bfloat16
             or w_gate.shape != (N, K) or w_up.shape != (N, K) or not w_gate.is_contiguous()
             or not w_up.is_contiguous()):

@@ -23,7 +23,8 @@ import torch.nn.functional as F
 
 from . import _hip
 from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch,
-                          _preacts_launch, _rows16, fused_projections, plain_eager, plain_linear)
+                          _preacts_launch, _rows16, fused_projections, plain_eager, plain_linear,
+                          plain_mixer_weights)
 
 SCAN_MAX_LEN = 4096
 SCAN_MAX_LEVELS = 12
@@ -44,7 +45,7 @@ def _gate_rows(b, H, n_lv, T, like):
 
 
 def _scan_mask(mask, b, T, n_lv, cd):
-    """The level (T, L) or document (b, T, L) mask as a (b, T, n_lv) view in dtype cd."""
+    """The level (T, L) or document (b, T, L) mask as a (b, T, n_lv) view in dtype cd (other sizes raise)."""
     return mask[..., :n_lv].to(cd).expand(b, T, n_lv)
 
 
@@ -52,6 +53,7 @@ def _gate_scan_fwd(A, B, W, bias, mask, V0, H, n_lv, what):
     """(V, pre, states) of the gate path; A, B, V0 (b, T, .) with unit-stride, 16-byte aligned rows, A and B alike."""
     b, T, d = V0.shape
     cd, dev = A.dtype, A.device
+    _hip.same_gpu(what, V0, A, B, *W, *bias, mask)
     V = torch.empty(b, T, d, device=dev, dtype=cd)
     pre = _gate_rows(b, H, n_lv, T, A)
     states = torch.empty(n_lv - 1, b, T, d, device=dev, dtype=cd)
@@ -75,6 +77,7 @@ def _gate_scan_bwd(A, B, W, mask, V0, pre, states, dV, dV0, outs, H, n_lv, what)
     with unit-stride, 16-byte aligned rows."""
     b, T, d = V0.shape
     cd = A.dtype
+    _hip.same_gpu(what, V0, A, B, *W, mask, pre, states, dV, dV0, *outs)
     m = _scan_mask(mask, b, T, n_lv, cd)
     dpre = torch.empty_like(pre)
     scratch = torch.empty(b, T, d, device=A.device, dtype=cd)
@@ -203,22 +206,20 @@ def weight_grads(pairs):
 # a whole mixer layer
 # ---------------------------------------------------------------------------------------------
 def mixer_fits(mixer, x, mask, n_lv):
-    """Whether mixer_train takes this layer and input: one dtype (fp32 or bf16) throughout and no autocast, plain bias-free
-    projections, the training scan's limits, and plain eager execution (a compiler gets the layer-by-layer form,
-    whose gate path is one registered operation, and a torch.func transform that operation's refusal)."""
+    """The weights mixer_train takes (plain_mixer_weights) if it takes this layer and input, else None: one dtype (fp32 or
+    bf16) and device throughout and no autocast, plain bias-free projections, the training scan's limits, and plain eager
+    execution (a compiler gets the layer-by-layer form, whose gate path is one registered operation, and a torch.func
+    transform that operation's refusal)."""
     if not plain_eager():
-        return False
+        return None
     d, H, dt = mixer.embed_dim, mixer.num_heads, x.dtype
     if not (x.dim() == 3 and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
             and dt in (torch.float32, torch.bfloat16) and x.shape[-1] == d
             and not torch.is_autocast_enabled("cuda") and d == SCAN_HEAD * H and H <= 64 and x.shape[1] <= SCAN_MAX_LEN
-            and n_lv <= SCAN_MAX_LEVELS and not mask.requires_grad
+            and n_lv <= SCAN_MAX_LEVELS and not mask.requires_grad and mask.device == x.device
             and x.numel() * 3 * x.element_size() < 2 ** 31):                   # 32-bit offsets within the (rows, 3 d) buffers
-        return False
-    if not all(w.dtype == dt and b.dtype == dt for w, b in mixer._gate_params()):
-        return False
-    return all(plain_linear(l, dt, d) and l.weight.shape[0] == d
-               for l in (mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src, mixer.linear_out))
+        return None
+    return plain_mixer_weights(mixer, dt, x.device)
 
 
 class _MixerTrain(torch.autograd.Function):
@@ -260,14 +261,13 @@ class _MixerTrain(torch.autograd.Function):
         return (*[v if n else None for v, n in zip(g, need)], None, None, None)
 
 
-def mixer_train(mixer, x, mask, n_lv):
+def mixer_train(mixer, x, mask, n_lv, weights):
     """A DispatcherMixer's output (b, T, d), differentiable (once) in x and every parameter (reference
     dispatcher_hybrid/modeling_dispatcher.py:63-123): one product for the three input projections, the gate path of
-    gate_scan_train, the output projection; one backward, in which the four weight gradients are one launch. See
-    mixer_fits."""
-    (Wi, bi), (Wf, bf), (Wr, br) = mixer._gate_params()
-    return _MixerTrain.apply(x, mixer.linear_in.weight, mixer.gate_hidden.weight, mixer.gate_hidden_src.weight, Wi, Wf, Wr,
-                             bi, bf, br, mixer.linear_out.weight, mask, mixer.num_heads, n_lv)
+    gate_scan_train, the output projection; one backward, in which the four weight gradients are one launch. `weights` as
+    mixer_fits returns them."""
+    ((Wi, bi), (Wf, bf), (Wr, br)), (W_in, W_x, W_s, W_out) = weights
+    return _MixerTrain.apply(x, W_in, W_x, W_s, Wi, Wf, Wr, bi, bf, br, W_out, mask, mixer.num_heads, n_lv)
 
 
 # ---------------------------------------------------------------------------------------------
@@ -282,7 +282,7 @@ def attention_fits(attn, x):
     return (x.dim() == 3 and x.is_cuda and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
             and x.dtype == torch.bfloat16 and x.shape[-1] == d and attn.head_dim == 64
             and not torch.is_autocast_enabled("cuda") and x.numel() * 3 * x.element_size() < 2 ** 31
-            and all(plain_linear(l, x.dtype, d) and l.weight.shape[0] == d
+            and all(plain_linear(l, x.dtype, d, x.device) and l.weight.shape[0] == d
                     for l in (attn.linear_q, attn.linear_k, attn.linear_v, attn.linear_out)))
 
 

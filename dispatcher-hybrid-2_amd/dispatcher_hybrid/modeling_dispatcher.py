@@ -168,13 +168,14 @@ class DispatcherMixer(nn.Module):
             x.requires_grad or any(p.requires_grad for p in self.parameters()))
         if needs_grad:
             from . import fused_train as ft
-            if ft.mixer_fits(self, x, mask, n_lv):
+            weights = ft.mixer_fits(self, x, mask, n_lv)
+            if weights is not None:
                 # the whole layer as one operation with its own backward
-                return ft.mixer_train(self, x, mask, n_lv)
+                return ft.mixer_train(self, x, mask, n_lv, weights)
             V0, A, Bs = self.linear_in(x), self.gate_hidden(x), self.gate_hidden_src(x)
-        elif mixer_layer_fits(self, x):
+        elif (weights := mixer_layer_fits(self, x)) is not None:
             # inference on few rows: the whole layer in one native call
-            return mixer_layer(self, x, mask if mask.dim() == 3 else None, n_lv)
+            return mixer_layer(self, x, mask if mask.dim() == 3 else None, n_lv, weights)
         else:
             V0, A, Bs = input_projections(x, self)
         m3 = mask[..., :n_lv] if mask.dim() == 3 else None
@@ -327,7 +328,7 @@ class SwiGLU(nn.Module):
                 g, u = self.linear_gate(h), self.linear_up(h)
                 if g.shape == u.shape and g.dtype == u.dtype and g.dtype in (torch.float32, torch.bfloat16):
                     # (a hook may have kept the gate's output)
-                    a = silu_mul(g, u, out=g if plain_linear(self.linear_gate, h.dtype, h.shape[-1]) else None)
+                    a = silu_mul(g, u, out=g if plain_linear(self.linear_gate, h.dtype, h.shape[-1], h.device) else None)
                 else:
                     a = F.silu(g) * u
             # (bf16: the shapes it was measured on; fp32 stays on the library)

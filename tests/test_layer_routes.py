@@ -38,7 +38,8 @@ NOT_PLAIN = {"hook": _hooked, "replaced forward": _replaced, "unaligned weight":
 def test_only_plain_projections_are_multiplied_directly(kind):
     from dispatcher_hybrid import fused_gates as fg
     make = lambda: nn.Linear(64, 64, bias=False).bfloat16()
-    x = SimpleNamespace(is_cuda=True, dtype=torch.bfloat16, shape=(1, 8, 64))         # what the predicates read of a GPU input
+    # what the predicates read of a GPU input
+    x = SimpleNamespace(is_cuda=True, dtype=torch.bfloat16, shape=(1, 8, 64), device=torch.device("cpu"))
     assert fg.projections_fit(x, [make(), make()]) and fg.swiglu_fits(x, make(), make())
     assert not fg.projections_fit(x, [make(), NOT_PLAIN[kind](make())])
     assert not fg.swiglu_fits(x, NOT_PLAIN[kind](make()), make())
@@ -58,3 +59,65 @@ def test_rows_a_kernel_cannot_read_are_copied():
     for t in copied:
         r = _rows16(t, 8)
         assert torch.equal(r, t) and r.is_contiguous() and r.stride(-2) == t.shape[-1] and r.data_ptr() % 16 == 0
+
+
+def _mixer(dtype=torch.bfloat16, d=64):
+    from dispatcher_hybrid import DispatcherConfig
+    from dispatcher_hybrid.modeling_dispatcher import DispatcherMixer
+    torch.manual_seed(d)
+    return DispatcherMixer(DispatcherConfig(d_model=d, num_heads=d // 64, max_len=64, num_layers=1, attn_layers=(),
+                                            vocab_size=64, dim_feedforward=64)).to(dtype)
+
+
+class _NoLibrary:
+    def __getattr__(self, name):
+        raise AssertionError(f"{name}: the library was reached")
+
+
+def test_host_pointers_never_reach_a_kernel(monkeypatch):
+    """Tensors that are not on the GPU, or not all on one, raise before any library call."""
+    from dispatcher_hybrid import _hip
+    from dispatcher_hybrid import fused_gates as fg
+    from dispatcher_hybrid import fused_train as ft
+    monkeypatch.setattr(_hip, "lib", _NoLibrary())
+    mx, T, L = _mixer(), 8, 4
+    (Wi, bi), (Wf, bf), (Wr, br) = [(w.detach(), b.detach()) for w, b in mx._gate_params()]
+    A = torch.zeros(1, T, 64).bfloat16()
+    mask, pre = torch.ones(1, T, L).bfloat16(), torch.zeros(1, T, L, 1).bfloat16()
+    with torch.no_grad():
+        for call in (lambda: fg.fused_gate_scan(A, A, Wi, Wf, Wr, bi, bf, br, L, mask, A, 1),
+                     lambda: fg._scan_launch(pre, pre, pre, None, A, A, 1, L, 0, "scan"),
+                     lambda: fg.mixer_layer(mx, A, mask, L, fg.plain_mixer_weights(mx, A.dtype, A.device)),
+                     lambda: fg._preacts_bwd_launch(A, A, Wi, Wf, Wr, [pre] * 3, mask, [A, A], L, L, "bwd"),
+                     lambda: ft._gate_scan_fwd(A, A, (Wi, Wf, Wr), (bi, bf, br), mask, A, 1, L, "train")):
+            with pytest.raises(RuntimeError, match="GPU|device|Could not run"):
+                call()
+    on_gpu = SimpleNamespace(is_cuda=True, get_device=lambda: 0, device="cuda:0")
+    _hip.same_gpu("x", on_gpu, None, on_gpu)
+    with pytest.raises(RuntimeError, match="one device"):
+        _hip.same_gpu("x", on_gpu, None, A)
+
+
+def test_layers_and_masks_on_another_device_are_not_launched_directly():
+    from dispatcher_hybrid import fused_gates as fg
+    from dispatcher_hybrid import fused_train as ft
+    mx, elsewhere = _mixer(), torch.device("meta")
+    x = torch.zeros(1, 8, 64).bfloat16()
+    mask = torch.ones(8, 6).bfloat16()
+    assert fg.plain_linear(mx.linear_in, x.dtype, 64, x.device) and not fg.plain_linear(mx.linear_in, x.dtype, 64, elsewhere)
+    with torch.no_grad():
+        assert fg.mixer_layer_fits(mx, x) and not fg.mixer_layer_fits(mx, x.to(elsewhere))
+    assert ft.mixer_fits(mx, x, mask, 4)
+    assert not ft.mixer_fits(mx, x.to(elsewhere), mask.to(elsewhere), 4) and not ft.mixer_fits(mx, x, mask.to(elsewhere), 4)
+
+
+def test_masks_of_other_sizes_raise_or_broadcast():
+    from dispatcher_hybrid.fused_gates import _mask_view
+    b, T, n = 2, 8, 3
+    for shape in ((2, 8, 5), (2, 8, 3), (1, 8, 3), (2, 1, 1)):
+        mask = torch.rand(shape)
+        m, *strides = _mask_view(mask, torch.float32, b, T, n)
+        assert torch.equal(m.as_strided((b, T, n), strides), mask[..., :n].expand(b, T, n))
+    for shape in ((2, 7, 3), (2, 8, 2), (3, 8, 3), (8, 3)):
+        with pytest.raises((RuntimeError, ValueError)):
+            _mask_view(torch.rand(shape), torch.float32, b, T, n)

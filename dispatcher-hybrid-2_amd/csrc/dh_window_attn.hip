@@ -197,10 +197,12 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
 #pragma unroll
     for (int j = 0; j < 16; ++j) mx = fmaxf(mx, p[j]);
     mx = across_groups_max(mx) * a.scale2;        // scale2 > 0
-    // the running max moves only when it falls 2^8 behind (the weights stay below 2^8, exact in fp32 and bf16 alike), so
-    // the output is rarely rescaled
-    if (__builtin_amdgcn_ballot_w64(mx > m + 8.f)) {
-      const float mn = fmaxf(m, mx);
+    // a query's running max moves only when it falls 2^8 behind (its weights stay below 2^8), so the output is rarely
+    // rescaled; the decision is the query's own (a lane that keeps its max has alpha 1), so its result does not depend on the
+    // other queries of the wave
+    const bool behind = mx > m + 8.f;
+    if (__builtin_amdgcn_ballot_w64(behind)) {
+      const float mn = behind ? mx : m;
       const float alpha = __builtin_amdgcn_exp2f(m - mn);
       m = mn;
       l *= alpha;

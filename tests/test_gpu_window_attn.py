@@ -105,3 +105,21 @@ def test_window_attention_rejects_unsupported():
     k_wide.copy_(k)
     with pytest.raises(ValueError, match="one stride"):
         fa.window_attention(q, k_wide, v, cos, sin, 2, 0)
+
+
+@pytest.mark.parametrize("hd,window", [(64, 0), (64, 100), (32, 0), (128, 48)])
+def test_window_attention_of_a_position_does_not_see_later_ones(hd, window):
+    """y[:, :t] keeps its bits whatever stands from t on, and when the sequence ends there: t inside a 16-query group and a
+    64-key block, scores wide enough (std ~ 40 in log2) that the queries of a group rescale in different blocks."""
+    from dispatcher_hybrid import fused_attention as fa
+    T, H = 330, 2
+    cos, sin = _rope_tables(T, hd)
+    q, k, v = _inputs(2, T, H, hd, 21)
+    q, k = q * 5, k * 5
+    q2, k2, v2 = _inputs(2, T, H, hd, 22)
+    y = fa.window_attention(q, k, v, cos, sin, H, window)
+    for t in (1, 9, 37, 70, 137, 200, 325):
+        mixed = [torch.cat((a[:, :t], b[:, t:] * 9), 1) for a, b in ((q, q2), (k, k2), (v, v2))]
+        assert torch.equal(fa.window_attention(*mixed, cos, sin, H, window)[:, :t], y[:, :t]), t
+        cut = [a[:, :t].contiguous() for a in (q, k, v)]
+        assert torch.equal(fa.window_attention(*cut, cos, sin, H, window), y[:, :t]), t

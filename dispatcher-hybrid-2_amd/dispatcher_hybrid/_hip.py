@@ -165,6 +165,7 @@ def require_gpu(t, what):
 def same_gpu(what, x, *others):
     """Raise unless x is on a GPU and the other tensors (None allowed) are on the same one: a kernel gets bare pointers."""
     require_gpu(x, what)
+    index = x.get_device()
     for t in others:
-        if t is not None and t.get_device() != x.get_device():
+        if t is not None and t.get_device() != index:
             raise RuntimeError(f"{what}: all tensors must be on one device (got {x.device} and {t.device})")

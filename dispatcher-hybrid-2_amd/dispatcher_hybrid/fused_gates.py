@@ -467,16 +467,21 @@ def plain_linear(l, dtype, n_in, device=None):
     return plain_weight(l, dtype, n_in, device) is not None and not _has_any_global_hook()
 
 
+def plain_square_weights(linears, d, dtype, device):
+    """The (d, d) weights of these layers if each is plain (plain_linear) and of this dtype and device, else None."""
+    ws = [plain_weight(l, dtype, d, device) for l in linears]
+    return None if _has_any_global_hook() or any(w is None or w.shape[0] != d for w in ws) else ws
+
+
 def plain_mixer_weights(mixer, dtype, device):
     """(gate parameters, projection weights in, x, s, out) of a mixer layer whose (d, d) projections are plain (plain_linear)
     and whose parameters share this dtype and device; else None."""
-    d, gates = mixer.embed_dim, mixer._gate_params()
-    if _has_any_global_hook() or not all(w.dtype == dtype and b.dtype == dtype and w.device == device and b.device == device
-                                         for w, b in gates):
+    gates = mixer._gate_params()
+    if not all(w.dtype == dtype and b.dtype == dtype and w.device == device and b.device == device for w, b in gates):
         return None
-    lins = [plain_weight(l, dtype, d, device)
-            for l in (mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src, mixer.linear_out)]
-    return None if any(w is None or w.shape[0] != d for w in lins) else (gates, lins)
+    lins = plain_square_weights((mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src, mixer.linear_out),
+                                mixer.embed_dim, dtype, device)
+    return None if lins is None else (gates, lins)
 
 
 _PLAIN = (torch.Tensor, nn.Parameter)

@@ -24,7 +24,7 @@ import torch.nn.functional as F
 from . import _hip
 from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch,
                           _preacts_launch, _rows16, fused_projections, plain_eager, plain_linear,
-                          plain_mixer_weights)
+                          plain_mixer_weights, plain_square_weights)
 
 SCAN_MAX_LEN = 4096
 SCAN_MAX_LEVELS = 12
@@ -53,7 +53,7 @@ def _gate_scan_fwd(A, B, W, bias, mask, V0, H, n_lv, what):
     """(V, pre, states) of the gate path; A, B, V0 (b, T, .) with unit-stride, 16-byte aligned rows, A and B alike."""
     b, T, d = V0.shape
     cd, dev = A.dtype, A.device
-    _hip.same_gpu(what, V0, A, B, *W, *bias, mask)
+    _hip.same_gpu(what, V0, mask)                                              # (the others at the first launch)
     V = torch.empty(b, T, d, device=dev, dtype=cd)
     pre = _gate_rows(b, H, n_lv, T, A)
     states = torch.empty(n_lv - 1, b, T, d, device=dev, dtype=cd)
@@ -77,7 +77,7 @@ def _gate_scan_bwd(A, B, W, mask, V0, pre, states, dV, dV0, outs, H, n_lv, what)
     with unit-stride, 16-byte aligned rows."""
     b, T, d = V0.shape
     cd = A.dtype
-    _hip.same_gpu(what, V0, A, B, *W, mask, pre, states, dV, dV0, *outs)
+    _hip.same_gpu(what, V0, mask, pre, states, dV)                             # (the others at the second launch)
     m = _scan_mask(mask, b, T, n_lv, cd)
     dpre = torch.empty_like(pre)
     scratch = torch.empty(b, T, d, device=A.device, dtype=cd)
@@ -274,16 +274,16 @@ def mixer_train(mixer, x, mask, n_lv, weights):
 # a whole attention layer
 # ---------------------------------------------------------------------------------------------
 def attention_fits(attn, x):
-    """Whether attention_train takes this layer and input: bf16 throughout and no autocast, 64-wide heads, plain bias-free
-    projections, plain eager execution."""
+    """The weights (q, k, v, out) attention_train takes if it takes this layer and input, else None: bf16 and one device
+    throughout and no autocast, 64-wide heads, plain bias-free projections, plain eager execution."""
     if not plain_eager():
-        return False
+        return None
     d = attn.embed_dim
-    return (x.dim() == 3 and x.is_cuda and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
+    if not (x.dim() == 3 and x.is_cuda and type(x) in (torch.Tensor, nn.Parameter) and x.numel() > 0
             and x.dtype == torch.bfloat16 and x.shape[-1] == d and attn.head_dim == 64
-            and not torch.is_autocast_enabled("cuda") and x.numel() * 3 * x.element_size() < 2 ** 31
-            and all(plain_linear(l, x.dtype, d, x.device) and l.weight.shape[0] == d
-                    for l in (attn.linear_q, attn.linear_k, attn.linear_v, attn.linear_out)))
+            and not torch.is_autocast_enabled("cuda") and x.numel() * 3 * x.element_size() < 2 ** 31):
+        return None
+    return plain_square_weights((attn.linear_q, attn.linear_k, attn.linear_v, attn.linear_out), d, x.dtype, x.device)
 
 
 def _attention_grads(inputs, need, dout, cos, sin, H, window):
@@ -356,12 +356,12 @@ class _AttentionTrain(torch.autograd.Function):
         return (*[v if n else None for v, n in zip([dx, *dw], need)], None, None, None, None)
 
 
-def attention_train(attn, x):
+def attention_train(attn, x, weights):
     """A WindowAttention's output (b, T, d), differentiable in x and the four projections (reference
-    dispatcher_hybrid/modeling_dispatcher.py:168-182; under create_graph through torch operations): scores and probabilities stay in registers in both directions
-    (``dh_window_attention_train_fwd`` / ``dh_window_attention_bwd``; the softmax's log-sum is kept in fp32), one product for
-    q, k, v and one launch for the four weight gradients. See attention_fits."""
+    dispatcher_hybrid/modeling_dispatcher.py:168-182; under create_graph through torch operations): scores and probabilities
+    stay in registers in both directions (``dh_window_attention_train_fwd`` / ``dh_window_attention_bwd``; the softmax's
+    log-sum is kept in fp32), one product for q, k, v and one launch for the four weight gradients. `weights` as
+    attention_fits returns them."""
     T = x.shape[1]
     cos, sin = attn.rope_tables(T, x.device, x.dtype)
-    return _AttentionTrain.apply(x, attn.linear_q.weight, attn.linear_k.weight, attn.linear_v.weight, attn.linear_out.weight,
-                                 cos, sin, attn.num_heads, attn.band(T))
+    return _AttentionTrain.apply(x, *weights, cos, sin, attn.num_heads, attn.band(T))

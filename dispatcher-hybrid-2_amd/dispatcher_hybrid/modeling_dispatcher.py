@@ -280,8 +280,9 @@ class WindowAttention(nn.Module):
         elif self.use_fused and x.is_cuda and torch.is_grad_enabled() and (
                 x.requires_grad or any(p.requires_grad for p in self.parameters())):
             from . import fused_train as ft
-            if ft.attention_fits(self, x):
-                return ft.attention_train(self, x)
+            weights = ft.attention_fits(self, x)
+            if weights is not None:
+                return ft.attention_train(self, x, weights)
         return self._forward_eager(x)
 
     def band(self, T):

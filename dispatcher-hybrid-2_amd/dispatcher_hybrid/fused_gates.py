@@ -31,6 +31,8 @@ import torch
 import torch.nn as nn
 from torch.autograd import forward_ad
 from torch.nn.modules.module import _has_any_global_hook
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _hip
 
@@ -442,11 +444,17 @@ def project(x, linears, max_rows):
     return [l(x) for l in linears]
 
 
+def _function_mode():
+    """Whether a torch-function mode (other than a default device) watches or replaces calls of torch functions."""
+    return torch._C._len_torch_function_stack() > 0 and any(
+        type(m) is not DeviceContext for m in _get_current_function_mode_stack())
+
+
 def plain_eager():
     """Whether kernels may be launched without a registered operation around them: no compiler, tracer, torch.func transform
-    (grad, vmap, ...), forward-mode level or dispatch mode looks at the tensors' operations."""
+    (grad, vmap, ...), forward-mode level, dispatch mode or function mode looks at the tensors' operations."""
     return not (torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active() or torch.jit.is_tracing()
-                or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0)
+                or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0 or _function_mode())
 
 
 def plain_weight(l, dtype, n_in, device=None):
@@ -463,14 +471,15 @@ def plain_weight(l, dtype, n_in, device=None):
 
 
 def plain_linear(l, dtype, n_in, device=None):
-    """Whether x . weight^T is all that calling this layer does (plain_weight, and no hook on every module)."""
-    return plain_weight(l, dtype, n_in, device) is not None and not _has_any_global_hook()
+    """Whether x . weight^T is all that calling this layer does: plain_weight, no hook on every module and no function mode
+    that would see the call of F.linear."""
+    return plain_weight(l, dtype, n_in, device) is not None and not _has_any_global_hook() and not _function_mode()
 
 
 def plain_square_weights(linears, d, dtype, device):
     """The (d, d) weights of these layers if each is plain (plain_linear) and of this dtype and device, else None."""
     ws = [plain_weight(l, dtype, d, device) for l in linears]
-    return None if _has_any_global_hook() or any(w is None or w.shape[0] != d for w in ws) else ws
+    return None if _has_any_global_hook() or _function_mode() or any(w is None or w.shape[0] != d for w in ws) else ws
 
 
 def plain_mixer_weights(mixer, dtype, device):

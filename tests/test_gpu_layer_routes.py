@@ -113,3 +113,26 @@ def test_broadcast_inputs_in_inference(cls, T):
     x = torch.randn(256, device=DEV).bfloat16().expand(2, T, 256)
     with torch.no_grad():
         assert torch.equal(layer(*_inputs(layer, cls, x)), layer(*_inputs(layer, cls, x.contiguous())))
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("cls", ["DispatcherMixer", "WindowAttention", "SwiGLU"])
+def test_a_function_mode_sees_every_product(cls, train):
+    from torch.overrides import TorchFunctionMode
+    import torch.nn.functional as F
+    layer = _layer(cls, torch.bfloat16)
+    layer.use_fused_gates = layer.use_fused = True
+    x = torch.randn(1, 100, 256, device=DEV).bfloat16()
+    seen = []
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func is F.linear)
+            return func(*args, **(kwargs or {}))
+
+    with torch.set_grad_enabled(train):
+        want = layer(*_inputs(layer, cls, x))
+        with Watch():
+            got = layer(*_inputs(layer, cls, x))
+    assert sum(seen) == (3 if cls == "SwiGLU" else 4)
+    assert (got.double() - want.double()).norm() <= 1e-2 * want.double().norm()

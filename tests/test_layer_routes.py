@@ -121,3 +121,30 @@ def test_masks_of_other_sizes_raise_or_broadcast():
     for shape in ((2, 7, 3), (2, 8, 2), (3, 8, 3), (8, 3)):
         with pytest.raises((RuntimeError, ValueError)):
             _mask_view(torch.rand(shape), torch.float32, b, T, n)
+
+
+def test_function_modes_see_a_layers_products():
+    """Under a torch-function mode nothing is launched past it; a default device (a mode of torch's own) is not one."""
+    from dispatcher_hybrid import fused_gates as fg
+    from dispatcher_hybrid import fused_train as ft
+    from torch.overrides import TorchFunctionMode
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    mx, x, mask = _mixer(), torch.zeros(1, 8, 64).bfloat16(), torch.ones(8, 6).bfloat16()
+    gpu = SimpleNamespace(is_cuda=True, dtype=x.dtype, shape=x.shape, device=x.device)
+    lin = mx.linear_in
+
+    def routes():
+        return [fg.plain_eager(), fg.projections_fit(gpu, [lin]), fg.swiglu_fits(gpu, lin, lin),
+                fg.mixer_layer_fits(mx, x) is not None, ft.mixer_fits(mx, x, mask, 4) is not None]
+
+    assert all(routes())
+    with torch.device("cpu"):
+        assert all(routes())
+        with Watch():
+            assert not any(routes())
+    with Watch():
+        assert not any(routes())

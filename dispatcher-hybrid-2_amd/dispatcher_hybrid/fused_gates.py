@@ -319,7 +319,9 @@ def fused_gate_scan(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, num_heads):
     fused_level_scan(*fused_gate_preacts(...), mask, V0, num_heads, n_lv) up to the bf16 rounding
     of the activated gates, which follows the eager path (reference
     dispatcher_hybrid/modeling_dispatcher.py:86-88, 100-121)."""
-    if type(A) is torch.Tensor and A.is_cuda and plain_eager():
+    # (wanted gradients go through the registered operation, whose backward says that it has none)
+    if type(A) is torch.Tensor and A.is_cuda and plain_eager() and not (torch.is_grad_enabled() and any(
+            t.requires_grad for t in (A, B, Wi, Wf, Wr, bi, bf, br, V0))):
         return _gate_scan_body(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
     return torch.ops.dispatcher.gate_scan_fwd(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv)
 

@@ -136,3 +136,23 @@ def test_a_function_mode_sees_every_product(cls, train):
             got = layer(*_inputs(layer, cls, x))
     assert sum(seen) == (3 if cls == "SwiGLU" else 4)
     assert (got.double() - want.double()).norm() <= 1e-2 * want.double().norm()
+
+
+def test_gate_scan_without_a_gradient_says_so():
+    """fused_gate_scan has no backward: with a gradient wanted, its result asks for one and refuses it."""
+    from dispatcher_hybrid.fused_gates import fused_gate_scan
+    b, T, H, L = 1, 40, 2, 5
+    A, B, V0 = (torch.randn(b, T, 64 * H, device=DEV).bfloat16() for _ in range(3))
+    W = [(torch.randn(L, H, 64 * H, device=DEV) * 0.05).bfloat16() for _ in range(3)]
+    bias = [torch.zeros(L, H, device=DEV).bfloat16() for _ in range(3)]
+    run = lambda: fused_gate_scan(A, B, *W, *bias, L, None, V0, H)
+    want = run()
+    for t in (A, W[1], bias[2], V0):
+        t.requires_grad_()
+        got = run()
+        assert torch.equal(got, want) and got.requires_grad
+        with pytest.raises(RuntimeError):
+            got.sum().backward()
+        with torch.no_grad():
+            assert torch.equal(run(), want)
+        t.requires_grad_(False)

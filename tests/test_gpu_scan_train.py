@@ -210,3 +210,34 @@ def test_mixer_train_under_transforms():
     compiled = torch.compile(mx, backend="aot_eager", fullgraph=True)
     traced, = torch.autograd.grad(compiled(xg, mask).square().sum(), xg)
     assert (traced - want).norm() <= 2e-5 * want.norm()
+
+
+@pytest.mark.parametrize("T", [24, 100, 200, 256, 257, 500])
+def test_mixer_train_fp32_is_as_exact_as_layer_by_layer(T):
+    """Distance from float64 of the whole-layer operation's fp32 output and gradients against that of the layer-by-layer
+    form (torch products and scan; a mask that takes gradients keeps it there), whose sums are no longer than 1024 terms:
+    at most 1.15 times it, which covers the other order of the same sums."""
+    mx, ref = _mixer(torch.float32, 1024, 512), _mixer(torch.float64, 1024, 512)
+    with torch.no_grad():
+        for n, p in mx.named_parameters():
+            if "bias" not in n:
+                p.mul_(0.25)
+    ref.load_state_dict({n: p.double() for n, p in mx.state_dict().items()})
+    mx.use_fused_gates = True
+    t = torch.arange(T, device=DEV).unsqueeze(1)
+    mask = (t >= (1 << torch.arange(9, device=DEV))).float()
+    g = torch.Generator(device=DEV).manual_seed(2)
+    x, dy = (torch.randn(1, T, 1024, device=DEV, generator=g) for _ in range(2))
+
+    def grads(layer, x, m, dy):
+        x = x.clone().requires_grad_()
+        layer.zero_grad()
+        y = layer(x, m)
+        y.backward(dy)
+        return [("y", y.detach()), ("dx", x.grad)] + [(n, p.grad.clone()) for n, p in layer.named_parameters()]
+
+    exact = grads(ref, x.double(), mask.double(), dy.double())
+    whole, parts = grads(mx, x, mask, dy), grads(mx, x, mask.clone().requires_grad_(), dy)
+    for (n, e), (_, a), (_, b) in zip(exact, whole, parts):
+        if "bias" not in n:                                      # (a few hundred values: their distance is a matter of luck)
+            assert (a.double() - e).norm() <= 1.15 * (b.double() - e).norm(), n

@@ -166,6 +166,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t state_rows(const Args& a, int 
   return head_rows<T>((const T*)a.Vs + (int64_t)(l - 1) * plane, (int64_t)b * a.T * d, d, h, a.T);
 }
 
+// the gates' logistic function: fp32 as torch evaluates it (library exp, IEEE divide), as the states and gradients are kept in
+// full; bf16 pre-activations by the hardware exp and reciprocal (1 ulp of fp32 each, far below their own rounding)
+template <typename T>
+__device__ __forceinline__ float gate_sigmoid(float x) {
+  if constexpr (sizeof(T) == 4) return 1.0f / (1.0f + expf(-x));
+  return dh_sigmoid(x);
+}
+
 struct Gate {
   float m, si, sf, r;           // r: the transmit gate at the source
   __device__ __forceinline__ float f() const { return __builtin_fmaf(sf, m, 1.f - m); }
@@ -180,9 +188,9 @@ __device__ __forceinline__ Gate gate_at(const Args& a, int b, int h, int l, int 
   const int tc = in ? t : 0, ts = in ? t - lag : 0;
   const int64_t row = (int64_t)b * a.spb + (int64_t)h * a.sph + (int64_t)l * a.spl;
   Gate g;
-  g.si = dh_sigmoid(Elem<T>::load((const T*)a.pre[0] + row + tc));
-  g.sf = dh_sigmoid(Elem<T>::load((const T*)a.pre[1] + row + tc));
-  g.r = dh_sigmoid(Elem<T>::load((const T*)a.pre[2] + row + ts));
+  g.si = gate_sigmoid<T>(Elem<T>::load((const T*)a.pre[0] + row + tc));
+  g.sf = gate_sigmoid<T>(Elem<T>::load((const T*)a.pre[1] + row + tc));
+  g.r = gate_sigmoid<T>(Elem<T>::load((const T*)a.pre[2] + row + ts));
   g.m = in ? mask_of<T>(a, b, tc, l) : 0.f;
   return g;
 }
@@ -324,9 +332,9 @@ __device__ __forceinline__ Gate tile_gate(const Args& a, const GateTile<T, P>& g
   const bool in = lane < P && lane >= lg && t < a.T;
   const int j = in ? lane : 0, js = in ? lane - lg : 0;
   Gate g;
-  g.si = dh_sigmoid(Elem<T>::load(&gl.v[0][m][j][w]));
-  g.sf = dh_sigmoid(Elem<T>::load(&gl.v[1][m][j][w]));
-  g.r = dh_sigmoid(Elem<T>::load(&gl.v[2][m][js][w]));
+  g.si = gate_sigmoid<T>(Elem<T>::load(&gl.v[0][m][j][w]));
+  g.sf = gate_sigmoid<T>(Elem<T>::load(&gl.v[1][m][j][w]));
+  g.r = gate_sigmoid<T>(Elem<T>::load(&gl.v[2][m][js][w]));
   g.m = in ? mask_of<T>(a, b, t, kLocal + m) : 0.f;
   return g;
 }

@@ -241,3 +241,21 @@ def test_mixer_train_fp32_is_as_exact_as_layer_by_layer(T):
     for (n, e), (_, a), (_, b) in zip(exact, whole, parts):
         if "bias" not in n:                                      # (a few hundred values: their distance is a matter of luck)
             assert (a.double() - e).norm() <= 1.15 * (b.double() - e).norm(), n
+
+
+def test_gate_scan_train_fp32_far_gates():
+    """Gates far from the middle: admit pre-activations of -85 .. -20 (a bias alone, exact) and their gradients, value by
+    value. The library exp and an IEEE divide are within 2 ulp, the gradient's few products half of one each: 8 x 2^-24."""
+    from dispatcher_hybrid.fused_train import gate_scan_train
+    b, T, H, L = 1, 600, 1, 10
+    A, B, V0 = torch.zeros(b, T, 64, device=DEV), torch.zeros(b, T, 64, device=DEV), torch.ones(b, T, 64, device=DEV)
+    W = [torch.zeros(L, H, 64, device=DEV) for _ in range(3)]
+    far = -torch.linspace(20, 85, L, device=DEV).view(L, H)
+    bias = [far.clone().requires_grad_(), torch.full((L, H), 60.0, device=DEV), torch.full((L, H), 60.0, device=DEV)]
+    mask = (torch.arange(T, device=DEV).unsqueeze(1) >= (1 << torch.arange(L, device=DEV))).float()
+    V = gate_scan_train(A, B, *W, *bias, L, mask, V0, H)
+    only = torch.zeros_like(V)
+    only[0, T - 1, 0] = 1                                        # one destination: no sum over positions
+    got, = torch.autograd.grad(V, bias[0], only)
+    want = torch.sigmoid(far.double())                           # forget = transmit = V = 1 to 1e-9: d/dx sigmoid = itself
+    assert ((got.double() - want).abs() <= 8 * 2.0 ** -24 * want).all()

@@ -123,9 +123,9 @@ def _(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv):
 @torch.library.custom_op("dispatcher::gate_scan_train_bwd", mutates_args=(), device_types="cuda")
 def _gate_scan_train_bwd_op(A: torch.Tensor, B: torch.Tensor, Wi: torch.Tensor, Wf: torch.Tensor, Wr: torch.Tensor,
                             mask: torch.Tensor, V0: torch.Tensor, pre: torch.Tensor, states: torch.Tensor,
-                            dV: torch.Tensor, num_heads: int, n_lv: int) -> List[torch.Tensor]:
-    # the gradients in the inputs' dtype where they share one, else (autocast: wider weights) in fp32
-    od = A.dtype if Wi.dtype == A.dtype else torch.float32
+                            dV: torch.Tensor, num_heads: int, n_lv: int, wide: bool) -> List[torch.Tensor]:
+    # the gradients in A's dtype, or (wide: wider weights or biases, as under autocast) in fp32
+    od = torch.float32 if wide else A.dtype
     dV0 = torch.empty(V0.shape, device=A.device, dtype=A.dtype)
     outs = [torch.empty(A.shape, device=A.device, dtype=od) for _ in range(2)] + _gate_grads(Wi, A.shape[-1], od, A.device)
     if V0.numel() == 0:
@@ -137,8 +137,8 @@ def _gate_scan_train_bwd_op(A: torch.Tensor, B: torch.Tensor, Wi: torch.Tensor, 
 
 
 @_gate_scan_train_bwd_op.register_fake
-def _(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, num_heads, n_lv):
-    od = A.dtype if Wi.dtype == A.dtype else torch.float32
+def _(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, num_heads, n_lv, wide):
+    od = torch.float32 if wide else A.dtype
     return ([A.new_empty(V0.shape)] + [A.new_empty(A.shape, dtype=od) for _ in range(2)]
             + _gate_grads(Wi, A.shape[-1], od, A.device))
 
@@ -157,7 +157,8 @@ def _scan_backward(ctx, grads):
     if dV is None:
         return (None,) * 12
     A, B, Wi, Wf, Wr, mask, V0, pre, states = ctx.saved_tensors
-    dV0, *rest = torch.ops.dispatcher.gate_scan_train_bwd(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, *ctx.sizes)
+    wide = any(dt != A.dtype for dt in ctx.dtypes)
+    dV0, *rest = torch.ops.dispatcher.gate_scan_train_bwd(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, *ctx.sizes, wide)
     return (*[g.to(dt) for g, dt in zip(rest, ctx.dtypes)], None, dV0, None, None)
 
 

@@ -259,3 +259,28 @@ def test_gate_scan_train_fp32_far_gates():
     got, = torch.autograd.grad(V, bias[0], only)
     want = torch.sigmoid(far.double())                           # forget = transmit = V = 1 to 1e-9: d/dx sigmoid = itself
     assert ((got.double() - want).abs() <= 8 * 2.0 ** -24 * want).all()
+
+
+@pytest.mark.parametrize("wide", [(6,), (3,), (4, 7)])
+def test_gate_scan_train_keeps_wider_parameters_gradients(wide):
+    """bf16 activations with some fp32 gate weights or biases: those parameters' gradients are the fp32 sums, not their bf16
+    rounding, and the others round the same sums."""
+    from dispatcher_hybrid.fused_train import gate_scan_train
+    g = torch.Generator(device=DEV).manual_seed(4)
+    b, T, H, L = 2, 150, 2, 8
+    A, B, V0 = (torch.randn(b, T, 64 * H, device=DEV, generator=g).bfloat16() for _ in range(3))
+    P = [(torch.randn(L, H, 64 * H, device=DEV, generator=g) * 0.05).bfloat16() for _ in range(3)]
+    P += [torch.randn(L, H, device=DEV, generator=g).bfloat16() for _ in range(3)]
+    mask = (torch.arange(T, device=DEV).unsqueeze(1) >= (1 << torch.arange(L, device=DEV))).float()
+    dV = torch.randn(b, T, 64 * H, device=DEV, generator=g).bfloat16()
+
+    def grads(fp32):
+        leaves = [(p.float() if i + 2 in fp32 else p).clone().requires_grad_() for i, p in enumerate(P)]
+        return torch.autograd.grad(gate_scan_train(A, B, *leaves, L, mask, V0, H), leaves, dV)
+
+    full = grads(range(2, 8))
+    for i, (p, f) in enumerate(zip(grads(wide), full)):
+        if i + 2 in wide:
+            assert p.dtype == torch.float32 and torch.equal(p, f) and not torch.equal(p, p.bfloat16().float())
+        else:
+            assert torch.equal(p, f.bfloat16())

@@ -49,6 +49,12 @@ def _scan_mask(mask, b, T, n_lv, cd):
     return mask[..., :n_lv].to(cd).expand(b, T, n_lv)
 
 
+def _dense(t):
+    """A saved tensor in the layout it was saved in, contiguous and 16-byte aligned (a saved-tensor hook may hand back
+    another one)."""
+    return t if t.is_contiguous() and t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+
+
 def _gate_scan_fwd(A, B, W, bias, mask, V0, H, n_lv, what):
     """(V, pre, states) of the gate path; A, B, V0 (b, T, .) with unit-stride, 16-byte aligned rows, A and B alike."""
     b, T, d = V0.shape
@@ -78,7 +84,7 @@ def _gate_scan_bwd(A, B, W, mask, V0, pre, states, dV, dV0, outs, H, n_lv, what)
     b, T, d = V0.shape
     cd = A.dtype
     _hip.same_gpu(what, V0, mask, pre, states, dV)                             # (the others at the second launch)
-    m = _scan_mask(mask, b, T, n_lv, cd)
+    m, pre, states = _scan_mask(mask, b, T, n_lv, cd), _dense(pre), _dense(states)
     dpre = torch.empty_like(pre)
     scratch = torch.empty(b, T, d, device=A.device, dtype=cd)
     p = _hip.ptr
@@ -274,6 +280,7 @@ class _MixerTrain(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, dy):
         x, Wi, Wf, Wr, W_out, mask, proj, V, pre, states, W_cat = ctx.saved_tensors
+        proj, V, W_cat = _dense(proj), _dense(V), _dense(W_cat)
         num_heads, n_lv = ctx.sizes
         need = ctx.needs_input_grad
         b, T, d = x.shape
@@ -365,6 +372,7 @@ class _AttentionTrain(torch.autograd.Function):
         if torch.is_grad_enabled():                                            # create_graph: gradients of these are wanted
             g = _attention_grads((x, W_q, W_k, W_v, W_out), need, dout, cos, sin, H, window)
             return (*g, None, None, None, None)
+        cos, sin, proj, y, kv, lse, W_cat = (_dense(t) for t in (cos, sin, proj, y, kv, lse, W_cat))
         b, T, d = x.shape
         hd = d // H
         x2, do2 = _rows16(x.reshape(b * T, d), 8), _rows16(dout.reshape(b * T, d), 8)

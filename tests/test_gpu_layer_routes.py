@@ -156,3 +156,33 @@ def test_gate_scan_without_a_gradient_says_so():
         with torch.no_grad():
             assert torch.equal(run(), want)
         t.requires_grad_(False)
+
+
+def _last_dim_first(t):
+    return t.movedim(-1, 0).contiguous().movedim(0, -1) if t.dim() > 1 else t
+
+
+def _odd_offset(t):
+    return torch.cat((t.flatten()[:1], t.flatten()))[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("unpack", [_last_dim_first, _odd_offset])
+@pytest.mark.parametrize("cls,route", [("DispatcherMixer", "layer"), ("DispatcherMixer", "operation"),
+                                       ("WindowAttention", "layer")])
+def test_saved_tensors_may_come_back_in_another_layout(cls, route, unpack):
+    """A saved-tensor hook that hands back the same values in other strides or at another alignment changes no gradient."""
+    layer = _layer(cls, torch.bfloat16)
+    layer.use_fused_gates = layer.use_fused = True
+    if route == "operation":                                     # a hook on a projection: the gate path's registered operation
+        layer.linear_in.register_forward_hook(lambda m, i, o: o * 1)
+    x, dy = (torch.randn(2, 70, 256, device=DEV).bfloat16() for _ in range(2))
+    x.requires_grad_()
+    leaves = [x, *layer.parameters()]
+    want = torch.autograd.grad(layer(*_inputs(layer, cls, x)), leaves, dy)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach().clone(), unpack):
+        y = layer(*_inputs(layer, cls, x))
+    for a, e in zip(torch.autograd.grad(y, leaves, dy), want):
+        if route == "layer":
+            assert torch.equal(a, e)
+        else:                                                    # (library products of other layouts sum in other orders)
+            assert (a.double() - e.double()).norm() <= 1e-2 * e.double().norm()

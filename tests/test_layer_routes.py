@@ -148,3 +148,13 @@ def test_function_modes_see_a_layers_products():
             assert not any(routes())
     with Watch():
         assert not any(routes())
+
+
+def test_saved_tensors_in_another_layout_are_copied_back():
+    from dispatcher_hybrid.fused_train import _dense
+    t = torch.arange(120.).view(2, 3, 20)
+    assert _dense(t).data_ptr() == t.data_ptr()
+    for other in (t.transpose(0, 2).contiguous().transpose(0, 2), torch.cat((t[..., :1], t), -1)[..., 1:],
+                  torch.cat((torch.zeros(1), t.flatten()))[1:].view_as(t)):
+        d = _dense(other)
+        assert torch.equal(d, t) and d.is_contiguous() and d.data_ptr() % 16 == 0

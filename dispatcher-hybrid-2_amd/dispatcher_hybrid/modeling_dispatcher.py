@@ -49,6 +49,12 @@ def level_gate_matmul(hidden, W, W_t=None):
     return torch.bmm(lhs, rhs).view(n, b, t, -1).permute(1, 2, 0, 3)
 
 
+def _replaced(module, base, names):
+    """Whether a subclass, or the module itself, has methods of its own in place of these of `base`."""
+    cls = type(module)
+    return any(n in module.__dict__ or (cls is not base and getattr(cls, n) is not getattr(base, n)) for n in names)
+
+
 class DispatcherMixer(nn.Module):
     """Gated dyadic shift-and-sum sequence mixer (the layer that replaces attention)."""
 
@@ -168,7 +174,9 @@ class DispatcherMixer(nn.Module):
             x.requires_grad or any(p.requires_grad for p in self.parameters()))
         if needs_grad:
             from . import fused_train as ft
-            weights = ft.mixer_fits(self, x, mask, n_lv)
+            # (a scan of the module's own runs as torch operations)
+            own_scan = _replaced(self, DispatcherMixer, ("_masks", "_scan_eager", "activate", "level_update"))
+            weights = None if own_scan else ft.mixer_fits(self, x, mask, n_lv)
             if weights is not None:
                 # the whole layer as one operation with its own backward
                 return ft.mixer_train(self, x, mask, n_lv, weights)
@@ -180,7 +188,7 @@ class DispatcherMixer(nn.Module):
             V0, A, Bs = input_projections(x, self)
         m3 = mask[..., :n_lv] if mask.dim() == 3 else None
         (Wi, bi), (Wf, bf), (Wr, br) = self._gate_params()
-        if needs_grad and ft.scan_fits(A, Bs, V0, mask, H, n_lv):
+        if needs_grad and not own_scan and ft.scan_fits(A, Bs, V0, mask, H, n_lv):
             # differentiable: pre-activations and level scan as one operation with its own backward
             V = ft.gate_scan_train(A, Bs, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, H)
         elif needs_grad:
@@ -280,7 +288,8 @@ class WindowAttention(nn.Module):
         elif self.use_fused and x.is_cuda and torch.is_grad_enabled() and (
                 x.requires_grad or any(p.requires_grad for p in self.parameters())):
             from . import fused_train as ft
-            weights = ft.attention_fits(self, x)
+            own = _replaced(self, WindowAttention, ("_forward_eager", "apply_rope"))
+            weights = None if own else ft.attention_fits(self, x)
             if weights is not None:
                 return ft.attention_train(self, x, weights)
         return self._forward_eager(x)

@@ -186,3 +186,19 @@ def test_saved_tensors_may_come_back_in_another_layout(cls, route, unpack):
             assert torch.equal(a, e)
         else:                                                    # (library products of other layouts sum in other orders)
             assert (a.double() - e.double()).norm() <= 1e-2 * e.double().norm()
+
+
+def test_training_runs_a_modules_own_scan_and_rotation():
+    """A mixer with another gate activation and an attention layer with another rotation train with them (the torch path's
+    output, tolerance as above)."""
+    import dispatcher_hybrid.modeling_dispatcher as md
+    mx, at = _layer("DispatcherMixer", torch.bfloat16), _layer("WindowAttention", torch.bfloat16)
+    mx.activate = lambda i, f, r, m: md.DispatcherMixer.activate(i, f, r, 0.5 * m)
+    at.apply_rope = lambda x, T: x
+    x = torch.randn(1, 100, 256, device=DEV).bfloat16()
+    for layer, cls in ((mx, "DispatcherMixer"), (at, "WindowAttention")):
+        want = layer(*_inputs(layer, cls, x))
+        layer.use_fused_gates = layer.use_fused = True
+        got = layer(*_inputs(layer, cls, x))
+        assert (got.double() - want.double()).norm() <= 1e-2 * want.double().norm()
+        got.sum().backward()

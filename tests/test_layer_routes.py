@@ -158,3 +158,24 @@ def test_saved_tensors_in_another_layout_are_copied_back():
                   torch.cat((torch.zeros(1), t.flatten()))[1:].view_as(t)):
         d = _dense(other)
         assert torch.equal(d, t) and d.is_contiguous() and d.data_ptr() % 16 == 0
+
+
+def test_methods_of_a_subclass_or_an_instance_are_seen():
+    from dispatcher_hybrid.modeling_dispatcher import DispatcherMixer, _replaced
+
+    class Named(DispatcherMixer):
+        pass
+
+    class Gentle(Named):
+        @staticmethod
+        def activate(pre_i, pre_f, pre_r, m):
+            return DispatcherMixer.activate(pre_i, pre_f, pre_r, 0.5 * m)
+
+    mx, names = _mixer(), ("_scan_eager", "activate")
+    assert not _replaced(mx, DispatcherMixer, names)
+    for cls, other in ((Named, False), (Gentle, True)):
+        mx.__class__ = cls
+        assert _replaced(mx, DispatcherMixer, names) is other
+    mx.__class__ = DispatcherMixer
+    mx.activate = Gentle.activate
+    assert _replaced(mx, DispatcherMixer, names)

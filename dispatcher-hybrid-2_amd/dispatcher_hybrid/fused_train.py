@@ -15,6 +15,7 @@ Importing this module loads the kernel library and raises ImportError if it is m
 """
 
 import ctypes
+from types import SimpleNamespace
 from typing import List
 
 import torch
@@ -22,9 +23,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _hip
-from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch,
-                          _preacts_launch, _rows16, fused_projections, plain_eager, plain_linear,
-                          plain_mixer_weights, plain_square_weights)
+from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch, _preacts_launch, _rows16,
+                          fused_gate_preacts, fused_projections, plain_eager, plain_mixer_weights, plain_square_weights)
 
 SCAN_MAX_LEN = 4096
 SCAN_MAX_LEVELS = 12
@@ -149,11 +149,32 @@ def _(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, num_heads, n_lv, wide):
             + _gate_grads(Wi, A.shape[-1], od, A.device))
 
 
+def _scan_again(A, B, Wi, Wf, Wr, bi, bf, br, V0, mask, H, n_lv):
+    """The gate path as torch operations after fused_gate_preacts: differentiable twice in all but the pre-activations (whose
+    operation refuses that), as the layer was before it had a backward of its own."""
+    from .modeling_dispatcher import DispatcherMixer
+    b, T, d = V0.shape
+    m3 = mask[..., :n_lv].expand(b, T, n_lv) if mask.dim() == 3 else None
+    pre = fused_gate_preacts(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, m3)
+    mx = SimpleNamespace(num_heads=H, shifts=[1 << l for l in range(n_lv)], activate=DispatcherMixer.activate,
+                         level_update=DispatcherMixer.level_update)
+    _, m_heads = DispatcherMixer._masks(mx, mask, b, T, n_lv)
+    V = V0.view(b, T, H, d // H).transpose(1, 2).reshape(b * H, T, d // H)
+    V = DispatcherMixer._scan_eager(mx, V, *pre, m_heads.to(V.dtype), b, T, n_lv)
+    return V.view(b, H, T, d // H).transpose(1, 2).reshape(b, T, d)
+
+
+def _grads_again(out, inputs, need, dout):
+    """The gradients of `inputs` (None where not needed) from dout, differentiable themselves."""
+    g = iter(torch.autograd.grad(out, [t for t, n in zip(inputs, need) if n], dout, create_graph=True))
+    return [next(g) if n else None for n in need]
+
+
 def _scan_setup(ctx, inputs, output):
     A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, num_heads, n_lv = inputs
     _, pre, states = output
     ctx.set_materialize_grads(False)
-    ctx.save_for_backward(A, B, Wi, Wf, Wr, mask, V0, pre, states)
+    ctx.save_for_backward(A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, pre, states)
     ctx.sizes = (num_heads, n_lv)
     ctx.dtypes = [t.dtype for t in (A, B, Wi, Wf, Wr, bi, bf, br)]
 
@@ -162,7 +183,11 @@ def _scan_backward(ctx, grads):
     dV = grads[0]
     if dV is None:
         return (None,) * 12
-    A, B, Wi, Wf, Wr, mask, V0, pre, states = ctx.saved_tensors
+    A, B, Wi, Wf, Wr, bi, bf, br, mask, V0, pre, states = ctx.saved_tensors
+    if torch.is_grad_enabled():                                                # create_graph: gradients of these are wanted
+        ins = [t.view_as(t) for t in (A, B, Wi, Wf, Wr, bi, bf, br, V0)]
+        g = _grads_again(_scan_again(*ins, mask, *ctx.sizes), ins, [ctx.needs_input_grad[i] for i in (*range(8), 9)], dV)
+        return (*g[:8], None, g[8], None, None)
     wide = any(dt != A.dtype for dt in ctx.dtypes)
     dV0, *rest = torch.ops.dispatcher.gate_scan_train_bwd(A, B, Wi, Wf, Wr, mask, V0, pre, states, dV, *ctx.sizes, wide)
     return (*[g.to(dt) for g, dt in zip(rest, ctx.dtypes)], None, dV0, None, None)
@@ -272,17 +297,23 @@ class _MixerTrain(torch.autograd.Function):
         V0, A, B = proj.view(b, T, 3 * d).split(d, -1)
         V, pre, states = _gate_scan_fwd(A, B, (Wi, Wf, Wr), (bi, bf, br), mask, V0, num_heads, n_lv, "mixer_train")
         y = _linear(V.view(b * T, d), W_out, OUT_GEMM_MAX_ROWS)
-        ctx.save_for_backward(x, Wi, Wf, Wr, W_out, mask, proj, V, pre, states, W_cat)
+        ctx.save_for_backward(x, W_in, W_x, W_s, Wi, Wf, Wr, bi, bf, br, W_out, mask, proj, V, pre, states, W_cat)
         ctx.sizes = (num_heads, n_lv)
         return y.view(b, T, d)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, dy):
-        x, Wi, Wf, Wr, W_out, mask, proj, V, pre, states, W_cat = ctx.saved_tensors
-        proj, V, W_cat = _dense(proj), _dense(V), _dense(W_cat)
+        *inputs, mask, proj, V, pre, states, W_cat = ctx.saved_tensors
         num_heads, n_lv = ctx.sizes
         need = ctx.needs_input_grad
+        if torch.is_grad_enabled():                                            # create_graph: gradients of these are wanted
+            inputs = [t.view_as(t) for t in inputs]                            # (tied weights: a gradient for each use)
+            x, W_in, W_x, W_s, *gates, W_out = inputs
+            V0, A, B = (F.linear(x, w) for w in (W_in, W_x, W_s))
+            y = F.linear(_scan_again(A, B, *gates, V0, mask, num_heads, n_lv), W_out)
+            return (*_grads_again(y, inputs, need[:11], dy), None, None, None)
+        x, _, _, _, Wi, Wf, Wr, _, _, _, W_out = inputs
+        proj, V, W_cat = _dense(proj), _dense(V), _dense(W_cat)
         b, T, d = x.shape
         x2, dy2 = _rows16(x.reshape(b * T, d), 8), _rows16(dy.reshape(b * T, d), 8)
         dV = torch.mm(dy2, W_out).view(b, T, d)
@@ -300,8 +331,8 @@ class _MixerTrain(torch.autograd.Function):
 
 
 def mixer_train(mixer, x, mask, n_lv, weights):
-    """A DispatcherMixer's output (b, T, d), differentiable (once) in x and every parameter (reference
-    dispatcher_hybrid/modeling_dispatcher.py:63-123): one product for the three input projections, the gate path of
+    """A DispatcherMixer's output (b, T, d), differentiable in x and every parameter (reference
+    dispatcher_hybrid/modeling_dispatcher.py:63-123; under create_graph layer by layer, see _scan_again): one product for the three input projections, the gate path of
     gate_scan_train, the output projection; one backward, in which the four weight gradients are one launch. `weights` as
     mixer_fits returns them."""
     ((Wi, bi), (Wf, bf), (Wr, br)), (W_in, W_x, W_s, W_out) = weights
@@ -335,9 +366,7 @@ def _attention_grads(inputs, need, dout, cos, sin, H, window):
     q, k = (rope_rotate(t, cos.float(), sin.float()) for t in (q, k))
     y = causal_window_attention(q, k, v, window).transpose(1, 2).reshape(b, T, d)
     out = F.linear(y, W[3]).to(inputs[0].dtype)
-    wanted = [t for t, n in zip(inputs, need) if n]
-    g = iter(torch.autograd.grad(out, wanted, dout, create_graph=True))
-    return [next(g) if n else None for n in need[:5]]
+    return _grads_again(out, inputs, need[:5], dout)
 
 
 class _AttentionTrain(torch.autograd.Function):

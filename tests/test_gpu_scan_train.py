@@ -284,3 +284,29 @@ def test_gate_scan_train_keeps_wider_parameters_gradients(wide):
             assert p.dtype == torch.float32 and torch.equal(p, f) and not torch.equal(p, p.bfloat16().float())
         else:
             assert torch.equal(p, f.bfloat16())
+
+
+@pytest.mark.parametrize("route", ["layer", "operation"])
+def test_mixer_gradients_of_gradients_that_avoid_the_gate_readouts(route):
+    """A penalty on the gradients of the value and output projections can be differentiated (through the scan, against the
+    eager mixer in float64); one that needs second derivatives of the gate readouts is refused. fp32, 12 levels of updates in
+    each direction: 5e-5."""
+    mx, ref = _mixer(torch.float32), _mixer(torch.float64)
+    ref.load_state_dict({n: p.double() for n, p in mx.state_dict().items()})
+    mx.use_fused_gates = True
+    if route == "operation":
+        mx.linear_in.register_forward_hook(lambda m, i, o: o * 1)
+    T = 70
+    mask = (torch.arange(T, device=DEV).unsqueeze(1) >= (1 << torch.arange(8, device=DEV))).float()
+    g = torch.Generator(device=DEV).manual_seed(6)
+    x, dy = (torch.randn(2, T, 128, device=DEV, generator=g) for _ in range(2))
+
+    def penalty(layer, x, m, dy):
+        first = torch.autograd.grad(layer(x, m), [layer.linear_in.weight, layer.linear_out.weight], dy, create_graph=True)
+        return [*first, *torch.autograd.grad(sum(f.square().sum() for f in first), list(layer.parameters()))]
+
+    for a, e in zip(penalty(mx, x, mask, dy), penalty(ref, x.double(), mask.double(), dy.double())):
+        assert (a.double() - e).norm() <= 5e-5 * e.norm()
+    first, = torch.autograd.grad(mx(x, mask), mx.gate_hidden.weight, dy, create_graph=True)
+    with pytest.raises(RuntimeError):
+        torch.autograd.grad(first.square().sum(), mx.gate_out)

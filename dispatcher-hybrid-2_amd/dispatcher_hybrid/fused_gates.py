@@ -417,8 +417,13 @@ def input_projections(x, mixer):
 # single 1024 x 1024 output projection (the mixer's and attention's linear_out) 6.7 / 8.9 at 1024, 9.3 / 10.7 at 2048,
 # 11.4 / 11.5 at 3000, 13.1 / 14.1 at 4096, 15.9 / 14.8 at 4608; the SwiGLU down projection (1024 x 2816) 12.1 / 14.0 at
 # 1024, 20.4 / 19.7 at 2048, 25.5 / 22.9 at 3000.
-# fp32: the 1024 x 1024 output projection 23.9 / 36.7 / 57.6 / 75.6 us at 1024 / 2048 / 3002 / 4096 rows against 20.6 / 36.7
-# / 68.2 / 63.8 for the library.
+# fp32: the line is a whole mixer layer's, which is one native call up to it (mixer_layer) and separate calls with the
+# library's output projection above (eager, us, one call against separate; a call that waits for the host takes ~112): d 512
+# 38 / 114 at 24 rows, 49 / 115 at 1024, 69 / 114 at 2048, 100 / 115 at 2750, 104 / 117 at 3012, 118 / 123 at 3500, 127 / 128
+# at 4096; d 1024 57 / 114 at 24 rows, 68 / 112 at 200, 106 / 112 at 777, 112 / 112 at 1024, 173 / 171 at 1501, 202 / 195 at
+# 2048, 254 / 264 at 2600, 293 / 303 at 3002, 292 / 286 at 3072, 357 / 347 at 4096. Beyond ~1024 rows of d 1024 the two are
+# within 4 % either way (the 1024 x 1024 product alone: dh_proj_gemm 24.0 / 33 / 40 / 52 / 58 / 75 us at 1024 / 1501 / 2048 /
+# 2500 / 3002 / 4096 rows, the library 19.3 / 32 / 34 / 50 / 68 / 64), so the line stands where d 512 stops gaining much.
 QKV_GEMM_MAX_ROWS = 8192
 OUT_GEMM_MAX_ROWS = 4096
 OUT_GEMM_MAX_ROWS_F32 = 3072

@@ -332,9 +332,9 @@ class _MixerTrain(torch.autograd.Function):
 
 def mixer_train(mixer, x, mask, n_lv, weights):
     """A DispatcherMixer's output (b, T, d), differentiable in x and every parameter (reference
-    dispatcher_hybrid/modeling_dispatcher.py:63-123; under create_graph layer by layer, see _scan_again): one product for the three input projections, the gate path of
-    gate_scan_train, the output projection; one backward, in which the four weight gradients are one launch. `weights` as
-    mixer_fits returns them."""
+    dispatcher_hybrid/modeling_dispatcher.py:63-123; under create_graph layer by layer, see _scan_again): one product for
+    the three input projections, the gate path of gate_scan_train, the output projection; one backward, in which the four
+    weight gradients are one launch. `weights` as mixer_fits returns them."""
     ((Wi, bi), (Wf, bf), (Wr, br)), (W_in, W_x, W_s, W_out) = weights
     return _MixerTrain.apply(x, W_in, W_x, W_s, Wi, Wf, Wr, bi, bf, br, W_out, mask, mixer.num_heads, n_lv)
 

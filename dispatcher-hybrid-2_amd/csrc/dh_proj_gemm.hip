@@ -502,9 +502,11 @@ constexpr int64_t kWideGrid = 256;        // persistent workgroups: one per CU (
 // and stage counts.
 //
 // The persistent form's last round: with a few tiles more than a multiple of the 256 CUs, most CUs idle while a few compute
-// one more 256 x 256 tile (28-30 us at K = 1024). When less than a quarter of a round is left over, the whole rounds' rows go
-// first and the remaining rows take whatever form fits them, as a second launch (M = 3000, N = 2 x 2816, 264 tiles: 60.8 ->
-// 44.8 us; with 96 tiles left over, M = 4096, the split measured 62.8 against 61.2).
+// one more 256 x 256 tile (28-30 us at K = 1024). With less than 3/8 of a round left over, the whole rounds' rows go first and
+// the remaining rows take whatever form fits them, as a second launch. Measured by tiles left (us, one launch / split): after
+// one round N = 2 x 2816 8 59.5 / 44.1, 52 59.2 / 53.3, 74 59.6 / 54.1, 96 59.9 / 62.9, 118 60.7 / 65.9; N = 3072 8 57.3 /
+// 39.7, 56 57.9 / 49.4, 80 58.3 / 51.7, 92 58.5 / 52.1, 104 58.7 / 59.8; after two rounds N = 2 x 2816 16 94.1 / 79.8, 82
+// 96.2 / 89.6, 104 97.3 / 98.5; after four 10 159 / 146, 76 161 / 155.
 template <bool SWI>
 int launch_wide(GemmArgs& a, hipStream_t s, const char* who) {
   const int M = a.M, N = a.Ntot;
@@ -512,7 +514,7 @@ int launch_wide(GemmArgs& a, hipStream_t s, const char* who) {
     const int nt = (N + 255) / 256, mt = (M + 255) / 256;
     const int64_t rounds = (int64_t)mt * nt / kWideGrid, left = (int64_t)mt * nt - rounds * kWideGrid;
     const int whole = (int)(rounds * kWideGrid / nt);              // row tiles within the whole rounds
-    if (rounds >= 1 && left > 0 && left < kWideGrid / 4 && whole >= 1) {
+    if (rounds >= 1 && left > 0 && left < kWideGrid * 3 / 8 && whole >= 1) {
       GemmArgs head = a, tail = a;
       head.M = whole * 256;
       tail.M = M - head.M;
@@ -599,7 +601,7 @@ extern "C" int dh_proj_gemm(int dtype, const void* X, int64_t ldx, int M, int K,
   hipStream_t s = (hipStream_t)stream;
   // bf16 launches whose operands and outputs meet the ping-pong kernels' conditions (32-bit operand
   // offsets, segment widths multiples of 8, 16-byte aligned output rows) take them (launch_wide);
-  // the rest (fp32 among them) the 128 x 128 register-staged kernel.
+  // the rest the register-staged kernel (fp32 with the tile launch_f32 picks).
   bool wide = dtype == DH_BF16 && (int64_t)M * ldx * esz < (1ll << 31);
   for (int i = 0; i < nseg; ++i)
     wide = wide && N[i] % 8 == 0 && (int64_t)N[i] * K * esz < (1ll << 31) && ldo[i] % 8 == 0 && aligned(out[i], 16);

@@ -224,3 +224,30 @@ def test_proj_gemm_swiglu_batched_view_and_rejects():
                                         null, 96, _hip.stream_handle(x.device)) != 0
     assert _hip.lib.dh_proj_gemm_swiglu(_hip.DH_F32, _hip.ptr(x), 128, 600, 128, _hip.ptr(wg), _hip.ptr(wu), 96,
                                         null, 96, _hip.stream_handle(x.device)) != 0
+
+
+@pytest.mark.parametrize("M,left", [(2817, 8), (3000, 8), (3328 + 1, 52), (3768, 74), (4024, 96), (6072, 16), (6840, 82)])
+def test_swiglu_with_a_last_round_split_off_equals_its_row_blocks(M, left):
+    """Launches whose 256 x 256 tiles leave some after whole rounds of 256 (split into two launches below 96 left): every row
+    has the bits it has in a launch of few rows, which no form splits."""
+    from dispatcher_hybrid.fused_gates import fused_swiglu
+    assert -(-M // 256) * 22 % 256 == left
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, 128, device=DEV, generator=g).bfloat16()
+    wg, wu = ((torch.randn(2816, 128, device=DEV, generator=g) / 11).bfloat16() for _ in range(2))
+    got = fused_swiglu(x, wg, wu)
+    for r in range(0, M, 500):
+        assert torch.equal(got[r:r + 500], fused_swiglu(x[r:r + 500], wg, wu)), r
+
+
+@pytest.mark.parametrize("M,left", [(5377, 8), (5560, 8), (6584, 56), (7100, 80), (7352, 92), (7608, 104)])
+def test_projections_with_a_last_round_split_off_equal_their_row_blocks(M, left):
+    from dispatcher_hybrid.fused_gates import fused_projections
+    assert -(-M // 256) * 12 % 256 == left
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, 128, device=DEV, generator=g).bfloat16()
+    Ws = [(torch.randn(1024, 128, device=DEV, generator=g) / 11).bfloat16() for _ in range(3)]
+    got = fused_projections(x, Ws)
+    for r in range(0, M, 900):
+        for a, e in zip(got, fused_projections(x[r:r + 900], Ws)):
+            assert torch.equal(a[r:r + 900], e), r

@@ -49,7 +49,7 @@ def _mask_view(mask, cd, b, T, n_lv):
     if mask.dim() != 3:
         raise ValueError(f"document mask: (b, T, levels) expected, got {tuple(mask.shape)}")
     if mask.shape[0] != b or mask.shape[1] != T or mask.shape[2] < n_lv:
-        mask = mask.expand(b, T, n_lv)
+        mask = mask[..., :n_lv].expand(b, T, n_lv)
     m = mask.to(cd)
     return m, m.stride(0), m.stride(1), m.stride(2)
 

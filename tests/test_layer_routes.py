@@ -114,7 +114,7 @@ def test_layers_and_masks_on_another_device_are_not_launched_directly():
 def test_masks_of_other_sizes_raise_or_broadcast():
     from dispatcher_hybrid.fused_gates import _mask_view
     b, T, n = 2, 8, 3
-    for shape in ((2, 8, 5), (2, 8, 3), (1, 8, 3), (2, 1, 1)):
+    for shape in ((2, 8, 5), (2, 8, 3), (1, 8, 3), (1, 8, 5), (2, 1, 1)):
         mask = torch.rand(shape)
         m, *strides = _mask_view(mask, torch.float32, b, T, n)
         assert torch.equal(m.as_strided((b, T, n), strides), mask[..., :n].expand(b, T, n))

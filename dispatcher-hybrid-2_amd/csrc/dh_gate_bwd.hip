@@ -492,7 +492,7 @@ constexpr int kHidRow = 160;    // padded LDS row of 64 bf16: four rows a transp
 template <typename T>
 __global__ __launch_bounds__(kWThreads, 3) void gate_bwd_w(WArgs a) {
   constexpr int TB = Lay<T>::TB;
-  __shared__ __align__(16) unsigned char lds[4 * 32 * kHidRow];          // also the waves' sums at the end (12 KB)
+  __shared__ __align__(16) unsigned char lds[4 * 32 * kHidRow];          // also the waves' sums at the end (16 KB)
   const Dims& d = a.d;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, g = lane >> 4;

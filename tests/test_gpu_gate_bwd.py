@@ -112,3 +112,26 @@ def test_gate_backward_infinite_source_reaches_only_its_destinations():
     outs += [torch.empty(n_lv, H, GH, device=DEV) for _ in range(3)] + [torch.empty(n_lv, H, device=DEV) for _ in range(3)]
     _preacts_bwd_launch(A, B, *W, dP, mask, outs, n_lv, n_lv, "test")
     assert all(bool(o.isfinite().all()) for o in outs) and not outs[1][0, 7].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,T,GH,H,n_lv,masked", [(1, 1, 64, 1, 1, False), (2, 33, 128, 17, 5, True), (1, 70, 320, 16, 8, True)])
+def test_backward_without_scratch_equals_the_one_with(b, T, GH, H, n_lv, masked, dtype):
+    """dh_gate_preacts_bwd (the C entry for callers without scratch memory: fp32 atomics, any order) against float64."""
+    from dispatcher_hybrid import _hip
+    g = torch.Generator(device=DEV).manual_seed(T)
+    rn = lambda *s: torch.randn(*s, device=DEV, generator=g).to(dtype)
+    A, B, W = rn(b, T, GH), rn(b, T, GH), [rn(n_lv, H, GH) * 0.1 for _ in range(3)]
+    dP = [rn(b, T, n_lv, H) for _ in range(3)]
+    mask = (torch.rand(b, T, n_lv, device=DEV, generator=g) < 0.8).to(dtype) if masked else None
+    outs = [torch.full((b, T, GH), float("nan"), device=DEV) for _ in range(2)]
+    outs += [torch.full((n_lv, H, GH), float("nan"), device=DEV) for _ in range(3)]
+    outs += [torch.full((n_lv, H), float("nan"), device=DEV) for _ in range(3)]
+    p = _hip.ptr
+    st = _hip.lib.dh_gate_preacts_bwd(
+        _hip.dtype_code(dtype), p(A), p(B), A.stride(0), A.stride(1), *[p(w) for w in W], W[0].stride(0), W[0].stride(1),
+        *[p(d) for d in dP], p(mask), *(mask.stride() if masked else (0, 0, 0)), *[p(o) for o in outs], b, T, GH, H, n_lv,
+        _hip.stream_handle(A.device))
+    _hip.check(st, "dh_gate_preacts_bwd")
+    for i, (x, y) in enumerate(zip(outs, _reference(A, B, W, dP, mask, n_lv, dtype))):
+        assert (x.double() - y).abs().max() <= 2e-5 * y.abs().max().clamp_min(1e-6), i

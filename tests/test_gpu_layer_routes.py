@@ -202,3 +202,26 @@ def test_training_runs_a_modules_own_scan_and_rotation():
         got = layer(*_inputs(layer, cls, x))
         assert (got.double() - want.double()).norm() <= 1e-2 * want.double().norm()
         got.sum().backward()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b,T,masked", [(1, 1, False), (1, 203, False), (2, 70, True), (3, 257, True), (3, 64, "shared"),
+                                        (2, 1500, True)])
+def test_one_call_mixer_layer_equals_its_launches(b, T, masked, dtype):
+    """mixer_layer against fused_projections, fused_gate_scan and the output projection on their own, bit for bit."""
+    from dispatcher_hybrid import fused_gates as fg
+    mx = _layer("DispatcherMixer", dtype)
+    L = mx.levels
+    n_lv = min(L, T.bit_length())
+    x = torch.randn(b, T, 256, device=DEV).to(dtype)
+    mask = None
+    if masked:
+        mask = (torch.rand(1 if masked == "shared" else b, T, L, device=DEV) < 0.8).to(dtype)
+    with torch.no_grad():
+        weights = fg.mixer_layer_fits(mx, x)
+        got = fg.mixer_layer(mx, x, mask, n_lv, weights)
+        V0, A, B = fg.fused_projections(x, [mx.linear_in.weight, mx.gate_hidden.weight, mx.gate_hidden_src.weight])
+        (Wi, bi), (Wf, bf), (Wr, br) = weights[0]
+        m = None if mask is None else mask.expand(b, T, L)
+        V = fg.fused_gate_scan(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, m, V0, mx.num_heads)
+        assert torch.equal(got, fg.fused_projections(V, [mx.linear_out.weight])[0])

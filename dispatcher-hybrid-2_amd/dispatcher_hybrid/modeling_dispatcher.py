@@ -278,10 +278,12 @@ class WindowAttention(nn.Module):
         if self.use_fused and not torch.is_grad_enabled() and x.is_cuda:
             from . import fused_attention as fa
             if fa.supported(x.dtype, self.head_dim):
-                from .fused_gates import out_max_rows, project, qkv_max_rows
+                from .fused_gates import _rows16 as rows16, out_max_rows, project, qkv_max_rows
                 # q, k, v as one GEMM launch (up to qkv_max_rows rows); RoPE, banded scores,
                 # softmax and the value average in one launch, (B, T, d) in/out
-                q, k, v = project(x, [self.linear_q, self.linear_k, self.linear_v], qkv_max_rows())
+                q, k, v = (rows16(t, 8) for t in project(x, [self.linear_q, self.linear_k, self.linear_v], qkv_max_rows()))
+                if not (q.stride() == k.stride() == v.stride()):               # (what stands around a projection may differ)
+                    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
                 cos, sin = self.rope_tables(T, x.device, x.dtype)
                 y = fa.window_attention(q, k, v, cos, sin, self.num_heads, self.band(T))
                 return project(y, [self.linear_out], out_max_rows(y.dtype))[0]

@@ -225,3 +225,16 @@ def test_one_call_mixer_layer_equals_its_launches(b, T, masked, dtype):
         m = None if mask is None else mask.expand(b, T, L)
         V = fg.fused_gate_scan(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, m, V0, mx.num_heads)
         assert torch.equal(got, fg.fused_projections(V, [mx.linear_out.weight])[0])
+
+
+@pytest.mark.parametrize("T", [100, 2500])
+def test_attention_takes_a_hooked_projection_in_another_layout(T):
+    layer = _layer("WindowAttention", torch.bfloat16)
+    layer.linear_k.register_forward_hook(lambda m, i, o: 2 * torch.cat((o[..., :8], o), -1)[..., 8:])
+    layer.linear_v.register_forward_hook(lambda m, i, o: _last_dim_first(o))
+    x = torch.randn(2, T, 256, device=DEV).bfloat16()
+    with torch.no_grad():
+        want = layer(x)
+        layer.use_fused = True
+        got = layer(x)
+    assert (got.double() - want.double()).norm() <= 1e-2 * want.double().norm()

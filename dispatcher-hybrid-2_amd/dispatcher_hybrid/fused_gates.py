@@ -361,32 +361,45 @@ def fused_projections(x, weights):
     weights: up to three (N_s, K) tensors of x's dtype. Inference only (no autograd)."""
     _hip.require_gpu(x, "fused_projections")
     K = x.shape[-1]
-    x2 = _rows16(x.reshape(-1, K), 16 // x.element_size())
-    M = x2.shape[0]
-    n = len(weights)
     for w in weights:
         if w.dtype != x.dtype or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous():
             raise ValueError("fused_projections: weights must be contiguous (N, K) tensors of x's dtype")
     _hip.same_gpu("fused_projections", x, *weights)
-    outs = [torch.empty(*x.shape[:-1], w.shape[0], device=x.device, dtype=x.dtype) for w in weights]
+    return projections_launch(x, weights)
+
+
+def projections_launch(x, weights):
+    """fused_projections of weights that are known to be what it asks for."""
+    K = x.shape[-1]
+    x2 = _rows16(x.reshape(-1, K), 16 // x.element_size())
+    M = x2.shape[0]
+    n = len(weights)
+    widths = [w.shape[0] for w in weights]
+    outs = [torch.empty(*x.shape[:-1], N, device=x.device, dtype=x.dtype) for N in widths]
     if M == 0:
         return outs
     Ws = (ctypes.c_void_p * n)(*[w.data_ptr() for w in weights])
-    Ns = (ctypes.c_int * n)(*[w.shape[0] for w in weights])
+    Ns = (ctypes.c_int * n)(*widths)
     Os = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
-    Ls = (ctypes.c_int64 * n)(*[w.shape[0] for w in weights])
+    Ls = (ctypes.c_int64 * n)(*widths)
     st = _hip.lib.dh_proj_gemm(_hip.dtype_code(x.dtype), _hip.ptr(x2), x2.stride(0), M, K, n, Ws, Ns, Os, Ls,
                                _hip.stream_handle(x.device))
     _hip.check(st, "dh_proj_gemm")
     return outs
 
 
+def fitting_weights(x, linears):
+    """The layers' weights if dh_proj_gemm gives what calling these layers gives, else None: plain bias-free nn.Linear layers
+    (plain_linear), CUDA input, weights of x's dtype, K a multiple of 64 (bf16) / 32 (fp32), output widths multiples of 4."""
+    if not (x.is_cuda and len(linears) <= 3 and x.shape[-1] % (64 if x.dtype == torch.bfloat16 else 32) == 0):
+        return None
+    dt, K, dev = x.dtype, x.shape[-1], x.device
+    ws = [plain_weight(l, dt, K, dev) for l in linears]
+    return None if any(w is None or w.shape[0] % 4 for w in ws) or _has_any_global_hook() or _function_mode() else ws
+
+
 def projections_fit(x, linears):
-    """True when dh_proj_gemm gives what calling these layers gives: plain bias-free nn.Linear layers (plain_linear), CUDA
-    input, weights of x's dtype, K a multiple of 64 (bf16) / 32 (fp32), output widths multiples of 4."""
-    return (x.is_cuda and len(linears) <= 3 and all(plain_linear(l, x.dtype, x.shape[-1], x.device) for l in linears)
-            and x.shape[-1] % (64 if x.dtype == torch.bfloat16 else 32) == 0
-            and all(l.weight.shape[0] % 4 == 0 for l in linears))
+    return fitting_weights(x, linears) is not None
 
 
 # Rows above which the three library GEMMs (hipBLASLt through nn.Linear) beat dh_proj_gemm for the
@@ -406,9 +419,8 @@ def input_projections(x, mixer):
     Inference only."""
     lins = (mixer.linear_in, mixer.gate_hidden, mixer.gate_hidden_src)
     rows = x.numel() // max(x.shape[-1], 1)
-    if rows <= PROJ_GEMM_MAX_ROWS and projections_fit(x, lins):
-        return fused_projections(x, [l.weight for l in lins])
-    return tuple(l(x) for l in lins)
+    weights = fitting_weights(x, lins) if rows <= PROJ_GEMM_MAX_ROWS else None
+    return tuple(l(x) for l in lins) if weights is None else projections_launch(x, weights)
 
 
 # Rows up to which one dh_proj_gemm launch beats the library, measured on MI355X in captured graphs over 18 distinct weights,
@@ -444,11 +456,10 @@ def qkv_max_rows():
 
 def project(x, linears, max_rows):
     """[l(x) for l in linears] (layers over the same input) as one dh_proj_gemm launch when x has at most max_rows rows and
-    the kernel takes them (projections_fit), else the layers' own calls. Inference only."""
+    the kernel takes them (fitting_weights), else the layers' own calls. Inference only."""
     rows = x.numel() // max(x.shape[-1], 1)
-    if rows <= max_rows and projections_fit(x, linears):
-        return fused_projections(x, [l.weight for l in linears])
-    return [l(x) for l in linears]
+    weights = fitting_weights(x, linears) if rows <= max_rows else None
+    return [l(x) for l in linears] if weights is None else projections_launch(x, weights)
 
 
 def _function_mode():
@@ -541,13 +552,20 @@ def mixer_layer(mixer, x, mask, n_lv, weights):
     return y
 
 
+def swiglu_weights(x, gate, up):
+    """The two weights if dh_proj_gemm_swiglu gives silu(gate(x)) * up(x) for these layers, else None: plain bias-free
+    nn.Linear layers (plain_linear), a bf16 CUDA input, bf16 weights of one shape, K a multiple of 64 and N of 8."""
+    if not (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[-1] % 64 == 0):
+        return None
+    K, dev = x.shape[-1], x.device
+    wg, wu = plain_weight(gate, x.dtype, K, dev), plain_weight(up, x.dtype, K, dev)
+    if wg is None or wu is None or wg.shape != wu.shape or wg.shape[0] % 8 or _has_any_global_hook() or _function_mode():
+        return None
+    return wg, wu
+
+
 def swiglu_fits(x, gate, up):
-    """True when dh_proj_gemm_swiglu gives silu(gate(x)) * up(x) for these layers: plain bias-free nn.Linear layers
-    (plain_linear), a bf16 CUDA input, bf16 weights of one shape, K a multiple of 64 and N of 8."""
-    K = x.shape[-1]
-    return (x.is_cuda and x.dtype == torch.bfloat16 and plain_linear(gate, x.dtype, K, x.device)
-            and plain_linear(up, x.dtype, K, x.device)
-            and gate.weight.shape == up.weight.shape and K % 64 == 0 and gate.weight.shape[0] % 8 == 0)
+    return swiglu_weights(x, gate, up) is not None
 
 
 def fused_swiglu(x, w_gate, w_up):
@@ -557,14 +575,19 @@ def fused_swiglu(x, w_gate, w_up):
     rounded -- without the two GEMM outputs ever reaching memory. x: (..., K) bf16; w_gate, w_up:
     (N, K) bf16. Returns (..., N). Inference only (no autograd)."""
     _hip.require_gpu(x, "fused_swiglu")
-    K = x.shape[-1]
-    x2 = _rows16(x.reshape(-1, K), 8)
-    N = w_gate.shape[0]
+    N, K = w_gate.shape[0], x.shape[-1]
     _hip.same_gpu("fused_swiglu", x, w_gate, w_up)
     if (x.dtype != torch.bfloat16 or w_gate.dtype != torch.bfloat16 or w_up.dtype != torch.bfloat16
             or w_gate.shape != (N, K) or w_up.shape != (N, K) or not w_gate.is_contiguous()
             or not w_up.is_contiguous()):
         raise ValueError("fused_swiglu: bf16 x (..., K) and contiguous bf16 (N, K) gate and up weights")
+    return swiglu_launch(x, w_gate, w_up)
+
+
+def swiglu_launch(x, w_gate, w_up):
+    """fused_swiglu of operands that are known to be what it asks for."""
+    N, K = w_gate.shape
+    x2 = _rows16(x.reshape(-1, K), 8)
     out = torch.empty(*x.shape[:-1], N, device=x.device, dtype=x.dtype)
     M = x2.shape[0]
     if M == 0:

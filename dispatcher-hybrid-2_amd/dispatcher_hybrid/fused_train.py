@@ -24,7 +24,8 @@ import torch.nn.functional as F
 
 from . import _hip
 from .fused_gates import (OUT_GEMM_MAX_ROWS, PROJ_GEMM_MAX_ROWS, _preacts_bwd_launch, _preacts_launch, _rows16,
-                          fused_gate_preacts, fused_projections, plain_eager, plain_mixer_weights, plain_square_weights)
+                          fused_gate_preacts, plain_eager, plain_mixer_weights, plain_square_weights,
+                          projections_launch)
 
 SCAN_MAX_LEN = 4096
 SCAN_MAX_LEVELS = 12
@@ -211,7 +212,7 @@ def gate_scan_train(A, B, Wi, Wf, Wr, bi, bf, br, n_lv, mask, V0, num_heads):
 def _linear(x2, w, max_rows):
     """x2 (M, K) . w^T: dh_proj_gemm in bf16 up to max_rows rows (measured in fused_gates), else the library."""
     if x2.dtype == torch.bfloat16 and x2.shape[0] <= max_rows and w.shape[1] % 64 == 0 and w.shape[0] % 4 == 0:
-        return fused_projections(x2, [w])[0]
+        return projections_launch(x2, [w])[0]
     return F.linear(x2, w)
 
 

@@ -278,12 +278,13 @@ class WindowAttention(nn.Module):
         if self.use_fused and not torch.is_grad_enabled() and x.is_cuda:
             from . import fused_attention as fa
             if fa.supported(x.dtype, self.head_dim):
-                from .fused_gates import _rows16 as rows16, out_max_rows, project, qkv_max_rows
+                from .fused_gates import out_max_rows, project, qkv_max_rows
                 # q, k, v as one GEMM launch (up to qkv_max_rows rows); RoPE, banded scores,
                 # softmax and the value average in one launch, (B, T, d) in/out
-                q, k, v = (rows16(t, 8) for t in project(x, [self.linear_q, self.linear_k, self.linear_v], qkv_max_rows()))
-                if not (q.stride() == k.stride() == v.stride()):               # (what stands around a projection may differ)
-                    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+                q, k, v = project(x, [self.linear_q, self.linear_k, self.linear_v], qkv_max_rows())
+                if not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
+                    # (what stands around a projection may return any layout)
+                    q, k, v = (t.clone(memory_format=torch.contiguous_format) for t in (q, k, v))
                 cos, sin = self.rope_tables(T, x.device, x.dtype)
                 y = fa.window_attention(q, k, v, cos, sin, self.num_heads, self.band(T))
                 return project(y, [self.linear_out], out_max_rows(y.dtype))[0]
@@ -333,9 +334,10 @@ class SwiGLU(nn.Module):
     def forward(self, h):
         if (self.use_fused and h.is_cuda and not torch.is_grad_enabled()
                 and h.dtype in (torch.float32, torch.bfloat16)):                   # dh_silu_mul's dtypes
-            from .fused_gates import DOWN_GEMM_MAX_ROWS, fused_swiglu, plain_linear, project, silu_mul, swiglu_fits
-            if swiglu_fits(h, self.linear_gate, self.linear_up):
-                a = fused_swiglu(h, self.linear_gate.weight, self.linear_up.weight)
+            from .fused_gates import DOWN_GEMM_MAX_ROWS, plain_linear, project, silu_mul, swiglu_launch, swiglu_weights
+            weights = swiglu_weights(h, self.linear_gate, self.linear_up)
+            if weights is not None:
+                a = swiglu_launch(h, *weights)
             else:
                 g, u = self.linear_gate(h), self.linear_up(h)
                 if g.shape == u.shape and g.dtype == u.dtype and g.dtype in (torch.float32, torch.bfloat16):

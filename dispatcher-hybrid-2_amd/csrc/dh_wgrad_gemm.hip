@@ -7,11 +7,13 @@
 // 32-byte granule q of row m is kept at q ^ (m & 3).
 // A workgroup (4 waves) owns 128 x 128 outputs (64 x 64 a wave) or 128 x 256 (64 x 128 a wave) over one range of rows; up
 // to four layers with the same rows go into one launch (a mixer's four projections: 256 or 128 tiles). With fewer tiles
-// than workgroup slots the rows are split and a second launch adds the ranges' fp32 sums in order and rounds once; the same inputs give the same bits. Consecutive
-// work items (the tiles of one layer and range, which read the same rows) go to one XCD.
+// than workgroup slots the rows are split and a second launch adds the ranges' fp32 sums in order and rounds once; the same
+// inputs give the same bits. Consecutive work items (the tiles of one layer and range, which read the same rows) go to one
+// XCD.
 // Bound: LDS (the fragment reads and the staging stores, see tile_k) beside the matrix cores. Measured on MI355X, four
-// 1024 x 1024 gradients: 152 us at 16384 rows (900 TFLOP/s; 170 with the 128-wide tile), 57 at 4096, against 453 and 124 for
-// the library's four.
+// 1024 x 1024 gradients: called in a row on the same rows 152 us at 16384 rows (170 with the 128-wide tile), 57 at 4096, the
+// library's four 453 and 124; within a training layer's pass, traced, 153-171 + 13 for the reduction at 16384 rows (over
+// boxes; 745-900 TFLOP/s), 50 + 8 at 4096.
 #include "dh_common.h"
 
 namespace {

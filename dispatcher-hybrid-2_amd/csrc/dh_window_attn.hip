@@ -24,7 +24,7 @@
 // permlane swaps), this lane's part of the sum and the rescale stay in registers, and the probabilities are already in
 // the B-operand layout of O^T = V^T P^T, whose A operand is read transposed from the value rows (ds_read_tr16_b64).
 // Bound: VALU (the 16 exponentials a block and lane cost as much as its 16 MFMA products). Measured on MI355X at B 2, T 3001,
-// window 1024, 16 heads of 64: 59 us; with the values transposed through 4-byte LDS writes, LDS shuffles for both
+// window 1024, 16 heads of 64: 56-59 us; with the values transposed through 4-byte LDS writes, LDS shuffles for both
 // reductions and a rescale per block 66 us.
 // Workgroups are numbered so consecutive query blocks of one (batch row, head) run on one XCD (round-robin dispatch: block id
 // mod 8), sharing the band's key and value lines in that XCD's L2.

@@ -72,9 +72,8 @@ def _preacts_launch(A_, B_, Wi_, Wf_, Wr_, bi_, bf_, br_, mask, outs, ostrides, 
 
 def _prep_gate_inputs(A, B, Wi, Wf, Wr, bi, bf, br, n_lv):
     cd = _compute_dtype(A)
-    A_ = A.contiguous().to(cd)
-    B_ = B.contiguous().to(cd)
-    Wi_, Wf_, Wr_ = (w[:n_lv].contiguous().to(cd) for w in (Wi, Wf, Wr))
+    A_, B_ = (_rows16(t.contiguous().to(cd), 8) for t in (A, B))
+    Wi_, Wf_, Wr_ = (_rows16(w[:n_lv].contiguous().to(cd), 8) for w in (Wi, Wf, Wr))
     # the kernel reads biases of the compute dtype as they are, others as fp32 copies
     bd = cd if bi.dtype == bf.dtype == br.dtype == cd else torch.float32
     bi_, bf_, br_ = (v[:n_lv].contiguous().to(bd) for v in (bi, bf, br))
@@ -244,7 +243,7 @@ def _level_scan_fwd_op(pre_i: torch.Tensor, pre_f: torch.Tensor, pre_r: torch.Te
 def _scan_launch(pre_i, pre_f, pre_r, mask, V0, out, num_heads, n_lv, activated, what, ring=None, ring_L=0):
     b, T, d = V0.shape
     cd = V0.dtype
-    V0_ = V0 if V0.stride(-1) == 1 else V0.contiguous()
+    V0_ = _rows16(V0, 16 // V0.element_size())
     pi, pf, pr = (g.to(cd) for g in (pre_i, pre_f, pre_r))       # keeps each tensor's layout
     if not (pi.stride() == pf.stride() == pr.stride()):
         pi, pf, pr = pi.contiguous(), pf.contiguous(), pr.contiguous()

@@ -238,3 +238,22 @@ def test_attention_takes_a_hooked_projection_in_another_layout(T):
         layer.use_fused = True
         got = layer(x)
     assert (got.double() - want.double()).norm() <= 1e-2 * want.double().norm()
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("moved", [_last_dim_first, _odd_offset])
+def test_mixer_takes_hooked_projections_and_gate_weights_in_another_layout(moved, dtype, train):
+    mx = _layer("DispatcherMixer", dtype)
+    for l in (mx.linear_in, mx.gate_hidden, mx.gate_hidden_src):
+        l.register_forward_hook(lambda m, i, o: moved(o))
+    mx.forget_out.data = _odd_offset(mx.forget_out.data)
+    x = torch.randn(2, 100, 256, device=DEV).to(dtype)
+    with torch.set_grad_enabled(train):
+        want = mx(*_inputs(mx, "DispatcherMixer", x))
+        mx.use_fused_gates = True
+        got = mx(*_inputs(mx, "DispatcherMixer", x))
+    assert (got.double() - want.double()).norm() <= (1e-2 if dtype == torch.bfloat16 else 2e-5) * want.double().norm()
+    if train:
+        got.sum().backward()
+        assert all(p.grad.isfinite().all() for p in mx.parameters())

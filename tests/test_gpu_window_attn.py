@@ -123,3 +123,24 @@ def test_window_attention_of_a_position_does_not_see_later_ones(hd, window):
         assert torch.equal(fa.window_attention(*mixed, cos, sin, H, window)[:, :t], y[:, :t]), t
         cut = [a[:, :t].contiguous() for a in (q, k, v)]
         assert torch.equal(fa.window_attention(*cut, cos, sin, H, window), y[:, :t]), t
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128])
+def test_window_attention_leading_weight_is_not_rounded(hd):
+    """One key ahead of all others by less than 2^8, in a later block than the first: its probability before normalisation
+    is exactly 1, so the output (its value alone, the other values are zero) is off by its own bf16 rounding, half a spacing
+    (2^-8 of the power of two below it: 8 significant bits), and fp32 arithmetic (2^-17 covers ~100 roundings)."""
+    from dispatcher_hybrid import fused_attention as fa
+    T, H = 200, 16
+    cos, sin = torch.ones(T, hd // 2, device=DEV, dtype=DT), torch.zeros(T, hd // 2, device=DEV, dtype=DT)
+    q, k, v = (torch.zeros(1, T, H, hd, device=DEV, dtype=DT) for _ in range(3))
+    q[..., 0] = 2.0 ** round(math.log2(hd) / 2)                  # score = k[0] times a power of two over sqrt(hd)
+    lead = torch.linspace(0.3, 5.4, H, device=DEV).to(DT)
+    k[0, 100, :, 0] = lead
+    v[0, 100] = torch.randn(H, hd, device=DEV, generator=torch.Generator(device=DEV).manual_seed(hd)).to(DT)
+    y = fa.window_attention(*(t.view(1, T, H * hd) for t in (q, k, v)), cos, sin, H, 0).view(T, H, hd)[128:].double()
+    e = torch.exp(lead.double() * q[0, 0, 0, 0].double() / math.sqrt(hd))
+    t = torch.arange(128, T, device=DEV).double().view(-1, 1)
+    want = (e / (e + t)).unsqueeze(-1) * v[0, 100].double()
+    half = torch.exp2(torch.floor(torch.log2(want.abs()))) * 2.0 ** -8
+    assert ((y - want).abs() <= half + 2.0 ** -17 * want.abs()).all()

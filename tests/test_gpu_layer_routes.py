@@ -1,6 +1,6 @@
 """The fused inference layers call a projection that something stands around (a hook, an adapter, a replaced forward) at every
 row count: with one that doubles its result, the layer's output is what the torch path gives. Tolerance (2-norm relative):
-each projection, the layer's inner results and its output are rounded to bf16 (2^-9) on either path, at most ~12 roundings a
+each projection, the layer's inner results and its output are rounded to bf16 (2^-9 in the mean) on either path, at most ~12 roundings a
 path: 24 of them in quadrature 1e-2; fp32 sums of at most 1024 products and 12 levels 2e-5."""
 
 import pytest

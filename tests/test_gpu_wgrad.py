@@ -1,4 +1,4 @@
-"""dh_wgrad_gemm against float64: each output within half a bf16 ulp of its rounding (2^-9 relative) plus the fp32
+"""dh_wgrad_gemm against float64: each output within half a bf16 spacing of its rounding (at most 2^-8 relative) plus the fp32
 accumulation of M products (M 2^-24 of the sum of their magnitudes; 2^-11 of it covers M <= 8192)."""
 
 import pytest

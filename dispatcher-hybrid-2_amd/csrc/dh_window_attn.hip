@@ -21,11 +21,12 @@
 // alike, double-buffered, the next block's global loads in flight during the current block. Scores are computed transposed,
 // S^T = K Q^T (v_mfma_f32_16x16x32_bf16, A = key rows from LDS, B = the wave's rotated query fragments held in registers),
 // so the C fragment puts one query per lane column: the running max (exchanged between the four lanes of a query by
-// permlane swaps), this lane's part of the sum and the rescale stay in registers, and the probabilities are already in
+// permlane swaps), the running sum and the rescale stay in registers, and the probabilities are already in
 // the B-operand layout of O^T = V^T P^T, whose A operand is read transposed from the value rows (ds_read_tr16_b64).
 // Bound: VALU (the 16 exponentials a block and lane cost as much as its 16 MFMA products). Measured on MI355X at B 2, T 3001,
-// window 1024, 16 heads of 64: 57-60 us; with the values transposed through 4-byte LDS writes, LDS shuffles for both
-// reductions and a rescale in every block 66 us.
+// window 1024, 16 heads of 64, with the pre-pass: 66 us; with the values transposed through 4-byte LDS writes, LDS shuffles for
+// both reductions and a rescale in every block 70, to the same bits (the products with the scale and the sums keep their
+// roundings; folding the scale into the exponent's multiply-add and summing over the lanes at the end measured 63).
 // Workgroups are numbered so consecutive query blocks of one (batch row, head) run on one XCD (round-robin dispatch: block id
 // mod 8), sharing the band's key and value lines in that XCD's L2.
 #include "dh_attn_common.h"
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
   f32x4 o[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) o[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m = -1e30f, l = 0.f;                      // running max (finite floor); this lane's part of the running sum
+  float m = -1e30f, l = 0.f;                      // running max (finite floor) and sum of this query
 
   kv_fetch(kb_lo);
   kv_store(0);
@@ -178,14 +179,16 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
         sT[tau] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[s], sT[tau], 0, 0, 0);
       }
     }
-    // softmax via 2^x: scale * log2 e is folded into the exponent's multiply-add. A block strictly below
-    // the diagonal and wholly inside every query's window needs no mask (all blocks but the band's
-    // first and last): a uniform branch.
+    // scores in the log2 domain (scale * log2 e folded in; softmax via 2^x). A block strictly below the diagonal and wholly
+    // inside every query's window needs no mask (all blocks but the band's first and last): a uniform branch.
     const bool interior = kb < qb && (a.window == 0 || q0 + kBQ - 1 - kb * kBK < a.window);
     float p[16];
     float mx = -INFINITY;
+    {
+#pragma clang fp contract(off)
 #pragma unroll
-    for (int j = 0; j < 16; ++j) p[j] = sT[j >> 2][j & 3];
+      for (int j = 0; j < 16; ++j) p[j] = sT[j >> 2][j & 3] * a.scale2;
+    }
     if (!interior) {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
@@ -196,26 +199,31 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
     }
 #pragma unroll
     for (int j = 0; j < 16; ++j) mx = fmaxf(mx, p[j]);
-    mx = across_groups_max(mx) * a.scale2;        // scale2 > 0
+    mx = across_groups_max(mx);
     // the output is rescaled only in blocks where a query's max moves; a lane that keeps its max has alpha 1, so a query's
     // result does not depend on the others of its wave. The max itself is always the running one: the largest weight is
     // then exactly 1 in bf16. (Moving it only when it falls 2^8 behind saves 0-2 % and rounds the leading weights instead:
     // 2.05e-3 from exact where this is 1.73e-3, scores of standard deviation 4.)
+    float alpha = 1.f;
     if (__builtin_amdgcn_ballot_w64(mx > m)) {
       const float mn = fmaxf(m, mx);
-      const float alpha = __builtin_amdgcn_exp2f(m - mn);
+      alpha = __builtin_amdgcn_exp2f(m - mn);
       m = mn;
-      l *= alpha;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[nt][i] *= alpha;
     }
+    float ps = 0.f;
+    {
+#pragma clang fp contract(off)
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      p[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(p[j], a.scale2, -m));   // masked: 2^-inf = 0
-      l += p[j];
+      for (int j = 0; j < 16; ++j) {
+        p[j] = __builtin_amdgcn_exp2f(p[j] - m);  // masked: 2^-inf = 0
+        ps += p[j];
+      }
     }
+    l = __builtin_fmaf(l, alpha, across_groups_sum(ps));
 
     // ---- O^T += V^T P^T over the two 32-key steps; key order within a step: the lane group's
     // four keys of tile 2kk, then its four keys of tile 2kk + 1 (the same order on both operands)
@@ -240,7 +248,6 @@ __global__ __launch_bounds__(kThreads) void window_attn_kernel(WinArgs a) {
   }
 
   // ---- output: lane holds query tq, hd columns 16 nt + 4 g + i
-  l = across_groups_sum(l);
   if (tq < a.T) {
     const float inv = 1.f / l;
     if (a.lse != nullptr && g == 0) a.lse[((int64_t)b * a.H + h) * a.T + tq] = m + __builtin_amdgcn_logf(l);
